@@ -292,17 +292,33 @@ static void release_pending() {
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int kNT = 256;      // threads per workgroup of the FFT passes
-constexpr int kNTBig = 1024;  // dimension-1 passes with long lines (1D)
-constexpr int kNTSmall = 128;  // batched passes whose tile holds <= 128*kE elements
-constexpr int kE = 16;        // complex elements staged per thread and stage
+constexpr int kNT = 256;      // threads per workgroup of the vector kernels
+// FFT passes: kE complex elements of the tile per thread, so the workgroup
+// size follows from the tile (tile_nt): 256 or 512 threads up to kTile
+// elements, 1024 up to 8192 and, sized kNTLong, 1024 threads of 16 elements up
+// to kTileLong (dimension-1 passes only)
+constexpr int kE = 8;
+constexpr int kTile = 4096;
+// tiles grow to kTileGrow elements (256 threads), and beyond only while a row
+// of the tile spans less than 64 bytes: several small workgroups on a CU
+// overlap one's loads with another's transform
+constexpr int kTileGrow = 2048;
+inline bool tile_grows(int lg, int W, size_t cs) {
+  const int64_t e = (int64_t)(2 << lg) * W;
+  return e <= kTileGrow || (e <= kTile && ((size_t)1 << lg) * cs < 64);
+}
+constexpr int kTileLong = 16384;
+constexpr int kNTLong = 2048;   // names the last: 1024 threads, 16 elements each
+inline int tile_nt(int64_t elems) {
+  return elems <= 256 * kE ? 256 : elems <= 512 * kE ? 512 : elems <= 1024 * kE ? 1024 : kNTLong;
+}
 constexpr size_t kLdsSmall = 64 * 1024;
 constexpr size_t kLdsMax = 160 * 1024;
 
 struct LineCfg {
   int lg = 0, ntile1 = 0, grid = 0;
   size_t lds = 0;
-  int nt = 256;   // workgroup size of the batched pass (kNT or kNTSmall)
+  int nt = 256;   // workgroup size (tile_nt)
 };
 struct Dim1Cfg {
   int nt = 0, lg = 0, ps = 0, npairs = 0, grid = 0;
@@ -316,7 +332,6 @@ struct PrecState {
   void* tw[3] = {nullptr, nullptr, nullptr};
   void* chirp[3] = {nullptr, nullptr, nullptr};   // Bluestein tables (axes with bs)
   void* bfw[3] = {nullptr, nullptr, nullptr};
-  void* binv[3] = {nullptr, nullptr, nullptr};
   LineCfg lines[3];
   Dim1Cfg d1;
   // long 1D lines (four-step): twiddles of the column (B) and row (A)
@@ -383,38 +398,36 @@ static uint32_t magic(int d) {
   return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
 }
 
-// radix sequence for length L: the odd radices 31, 29, 23, 19 first (stage 0
-// has no twiddles, and these radices load theirs where they use them), then
-// 16, 8, 4, 2 for the power of two, then odd radices 17, 13, 11, 7, 15 (=3*5),
-// 9, 5, 3
+// radix sequence for length L: odd radices first, the power of two last.  The
+// first stages write their outputs R rows apart, which an odd R spreads over
+// the LDS banks (16 rows apart, all lanes of a one-line tile meet in one or
+// two banks), and the last stages write whole runs of rows.
 static bool factorize(int L, FftPlan& p) {
   p.L = L;
   p.nstages = 0;
+  p.variant = 0;
   int m = L;
   auto push = [&](int r) {
     if (p.nstages >= kMaxStages) return false;
-    p.radix[p.nstages++] = r;
+    p.st[p.nstages++].radix = r;
     return true;
   };
-  for (int r : {31, 29, 23, 19})
-    while (m % r == 0) { if (!push(r)) return false; m /= r; }
-  while (m % 16 == 0) { if (!push(16)) return false; m /= 16; }
-  while (m % 8 == 0) { if (!push(8)) return false; m /= 8; }
-  while (m % 4 == 0) { if (!push(4)) return false; m /= 4; }
-  while (m % 2 == 0) { if (!push(2)) return false; m /= 2; }
-  for (int r : {17, 13, 11, 7})
+  for (int r : {31, 29, 23, 19, 17, 13, 11, 7})
     while (m % r == 0) { if (!push(r)) return false; m /= r; }
   while (m % 15 == 0) { if (!push(15)) return false; m /= 15; }
   while (m % 9 == 0) { if (!push(9)) return false; m /= 9; }
   while (m % 5 == 0) { if (!push(5)) return false; m /= 5; }
   while (m % 3 == 0) { if (!push(3)) return false; m /= 3; }
+  for (int r : {16, 8, 4, 2})
+    while (m % r == 0) { if (!push(r)) return false; m /= r; }
   if (m != 1) return false;
-  int ns = 1;
+  int ns = 1, tw = 0;
   for (int s = 0; s < p.nstages; ++s) {
-    p.ns[s] = ns;
-    p.nsm[s] = magic(ns);
-    p.tws[s] = L / (ns * p.radix[s]);
-    ns *= p.radix[s];
+    p.st[s].ns = ns;
+    p.st[s].nsm = magic(ns);
+    p.st[s].tw = tw;
+    if (s > 0) tw += (p.st[s].radix - 1) * ns;
+    ns *= p.st[s].radix;
   }
   return true;
 }
@@ -568,13 +581,13 @@ static void host_fft_any(std::vector<std::complex<double>>& a) {
 }
 
 // Bluestein tables of line length L, convolution length M: the chirp
-// w_n = exp(-i pi (n^2 mod 2L) / L) and the kernel spectra FFT_M(b)/M of the
-// forward (b = conj w) and inverse (b = w) convolution kernels, wrapped so
-// that b_{M-m} = b_m.  Computed once in FP64 per (L, M) (the last pair is
+// w_n = exp(-i pi (n^2 mod 2L) / L) and the kernel spectrum FFT_M(b)/M of the
+// forward convolution kernel b = conj w, wrapped so that b_{M-m} = b_m (the
+// inverse kernel's is its conjugate).  Computed once in FP64 per (L, M) (the last pair is
 // kept, so the two precisions of a mixed handle share one computation).
 struct BluesteinHost {
   int L = 0, M = 0;
-  std::vector<std::complex<double>> w, bf, bi;
+  std::vector<std::complex<double>> w, bf;
 };
 
 static std::shared_ptr<const BluesteinHost> bluestein_host(int L, int M) {
@@ -597,18 +610,15 @@ static std::shared_ptr<const BluesteinHost> bluestein_host(int L, int M) {
     const double ang = -pi * ((double)q / (double)L);
     t.w[(size_t)n] = std::complex<double>(std::cos(ang), std::sin(ang));
   }
-  // kernel spectra: b is symmetric (b_{M-m} = b_m), so FFT(conj b) =
-  // conj(FFT(b)) and one transform gives both
+  // kernel spectrum: w is even (w_{M-m} = w_m), so FFT(conj w) = conj(FFT(w))
   std::vector<std::complex<double>> b((size_t)M, 0.0);
   for (int m = 0; m < L; ++m) {
     b[(size_t)m] = t.w[(size_t)m];
     if (m > 0) b[(size_t)(M - m)] = t.w[(size_t)m];
   }
   host_fft_any(b);
-  for (auto& x : b) x /= (double)M;
-  t.bf.resize(b.size());
-  for (size_t i = 0; i < b.size(); ++i) t.bf[i] = std::conj(b[i]);
-  t.bi.swap(b);
+  for (auto& x : b) x = std::conj(x / (double)M);
+  t.bf.swap(b);
   std::lock_guard<std::mutex> lock(mu);
   last = tp;
   return last;
@@ -625,25 +635,23 @@ static int upload_cpx(const std::vector<std::complex<double>>& v, void** out) {
 }
 
 template <typename T>
-static int upload_bluestein(int L, int M, void** chirp, void** bfw, void** binv) {
+static int upload_bluestein(int L, int M, void** chirp, void** bfw) {
   const std::shared_ptr<const BluesteinHost> t = bluestein_host(L, M);
   CHK(upload_cpx<T>(t->w, chirp));
   CHK(upload_cpx<T>(t->bf, bfw));
-  CHK(upload_cpx<T>(t->bi, binv));
   return CSIPM_OK;
 }
 
 // Rader tables of a prime length p with primitive root g: the permutation
 // perm[e] = q for e = g^q mod p (e = 1..p-1), perm[0] = p - 1 (the x_0 row
 // after the p - 1 convolution rows),
-// perm[p + m] = g^-m mod p (m = 0..p-2), and the kernel spectra
-// FFT_{p-1}(b) / (p-1) of b_j = exp(-+2 pi i g^-j / p) (forward / inverse),
-// in FP64; the last length's tables are kept (both precisions of a mixed
+// perm[p + m] = g^-m mod p (m = 0..p-2), and the kernel spectrum
+// FFT_{p-1}(b) / (p-1) of b_j = exp(-2 pi i g^-j / p), in FP64; the last length's tables are kept (both precisions of a mixed
 // handle, and the axes of a cube, share one computation)
 struct RaderHost {
   int p = 0;
   std::vector<int> perm;
-  std::vector<std::complex<double>> bf, bi;
+  std::vector<std::complex<double>> bf;
 };
 
 static int primitive_root(int p) {
@@ -688,21 +696,17 @@ static std::shared_ptr<const RaderHost> rader_host(int p) {
   int64_t e = 1, einv = 1;
   std::vector<std::complex<double>> roots;
   unit_roots(p, roots, p);   // exp(-2 pi i t / p)
-  std::vector<std::complex<double>> bf((size_t)p - 1), bi((size_t)p - 1);
+  std::vector<std::complex<double>> bf((size_t)p - 1);
   for (int q = 0; q < p - 1; ++q) {
     t.perm[(size_t)e] = q;                  // e = g^q
     t.perm[(size_t)p + q] = (int)einv;      // g^-q
     bf[(size_t)q] = roots[(size_t)einv];
-    bi[(size_t)q] = std::conj(roots[(size_t)einv]);
     e = e * g % p;
     einv = einv * ginv % p;
   }
   host_fft_any(bf);
-  host_fft_any(bi);
   for (auto& x : bf) x /= (double)(p - 1);
-  for (auto& x : bi) x /= (double)(p - 1);
   t.bf.swap(bf);
-  t.bi.swap(bi);
   std::lock_guard<std::mutex> lock(mu);
   last = tp;
   return last;
@@ -717,14 +721,15 @@ static int upload_rader_perm(int p, int** perm) {
 }
 
 template <typename T>
-static int upload_rader(int p, void** bfw, void** binv) {
+static int upload_rader(int p, void** bfw) {
   const std::shared_ptr<const RaderHost> t = rader_host(p);
   CHK(upload_cpx<T>(t->bf, bfw));
-  CHK(upload_cpx<T>(t->bi, binv));
   return CSIPM_OK;
 }
 
-// exp(-2 pi i t / L), t < L, in the op precision.  Tables are shared by the
+// Twiddles in the op precision: exp(-2 pi i t / L), t < L, in their order
+// (plan null; the four-step passes' table) or laid out for the stages of a
+// plan (FftStage::tw; L - radix_0 entries).  Tables are shared by the
 // handles on a device and counted: a table no handle holds stays cached
 // (a serving process meets the same lengths again) until the unheld tables
 // exceed kTwiddleKeepBytes, when the least recently used go back to the
@@ -747,10 +752,12 @@ static size_t g_tw_unheld_bytes = 0;
 static uint64_t g_tw_clock = 0;
 
 template <typename T>
-static int upload_twiddles(int L, void** out) {
+static int upload_twiddles(int L, const FftPlan* plan, void** out) {
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
-  const int64_t key = ((int64_t)dev << 40) | ((int64_t)sizeof(T) << 32) | (int64_t)L;
+  const int64_t layout = plan ? 1 + plan->variant : 0;
+  const int64_t key = ((int64_t)dev << 48) | (layout << 40) | ((int64_t)sizeof(T) << 32) |
+                      (int64_t)L;
   // an existing table with no holder is in the unheld set (a new one is not)
   auto hold = [&](TwiddleEntry& e, bool fresh) {
     if (e.refs == 0 && !fresh) {
@@ -772,8 +779,19 @@ static int upload_twiddles(int L, void** out) {
   // a new table: computed and uploaded without holding the cache lock
   std::vector<std::complex<double>> r;
   unit_roots(L, r, L);
-  std::vector<cpx<T>> h((size_t)L);
-  for (int t = 0; t < L; ++t) h[(size_t)t] = {(T)r[(size_t)t].real(), (T)r[(size_t)t].imag()};
+  std::vector<cpx<T>> h;
+  h.reserve((size_t)L);
+  auto put = [&](int64_t t) { h.push_back({(T)r[(size_t)t].real(), (T)r[(size_t)t].imag()}); };
+  if (!plan)
+    for (int t = 0; t < L; ++t) put(t);
+  else
+    for (int s = 1; s < plan->nstages; ++s) {
+      const int R = plan->st[s].radix, ns = plan->st[s].ns;
+      const int64_t step = L / ((int64_t)ns * R);
+      for (int q = 1; q < R; ++q)
+        for (int k = 0; k < ns; ++k) put(q * k * step);
+    }
+  h.resize((size_t)L);
   void* p = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_capture_mu);
@@ -832,11 +850,10 @@ static void release_twiddles(void* p) {
 // (csipm.tune, persisted in a committed table and loaded at start-up): for a
 // pass kind (0: line pass, 1: dimension-1 pass), the complex element size,
 // the FFT length W and the LDS rows R of a line, the largest tile (log2 of
-// the lines or line pairs per workgroup) and the workgroup size (128 or
-// 256).  Shapes without an entry keep the built-in rules.
+// the lines or line pairs per workgroup).  Shapes without an entry keep the
+// built-in rules.
 struct TuneVal {
   int lg_cap = 30;
-  int nt = 0;   // 0: the built-in choice
 };
 static std::mutex g_tune_mu;
 static std::map<std::tuple<int, int, int, int>, TuneVal> g_tune;
@@ -867,7 +884,7 @@ static LineCfg line_cfg(int H1, int W, int R, int64_t others, size_t cs,
                         int min_grid = 1024, int lg_cap = 30) {
   LineCfg c{};
   int lg = 0;
-  while ((2 << lg) * W <= kNT * kE && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
+  while (tile_grows(lg, W, cs) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
          lg < lg_cap)
     ++lg;
   // below 64-byte rows only while the launch would not even give a
@@ -880,6 +897,7 @@ static LineCfg line_cfg(int H1, int W, int R, int64_t others, size_t cs,
   c.ntile1 = (H1 + (1 << lg) - 1) >> lg;
   c.grid = (int)(c.ntile1 * others);
   c.lds = (size_t)(1 << lg) * R * cs;
+  c.nt = tile_nt((int64_t)W << lg);
   return c;
 }
 
@@ -887,7 +905,7 @@ static LineCfg line_cfg(int H1, int W, int R, int64_t others, size_t cs,
 static LineCfg col_cfg(int A, int B, size_t cs, int min_grid = 1024) {
   LineCfg c{};
   int lg = 0;
-  while ((2 << lg) * B <= kNT * kE && (size_t)(2 << lg) * B * cs <= kLdsSmall && (2 << lg) <= A)
+  while (tile_grows(lg, B, cs) && (size_t)(2 << lg) * B * cs <= kLdsSmall && (2 << lg) <= A)
     ++lg;
   const int lg_min = std::min(lg, min_tile_lg(cs));
   auto grid_of = [&](int l) { return (A + (1 << l) - 1) >> l; };
@@ -896,21 +914,22 @@ static LineCfg col_cfg(int A, int B, size_t cs, int min_grid = 1024) {
   c.ntile1 = (A + (1 << lg) - 1) >> lg;
   c.grid = c.ntile1;
   c.lds = (size_t)(1 << lg) * B * cs;
+  c.nt = tile_nt((int64_t)B << lg);
   return c;
 }
 
 // four-step row pass: 2^lg rows of length A per workgroup (LDS stride padded)
 static Dim1Cfg row_cfg(int A, int B, size_t cs, int min_grid = 1024) {
   Dim1Cfg c{};
-  c.nt = kNT;
   int lg = 0;
   auto lds_of = [&](int l) { return (size_t)A * ((1 << l) + 1) * cs; };
-  while ((2 << lg) * A <= kNT * kE && lds_of(lg + 1) <= kLdsSmall && (2 << lg) <= B) ++lg;
+  while ((2 << lg) * A <= kTileGrow && lds_of(lg + 1) <= kLdsSmall && (2 << lg) <= B) ++lg;
   while (lg > 0 && ((B + (1 << lg) - 1) >> lg) < min_grid) --lg;
   c.lg = lg;
   c.ps = (1 << lg) + 1;
   c.grid = (B + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
+  c.nt = tile_nt((int64_t)A << lg);
   return c;
 }
 
@@ -918,10 +937,9 @@ static Dim1Cfg dim1_cfg(int W, int R, int nlines, size_t cs, int min_grid = 1024
                         int lg_cap = 30) {
   Dim1Cfg c{};
   c.npairs = (nlines + 1) / 2;
-  c.nt = (W <= kNT * kE) ? kNT : kNTBig;
   int lg = 0;
   auto lds_of = [&](int l) { return (size_t)R * ((1 << l) + (l > 0 ? 1 : 0)) * cs; };
-  while ((2 << lg) * W <= c.nt * kE && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
+  while ((2 << lg) * W <= kTileGrow && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
          lg < lg_cap)
     ++lg;
   while (lg > 0 && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
@@ -929,6 +947,7 @@ static Dim1Cfg dim1_cfg(int W, int R, int nlines, size_t cs, int min_grid = 1024
   c.ps = (1 << lg) + (lg > 0 ? 1 : 0);
   c.grid = (c.npairs + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
+  c.nt = tile_nt((int64_t)W << lg);
   return c;
 }
 
@@ -977,7 +996,6 @@ PassArgs<T> base_args(csipm_op* h, int axis) {
   a.rperm = h->rperm[axis];
   a.chirp = (const cpx<T>*)h->ps<T>().chirp[axis];
   a.bfw = (const cpx<T>*)h->ps<T>().bfw[axis];
-  a.binv = (const cpx<T>*)h->ps<T>().binv[axis];
   return a;
 }
 
@@ -1017,15 +1035,21 @@ PassArgs<T> dim1_args(csipm_op* h, const void* src, const T* real_in, T* real_ou
   return a;
 }
 
+#define CSIPM_PASS(NT, kern)                                                 \
+  do {                                                                       \
+    auto kern_ = kern;                                                       \
+    CHK(allow_lds(kern_, c.lds));                                            \
+    hipLaunchKernelGGL(kern_, dim3(c.grid), dim3(NT), c.lds, h->stream, a);  \
+    HIPCHK(hipGetLastError());                                               \
+    return CSIPM_OK;                                                         \
+  } while (0)
+
 template <typename T, int D, int SRC, int DST, bool FWD>
 int launch_lines(csipm_op* h, int axis, const void* src, const Epi<T>& epi, const int* done) {
   const LineCfg& c = h->ps<T>().lines[axis];
   PassArgs<T> a = lines_args<T>(h, axis, src, epi, done);
-  auto kern = k_lines<T, kNT, kE, D, SRC, DST, FWD>;
-  CHK(allow_lds(kern, c.lds));
-  hipLaunchKernelGGL(kern, dim3(c.grid), dim3(kNT), c.lds, h->stream, a);
-  HIPCHK(hipGetLastError());
-  return CSIPM_OK;
+  if (c.nt == 256) CSIPM_PASS(256, (k_lines<T, 256, kE, D, SRC, DST, FWD>));
+  CSIPM_PASS(512, (k_lines<T, 512, kE, D, SRC, DST, FWD>));
 }
 
 template <typename T, int D, int SRC, int DST, int MODE>
@@ -1033,17 +1057,12 @@ int launch_dim1(csipm_op* h, const void* src, const T* real_in, T* real_out, con
                 T scale, const int* done) {
   const Dim1Cfg& c = h->ps<T>().d1;
   PassArgs<T> a = dim1_args<T>(h, src, real_in, real_out, epi, scale, done);
-  if (c.nt == kNT) {
-    auto kern = k_dim1<T, kNT, kE, D, SRC, DST, MODE>;
-    CHK(allow_lds(kern, c.lds));
-    hipLaunchKernelGGL(kern, dim3(c.grid), dim3(kNT), c.lds, h->stream, a);
-  } else {
-    auto kern = k_dim1<T, kNTBig, kE, D, SRC, DST, MODE>;
-    CHK(allow_lds(kern, c.lds));
-    hipLaunchKernelGGL(kern, dim3(c.grid), dim3(kNTBig), c.lds, h->stream, a);
+  switch (c.nt) {
+    case 256: CSIPM_PASS(256, (k_dim1<T, 256, kE, D, SRC, DST, MODE>));
+    case 512: CSIPM_PASS(512, (k_dim1<T, 512, kE, D, SRC, DST, MODE>));
+    case 1024: CSIPM_PASS(1024, (k_dim1<T, 1024, kE, D, SRC, DST, MODE>));
+    default: CSIPM_PASS(1024, (k_dim1<T, 1024, 16, D, SRC, DST, MODE>));
   }
-  HIPCHK(hipGetLastError());
-  return CSIPM_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1137,33 +1156,35 @@ int launch_big_pass(csipm_op* h, const PassSpec& sp, const PassArgs<T>& a) {
   const PrecState& ps = h->ps<T>();
   const int grid = sp.kind == PK_COL ? ps.col.grid : ps.row.grid;
   const size_t lds = sp.kind == PK_COL ? ps.col.lds : ps.row.lds;
-#define CSIPM_BIG(kern)                                                      \
+  const int nt = sp.kind == PK_COL ? ps.col.nt : ps.row.nt;
+#define CSIPM_BIG(K, ...)                                                    \
   do {                                                                       \
+    auto kern = nt == 256 ? K<T, 256, kE, __VA_ARGS__> : K<T, 512, kE, __VA_ARGS__>; \
     CHK(allow_lds(kern, lds));                                               \
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kNT), lds, h->stream, a);      \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, h->stream, a);       \
     HIPCHK(hipGetLastError());                                               \
     return CSIPM_OK;                                                         \
   } while (0)
   if (sp.kind == PK_COL) {
     switch (sp.fm) {
       case C_FIRST:
-        if (sp.src == SRC_BETA) CSIPM_BIG((k_col<T, kNT, kE, SRC_BETA, DST_BUF, C_FIRST>));
-        CSIPM_BIG((k_col<T, kNT, kE, SRC_U, DST_BUF, C_FIRST>));
-      case C_REAL_IN: CSIPM_BIG((k_col<T, kNT, kE, SRC_REAL, DST_BUF, C_REAL_IN>));
-      case C_MID: CSIPM_BIG((k_col<T, kNT, kE, SRC_BUF, DST_BUF, C_MID>));
-      case C_MID_C2R: CSIPM_BIG((k_col<T, kNT, kE, SRC_BUF, DST_REAL, C_MID_C2R>));
+        if (sp.src == SRC_BETA) CSIPM_BIG(k_col, SRC_BETA, DST_BUF, C_FIRST);
+        CSIPM_BIG(k_col, SRC_U, DST_BUF, C_FIRST);
+      case C_REAL_IN: CSIPM_BIG(k_col, SRC_REAL, DST_BUF, C_REAL_IN);
+      case C_MID: CSIPM_BIG(k_col, SRC_BUF, DST_BUF, C_MID);
+      case C_MID_C2R: CSIPM_BIG(k_col, SRC_BUF, DST_REAL, C_MID_C2R);
       case C_LAST:
-        if (sp.dst == DST_BETA) CSIPM_BIG((k_col<T, kNT, kE, SRC_BUF, DST_BETA, C_LAST>));
-        CSIPM_BIG((k_col<T, kNT, kE, SRC_BUF, DST_U, C_LAST>));
+        if (sp.dst == DST_BETA) CSIPM_BIG(k_col, SRC_BUF, DST_BETA, C_LAST);
+        CSIPM_BIG(k_col, SRC_BUF, DST_U, C_LAST);
       default: break;
     }
   } else {
     switch (sp.fm) {
-      case R_MTM: CSIPM_BIG((k_row<T, kNT, kE, R_MTM>));
-      case R_C2R: CSIPM_BIG((k_row<T, kNT, kE, R_C2R>));
-      case R_R2C: CSIPM_BIG((k_row<T, kNT, kE, R_R2C>));
-      case R_CONV_INV: CSIPM_BIG((k_row<T, kNT, kE, R_CONV_INV>));
-      case R_CONV_FWD: CSIPM_BIG((k_row<T, kNT, kE, R_CONV_FWD>));
+      case R_MTM: CSIPM_BIG(k_row, R_MTM);
+      case R_C2R: CSIPM_BIG(k_row, R_C2R);
+      case R_R2C: CSIPM_BIG(k_row, R_R2C);
+      case R_CONV_INV: CSIPM_BIG(k_row, R_CONV_INV);
+      case R_CONV_FWD: CSIPM_BIG(k_row, R_CONV_FWD);
       default: break;
     }
   }
@@ -1768,7 +1789,7 @@ static void destroy_impl(csipm_op_t h) {
   std::vector<void*> blocks;
   for (PrecState* ps : {&h->p64, &h->p32})
     for (int i = 0; i < 3; ++i)
-      for (void* b : {ps->chirp[i], ps->bfw[i], ps->binv[i]})
+      for (void* b : {ps->chirp[i], ps->bfw[i]})
         if (b) blocks.push_back(b);
   for (int i = 0; i < 3; ++i)
     if (h->rperm[i]) blocks.push_back(h->rperm[i]);
@@ -1810,11 +1831,11 @@ static int plan_big1d(csipm_op* h) {
     F = 1;
     while (F < 2 * N - 1) F <<= 1;
   }
-  // the most balanced divisor pair with both factors <= kNT * kE
+  // the most balanced divisor pair with both factors <= kTile
   for (int b = 1; (int64_t)b * b <= F; ++b) {
     if (F % b) continue;
     const int a = F / b;
-    if (a <= kNT * kE && b <= kNT * kE) {
+    if (a <= kTile && b <= kTile) {
       A = a;
       B = b;
     }
@@ -1836,15 +1857,15 @@ static int upload_big1d(csipm_op* h) {
     const bool want = ps == &h->p64 ? h->has64() : h->has32();
     if (!want) continue;
     if (ps == &h->p64) {
-      CHK(upload_twiddles<double>(A, &ps->twA));
-      CHK(upload_twiddles<double>(B, &ps->twB));
-      CHK(upload_twiddles<double>(F, &ps->tw[0]));
-      if (h->obs) CHK(upload_bluestein<double>(N, F, &ps->chirp[0], &ps->bfw[0], &ps->binv[0]));
+      CHK(upload_twiddles<double>(A, &h->planA, &ps->twA));
+      CHK(upload_twiddles<double>(B, &h->planB, &ps->twB));
+      CHK(upload_twiddles<double>(F, nullptr, &ps->tw[0]));
+      if (h->obs) CHK(upload_bluestein<double>(N, F, &ps->chirp[0], &ps->bfw[0]));
     } else {
-      CHK(upload_twiddles<float>(A, &ps->twA));
-      CHK(upload_twiddles<float>(B, &ps->twB));
-      CHK(upload_twiddles<float>(F, &ps->tw[0]));
-      if (h->obs) CHK(upload_bluestein<float>(N, F, &ps->chirp[0], &ps->bfw[0], &ps->binv[0]));
+      CHK(upload_twiddles<float>(A, &h->planA, &ps->twA));
+      CHK(upload_twiddles<float>(B, &h->planB, &ps->twB));
+      CHK(upload_twiddles<float>(F, nullptr, &ps->tw[0]));
+      if (h->obs) CHK(upload_bluestein<float>(N, F, &ps->chirp[0], &ps->bfw[0]));
     }
   }
   return CSIPM_OK;
@@ -1863,13 +1884,13 @@ static int set_shapes(csipm_op* h, PrecState& ps, size_t cs) {
   // dim-1 line (L, M, Rader's 2L + 1)
   const int F0 = h->plan[0].L;
   ps.d1 = dim1_cfg(F0, h->rows[0], (int)(h->N / h->n[0]), cs);
-  if (ps.d1.nt * kE < F0 || ps.d1.lds > kLdsMax)
+  if (F0 > kTileLong || ps.d1.lds > kLdsMax)
     return fail(CSIPM_ERR_UNSUPPORTED, "dimension-1 length %d (FFT length %d) exceeds one "
                 "workgroup", h->n[0], F0);
   if (dim >= 2) ps.lines[1] = line_cfg(h->H1, h->plan[1].L, h->rows[1], h->n[2], cs);
   if (dim == 3) ps.lines[2] = line_cfg(h->H1, h->plan[2].L, h->rows[2], h->n[1], cs);
   for (int ax = 1; ax < dim; ++ax)
-    if (h->plan[ax].L > kNT * kE || ps.lines[ax].lds > kLdsMax)
+    if (h->plan[ax].L > kTile || ps.lines[ax].lds > kLdsMax)
       return fail(CSIPM_ERR_UNSUPPORTED, "dimension-%d length %d (%d LDS rows) exceeds one "
                   "workgroup", ax + 1, h->n[ax], h->rows[ax]);
   return CSIPM_OK;
@@ -1932,11 +1953,11 @@ static size_t handle_own_bytes(const csipm_op* h) {
     if (!(p == 0 ? h->has64() : h->has32())) continue;
     const size_t cs = p == 0 ? sizeof(cpx<double>) : sizeof(cpx<float>);
     if (h->big) {
-      if (h->obs) b += cs * ((size_t)h->n[0] + 2 * (size_t)h->bF);
+      if (h->obs) b += cs * ((size_t)h->n[0] + (size_t)h->bF);
     } else {
       for (int i = 0; i < h->dim; ++i) {
-        if (h->bs[i] == 1) b += cs * ((size_t)h->n[i] + 2 * (size_t)h->plan[i].L);
-        if (h->bs[i] == 2) b += cs * 2 * (size_t)h->plan[i].L + 8 * (size_t)h->n[i];
+        if (h->bs[i] == 1) b += cs * ((size_t)h->n[i] + (size_t)h->plan[i].L);
+        if (h->bs[i] == 2) b += cs * (size_t)h->plan[i].L + 8 * (size_t)h->n[i];
       }
     }
   }
@@ -1954,20 +1975,18 @@ static int create_impl(csipm_op* h, int dim, const int64_t sizes[3], int rdft, i
   if (h->big) CHK(upload_big1d(h));
   for (int i = 0; i < dim && !h->big; ++i) {
     const int F = h->plan[i].L;
-    if (h->has64()) CHK(upload_twiddles<double>(F, &h->p64.tw[i]));
-    if (h->has32()) CHK(upload_twiddles<float>(F, &h->p32.tw[i]));
+    if (h->has64()) CHK(upload_twiddles<double>(F, &h->plan[i], &h->p64.tw[i]));
+    if (h->has32()) CHK(upload_twiddles<float>(F, &h->plan[i], &h->p32.tw[i]));
     if (h->bs[i] == 2) {
       CHK(upload_rader_perm(h->n[i], &h->rperm[i]));
-      if (h->has64()) CHK(upload_rader<double>(h->n[i], &h->p64.bfw[i], &h->p64.binv[i]));
-      if (h->has32()) CHK(upload_rader<float>(h->n[i], &h->p32.bfw[i], &h->p32.binv[i]));
+      if (h->has64()) CHK(upload_rader<double>(h->n[i], &h->p64.bfw[i]));
+      if (h->has32()) CHK(upload_rader<float>(h->n[i], &h->p32.bfw[i]));
     }
     if (h->bs[i] == 1) {
       if (h->has64())
-        CHK(upload_bluestein<double>(h->n[i], F, &h->p64.chirp[i], &h->p64.bfw[i],
-                                     &h->p64.binv[i]));
+        CHK(upload_bluestein<double>(h->n[i], F, &h->p64.chirp[i], &h->p64.bfw[i]));
       if (h->has32())
-        CHK(upload_bluestein<float>(h->n[i], F, &h->p32.chirp[i], &h->p32.bfw[i],
-                                    &h->p32.binv[i]));
+        CHK(upload_bluestein<float>(h->n[i], F, &h->p32.chirp[i], &h->p32.bfw[i]));
     }
   }
   {
@@ -2070,7 +2089,7 @@ int csipm_op_fft_shape(csipm_op_t h, int axis, int* fft_len, int* rows, int* mod
 
 int csipm_tune_set(int kind, int elem_bytes, int fft_len, int rows, int lg_cap, int nt) {
   if ((kind != 0 && kind != 1) || (elem_bytes != 8 && elem_bytes != 16) || fft_len < 1 ||
-      rows < fft_len || (nt != 0 && nt != kNTSmall && nt != kNT))
+      rows < fft_len || (nt != 0 && nt != 128 && nt != 256))
     return fail(CSIPM_ERR_ARG, "bad tuning entry");
   std::lock_guard<std::mutex> lk(g_tune_mu);
   const auto key = std::make_tuple(kind, elem_bytes, fft_len, rows);
@@ -2080,7 +2099,6 @@ int csipm_tune_set(int kind, int elem_bytes, int fft_len, int rows, int lg_cap, 
   }
   TuneVal v;
   v.lg_cap = lg_cap;
-  v.nt = nt;
   g_tune[key] = v;
   return CSIPM_OK;
 }

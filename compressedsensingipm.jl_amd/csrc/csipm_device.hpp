@@ -25,11 +25,11 @@ template <typename T>
 __device__ __forceinline__ cpx<T> cmul(cpx<T> a, cpx<T> b) {
   return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
-// multiply by -i (FWD) or +i (inverse)
-template <typename T, bool FWD>
-__device__ __forceinline__ cpx<T> mul_mi(cpx<T> a) {
-  return FWD ? cpx<T>{a.y, -a.x} : cpx<T>{-a.y, a.x};
-}
+template <typename T>
+__device__ __forceinline__ cpx<T> mul_mi(cpx<T> a) { return {a.y, -a.x}; }   // a * (-i)
+// real and imaginary part exchanged: swap(DFT(swap(x))) is the inverse DFT
+template <typename T>
+__device__ __forceinline__ cpx<T> cswap(cpx<T> a) { return {a.y, a.x}; }
 
 // ---------------------------------------------------------------------------
 // Packing geometry.  Per dimension d of length n: M = n/2, P = (n-1)/2,
@@ -220,38 +220,38 @@ __host__ __device__ __forceinline__ bool scatter_targets(int k1, int k2, int k3,
 }
 
 // ---------------------------------------------------------------------------
-// Radix-R DFT butterflies on registers.  FWD: exp(-2 pi i jk/R).
+// Radix-R DFT butterflies on registers, forward: exp(-2 pi i jk/R).  There is
+// no inverse form: inverse = swap . forward . swap with swap exchanging real
+// and imaginary parts, which the passes fold into their LDS loads and stores.
 // ---------------------------------------------------------------------------
-template <typename T, bool FWD>
+template <typename T>
 __device__ __forceinline__ void dft2(cpx<T>* v) {
   cpx<T> a = v[0], b = v[1];
   v[0] = cadd(a, b);
   v[1] = csub(a, b);
 }
 
-template <typename T, bool FWD>
+template <typename T>
 __device__ __forceinline__ void dft4(cpx<T>* v) {
   cpx<T> t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-  cpx<T> t2 = cadd(v[1], v[3]), t3 = mul_mi<T, FWD>(csub(v[1], v[3]));
+  cpx<T> t2 = cadd(v[1], v[3]), t3 = mul_mi(csub(v[1], v[3]));
   v[0] = cadd(t0, t2);
   v[2] = csub(t0, t2);
   v[1] = cadd(t1, t3);
   v[3] = csub(t1, t3);
 }
 
-template <typename T, bool FWD>
+template <typename T>
 __device__ __forceinline__ void dft8(cpx<T>* v) {
   cpx<T> e[4] = {v[0], v[2], v[4], v[6]};
   cpx<T> o[4] = {v[1], v[3], v[5], v[7]};
-  dft4<T, FWD>(e);
-  dft4<T, FWD>(o);
+  dft4(e);
+  dft4(o);
   const T h = (T)0.70710678118654752440;
-  // w^1 = (h, -+h), w^2 = -+i, w^3 = (-h, -+h)
-  cpx<T> w1o = FWD ? cpx<T>{h * (o[1].x + o[1].y), h * (o[1].y - o[1].x)}
-                   : cpx<T>{h * (o[1].x - o[1].y), h * (o[1].y + o[1].x)};
-  cpx<T> w2o = mul_mi<T, FWD>(o[2]);
-  cpx<T> w3o = FWD ? cpx<T>{h * (-o[3].x + o[3].y), h * (-o[3].y - o[3].x)}
-                   : cpx<T>{h * (-o[3].x - o[3].y), h * (-o[3].y + o[3].x)};
+  // w^1 = (h, -h), w^2 = -i, w^3 = (-h, -h)
+  cpx<T> w1o = {h * (o[1].x + o[1].y), h * (o[1].y - o[1].x)};
+  cpx<T> w2o = mul_mi(o[2]);
+  cpx<T> w3o = {h * (-o[3].x + o[3].y), h * (-o[3].y - o[3].x)};
   v[0] = cadd(e[0], o[0]);
   v[4] = csub(e[0], o[0]);
   v[1] = cadd(e[1], w1o);
@@ -262,7 +262,7 @@ __device__ __forceinline__ void dft8(cpx<T>* v) {
   v[7] = csub(e[3], w3o);
 }
 
-template <typename T, bool FWD>
+template <typename T>
 __device__ __forceinline__ void dft16(cpx<T>* v) {
   // 4 x 4: columns of stride 4, twiddle, rows
   cpx<T> a[4][4];
@@ -270,13 +270,11 @@ __device__ __forceinline__ void dft16(cpx<T>* v) {
   for (int q = 0; q < 4; ++q) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) a[q][p] = v[q + 4 * p];
-    dft4<T, FWD>(a[q]);
+    dft4(a[q]);
   }
   // twiddle a[q][p] *= w16^(q*p)
   const T c1 = (T)0.92387953251128675613, s1 = (T)0.38268343236508977173;
   const T h = (T)0.70710678118654752440;
-  const T cs[10] = {1, c1, h, s1, 0, -s1, -h, -c1, -1, 0};
-  (void)cs;
 #pragma unroll
   for (int q = 1; q < 4; ++q) {
 #pragma unroll
@@ -291,23 +289,22 @@ __device__ __forceinline__ void dft16(cpx<T>* v) {
         case 6: c = -h; s = h; break;
         default: c = -c1; s = -s1; break;  // m == 9: angle 9*pi/8 -> cos=-c1, sin=-s1
       }
-      const T sg = FWD ? -s : s;
-      cpx<T> w = {c, sg};
+      const cpx<T> w = {c, -s};
       a[q][p] = cmul(a[q][p], w);
     }
   }
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     cpx<T> r[4] = {a[0][p], a[1][p], a[2][p], a[3][p]};
-    dft4<T, FWD>(r);
+    dft4(r);
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[p + 4 * q] = r[q];
   }
 }
 
-// odd R = 2H+1: X[k] = x0 + sum_j a_j cos(2pi jk/R) -/+ i sum_j b_j sin(2pi jk/R)
+// odd R = 2H+1: X[k] = x0 + sum_j a_j cos(2pi jk/R) - i sum_j b_j sin(2pi jk/R)
 // with a_j = x_j + x_{R-j}, b_j = x_j - x_{R-j}
-template <typename T, int R, bool FWD>
+template <typename T, int R>
 __device__ __forceinline__ void dft_odd(cpx<T>* v) {
   constexpr int H = (R - 1) / 2;
   cpx<T> a[H], b[H];
@@ -333,22 +330,15 @@ __device__ __forceinline__ void dft_odd(cpx<T>* v) {
       sre += b[j - 1].y * s;
       sim += b[j - 1].x * s;
     }
-    if (FWD) {
-      v[k] = {re + sre, im - sim};
-      v[R - k] = {re - sre, im + sim};
-    } else {
-      v[k] = {re - sre, im + sim};
-      v[R - k] = {re + sre, im - sim};
-    }
+    v[k] = {re + sre, im - sim};
+    v[R - k] = {re - sre, im + sim};
   }
   v[0] = y0;
 }
 
 // the same, writing X[k] to dst[k * stride] as it is formed: a_j and b_j
-// overwrite the inputs in place and no output array is held, which keeps the
-// large odd radices (11, 13, 15, 17) within the register budget of the small
-// ones
-template <typename T, int R, bool FWD>
+// overwrite the inputs in place and no output array is held
+template <typename T, int R>
 __device__ __forceinline__ void dft_odd_store(cpx<T>* v, cpx<T>* __restrict__ dst, int stride) {
   constexpr int H = (R - 1) / 2;
   const cpx<T> x0 = v[0];
@@ -362,36 +352,42 @@ __device__ __forceinline__ void dft_odd_store(cpx<T>* v, cpx<T>* __restrict__ ds
     y0 = cadd(y0, a);
   }
   dst[0] = y0;
-#pragma unroll
-  for (int k = 1; k <= H; ++k) {
+  auto output = [&](int k, const auto& c, const auto& s) {
     T re = x0.x, im = x0.y, sre = 0, sim = 0;
 #pragma unroll
     for (int j = 1; j <= H; ++j) {
-      const int m = (j * k) % R;
-      const T c = (T)OddRadix<R>::c[m];
-      const T sn = (T)OddRadix<R>::s[m];
-      re += v[j].x * c;
-      im += v[j].y * c;
-      sre += v[R - j].y * sn;
-      sim += v[R - j].x * sn;
+      re += v[j].x * c(j);
+      im += v[j].y * c(j);
+      sre += v[R - j].y * s(j);
+      sim += v[R - j].x * s(j);
     }
-    if (FWD) {
-      dst[k * stride] = {re + sre, im - sim};
-      dst[(R - k) * stride] = {re - sre, im + sim};
-    } else {
-      dst[k * stride] = {re - sre, im + sim};
-      dst[(R - k) * stride] = {re + sre, im - sim};
+    dst[k * stride] = {re + sre, im - sim};
+    dst[(R - k) * stride] = {re - sre, im + sim};
+  };
+  if constexpr (R < 17) {
+#pragma unroll
+    for (int k = 1; k <= H; ++k)
+      output(k, [&](int j) { return (T)OddRadix<R>::c[(j * k) % R]; },
+             [&](int j) { return (T)OddRadix<R>::s[(j * k) % R]; });
+  } else {
+    // a loop over the outputs, their coefficients by scalar loads: unrolled,
+    // the (H x H) products were scheduled across outputs and spilled hundreds
+    // of registers in FP64 (and radix 31 alone was 900 instructions)
+#pragma unroll 1
+    for (int k = 1; k <= H; ++k) {
+      const T* row = OddRows<T, R>::cs[k - 1];
+      output(k, [&](int j) { return row[j - 1]; }, [&](int j) { return row[H + j - 1]; });
     }
   }
 }
 
-template <typename T, int R, bool FWD>
+template <typename T, int R>
 __device__ __forceinline__ void dft(cpx<T>* v) {
-  if constexpr (R == 2) dft2<T, FWD>(v);
-  else if constexpr (R == 4) dft4<T, FWD>(v);
-  else if constexpr (R == 8) dft8<T, FWD>(v);
-  else if constexpr (R == 16) dft16<T, FWD>(v);
-  else dft_odd<T, R, FWD>(v);
+  if constexpr (R == 2) dft2(v);
+  else if constexpr (R == 4) dft4(v);
+  else if constexpr (R == 8) dft8(v);
+  else if constexpr (R == 16) dft16(v);
+  else dft_odd<T, R>(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -399,22 +395,51 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
 // [element][line] order: element e of line l at lds[e * ps + l] (ps >= 2^lg,
 // the line stride, padded where the load loops would otherwise conflict).
 // Stage s with radix R after Ns = product of earlier radices: butterfly j
-// reads elements j + r*L/R, multiplies input r by w^(r*(j mod Ns)*L/(Ns*R)),
-// and writes elements (j - j mod Ns)*R + j mod Ns + r*Ns.  Butterflies are
+// reads elements j + r*L/R, multiplies input r by exp(-2 pi i r k/(Ns*R)),
+// k = j mod Ns, and writes elements (j - k)*R + k + r*Ns.  Butterflies are
 // numbered b = j * 2^lg + l, so the lines of a tile run on adjacent lanes and
-// share twiddles.  Each thread stages at most E elements per stage in
-// registers; the caller guarantees 2^lg * L <= NT * E.
+// share twiddles.  The caller guarantees 2^lg * L <= NT * E: a thread holds
+// max(E, R) complex values in a stage.
+// What bounds a stage: the number of waves a SIMD holds.  With E = 16 (two
+// radix-9..15 butterflies and their twiddles per thread) the FP64 passes
+// took 248-260 registers, one or two waves per SIMD, and the 1024-thread ones
+// spilled 1300 registers; E = 8 with the waves per SIMD asked for by
+// pass_waves() keeps three (FP64) or five (FP32; radices 29 and 31 spill some
+// tens of registers there).  Twiddles are laid out per stage in the order in
+// which adjacent lanes read them: strided reads from one table of the length
+// L cost a cache line per lane.
+// Measured (before -> after, with tile_grows' tiles): line passes of the FP64
+// 256^3 apply 72 -> 65 and 70 -> 57 us (270 MB each, 4.1-4.7 TB/s), its
+// dimension-1 pass 140 -> 123 us; 509 x 384 FP64 (Rader) 19 -> 13 us.
 // ---------------------------------------------------------------------------
-constexpr int kMaxStages = 20;
+constexpr int kMaxStages = 15;
 
+struct FftStage {
+  int radix;
+  int ns;        // product of the radices of earlier stages
+  int tw;        // first twiddle of the stage (ns > 1): w^(r k), k < ns, at tw + (r - 1) ns + k
+  uint32_t nsm;  // ceil(2^32 / ns), ns >= 2: j / ns = umulhi(j, nsm)
+};
+
+// 64 words: a wave holds the whole plan in one register, word l in lane l
+// (plan_word), so a stage's parameters cost no memory access.  Read from
+// memory stage by stage (the stores in between keep the compiler from scalar
+// loads), each stage waited for two dependent L1 / L2 round trips.
 struct FftPlan {
   int L;
   int nstages;
-  int radix[kMaxStages];
-  int ns[kMaxStages];        // product of the radices of earlier stages
-  int tws[kMaxStages];       // twiddle index stride L / (ns * radix)
-  uint32_t nsm[kMaxStages];  // ceil(2^32 / ns), ns >= 2: j / ns = umulhi(j, nsm)
+  int variant;   // which radix order (the host planner's, names the twiddle table)
+  int pad;
+  FftStage st[kMaxStages];
 };
+static_assert(sizeof(FftPlan) == 64 * sizeof(int), "one plan word per lane");
+
+__device__ __forceinline__ int plan_load(const FftPlan* __restrict__ p) {
+  return reinterpret_cast<const int*>(p)[threadIdx.x & 63];
+}
+__device__ __forceinline__ int plan_word(int pl, int w) {
+  return __builtin_amdgcn_readlane(pl, w);
+}
 
 // a wave-uniform value into a scalar register (the value must be uniform)
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -427,124 +452,128 @@ __device__ __forceinline__ int fdiv(int a, uint32_t m) { return (int)__umulhi((u
 // k = (10 k1 + 6 k2) mod 15, X = DFT3 over a of DFT5 over b (W15^(nk) =
 // W3^(a k1) W5^(b k2) for these maps).  3 five-point and 5 three-point
 // transforms instead of the 15-point pair form's 7 x 7 products.
-template <typename T, bool FWD>
+template <typename T>
 __device__ __forceinline__ void dft15_store(cpx<T>* v, cpx<T>* __restrict__ dst, int stride) {
   cpx<T> y[3][5];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
 #pragma unroll
     for (int b = 0; b < 5; ++b) y[a][b] = v[(5 * a + 3 * b) % 15];
-    dft_odd<T, 5, FWD>(y[a]);
+    dft_odd<T, 5>(y[a]);
   }
 #pragma unroll
   for (int k2 = 0; k2 < 5; ++k2) {
     cpx<T> z[3] = {y[0][k2], y[1][k2], y[2][k2]};
-    dft_odd<T, 3, FWD>(z);
+    dft_odd<T, 3>(z);
 #pragma unroll
     for (int k1 = 0; k1 < 3; ++k1) dst[((10 * k1 + 6 * k2) % 15) * stride] = z[k1];
   }
 }
 
-template <typename T, int R, int E, int NT, bool FWD>
-__device__ __forceinline__ void stockham_stage(cpx<T>* __restrict__ lds, const FftPlan& p, int s,
-                                               int lg, int ps, const cpx<T>* __restrict__ tw) {
+template <typename T, int R, int E, int NT>
+__device__ __forceinline__ void stockham_stage(cpx<T>* __restrict__ lds, int L, int Ns,
+                                               uint32_t nsm, int lg, int ps,
+                                               const cpx<T>* __restrict__ tw) {
   constexpr int NQ = (E + R - 1) / R;
-  const int L = uniform(p.L);
+  // twiddles loaded before the LDS reads they multiply (the rest, of the large
+  // radices, in groups as the registers allow)
+  constexpr int CH = sizeof(T) == 4 ? (R <= 17 ? R - 1 : 8) : (R <= 9 ? R - 1 : 6);
   const int nb = L / R;
   const int nl = 1 << lg;
   const int total = nb << lg;
-  const int Ns = uniform(p.ns[s]);
-  const int tws = uniform(p.tws[s]);
-  const uint32_t nsm = (uint32_t)uniform((int)p.nsm[s]);
   // an opaque copy of the lane index: keeps the compiler from hoisting every
   // stage's per-lane address arithmetic out of the caller's stage loop (the
   // hoisted values of all radix cases would stay live across the whole FFT)
   int tid = (int)threadIdx.x;
   asm volatile("" : "+v"(tid));
   cpx<T> v[NQ][R];
-  // radices up to 17: twiddle loads first (index clamped into the table for
-  // idle lanes), so that their latency overlaps the LDS reads and the barrier
-  // instead of following them.  Radices 19..31 load each twiddle where it is
-  // used: holding R of them beside the R inputs would exceed the registers
-  // of the FP64 kernels.
-  constexpr bool kAhead = R <= 17;
-  cpx<T> w[NQ][kAhead ? R : 1];
-  if (kAhead && Ns > 1) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int b = min(tid + q * NT, total - 1);
-      const int j = b >> lg;
-      const int step = (j - fdiv(j, nsm) * Ns) * tws;
-#pragma unroll
-      for (int r = 1; r < R; ++r) w[q][kAhead ? r : 0] = tw[r * step];
-    }
-  }
+  int out[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
+    // idle lanes read nothing: 16-byte reads of one address by many lanes are
+    // serialised (3000 cycles a stage when they repeated the last butterfly)
     const int b = tid + q * NT;
     if (b < total) {
       const int j = b >> lg;
       const int line = b & (nl - 1);
       const cpx<T>* src = lds + j * ps + line;
+      if (Ns > 1) {
+        const int k = j - fdiv(j, nsm) * Ns;
+        out[q] = ((j - k) * R + k) * ps + line;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = src[r * nb * ps];
+        for (int r0 = 1; r0 < R; r0 += CH) {
+          cpx<T> w[CH];
+#pragma unroll
+          for (int r = r0; r < r0 + CH && r < R; ++r) w[r - r0] = tw[(r - 1) * Ns + k];
+          if (r0 == 1) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[q][r] = src[r * nb * ps];
+          }
+#pragma unroll
+          for (int r = r0; r < r0 + CH && r < R; ++r) v[q][r] = cmul(v[q][r], w[r - r0]);
+        }
+      } else {
+        out[q] = j * R * ps + line;
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[q][r] = src[r * nb * ps];
+      }
     }
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    const int b = tid + q * NT;
-    if (b < total) {
-      const int j = b >> lg;
-      const int line = b & (nl - 1);
-      int k = 0;
-      if (Ns > 1) {
-        k = j - fdiv(j, nsm) * Ns;
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          cpx<T> t = kAhead ? w[q][kAhead ? r : 0] : tw[r * k * tws];
-          if (!FWD) t.y = -t.y;
-          v[q][r] = cmul(v[q][r], t);
-        }
-      }
-      cpx<T>* dst = lds + ((j - k) * R + k) * ps + line;
+    if (tid + q * NT < total) {
+      cpx<T>* dst = lds + out[q];
       if constexpr (R == 2 || R == 4 || R == 8 || R == 16) {
-        dft<T, R, FWD>(v[q]);
+        dft<T, R>(v[q]);
 #pragma unroll
         for (int r = 0; r < R; ++r) dst[r * Ns * ps] = v[q][r];
+      } else if constexpr (R == 15) {
+        dft15_store<T>(v[q], dst, Ns * ps);
       } else {
-        if constexpr (R == 15)
-          dft15_store<T, FWD>(v[q], dst, Ns * ps);
-        else
-          dft_odd_store<T, R, FWD>(v[q], dst, Ns * ps);
+        dft_odd_store<T, R>(v[q], dst, Ns * ps);
       }
     }
   }
   __syncthreads();
 }
 
-template <typename T, int E, int NT, bool FWD>
-__device__ __forceinline__ void lds_fft(cpx<T>* lds, const FftPlan& plan, int lg, int ps,
-                        const cpx<T>* __restrict__ tw) {
-  const int nst = uniform(plan.nstages);
+// waves per SIMD asked of the compiler for the pass kernels (of 512 registers
+// a SIMD lane: 96 per thread in FP32, 168 in FP64; a 1024-thread workgroup
+// needs four waves, 128 registers)
+template <typename T, int NT>
+constexpr int pass_waves() {
+  return NT >= 1024 ? 4 : sizeof(T) == 4 ? 5 : 3;
+}
+
+// forward DFT of the tile; pl: the wave's plan register (plan_load)
+template <typename T, int E, int NT>
+__device__ __forceinline__ void lds_fft(cpx<T>* lds, int pl, int lg, int ps,
+                                        const cpx<T>* __restrict__ tw) {
+  const int L = plan_word(pl, 0), nst = plan_word(pl, 1);
+#pragma unroll 1
   for (int s = 0; s < nst; ++s) {
-    switch (uniform(plan.radix[s])) {
-      case 2: stockham_stage<T, 2, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 3: stockham_stage<T, 3, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 4: stockham_stage<T, 4, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 5: stockham_stage<T, 5, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 7: stockham_stage<T, 7, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 8: stockham_stage<T, 8, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 9: stockham_stage<T, 9, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 11: stockham_stage<T, 11, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 13: stockham_stage<T, 13, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 15: stockham_stage<T, 15, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 16: stockham_stage<T, 16, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 17: stockham_stage<T, 17, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 19: stockham_stage<T, 19, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 23: stockham_stage<T, 23, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 29: stockham_stage<T, 29, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
-      case 31: stockham_stage<T, 31, E, NT, FWD>(lds, plan, s, lg, ps, tw); break;
+    const int w = 4 + 4 * s;
+    const int ns = plan_word(pl, w + 1);
+    const cpx<T>* __restrict__ tws = tw + plan_word(pl, w + 2);
+    const uint32_t nsm = (uint32_t)plan_word(pl, w + 3);
+    switch (plan_word(pl, w)) {
+      case 2: stockham_stage<T, 2, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 3: stockham_stage<T, 3, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 4: stockham_stage<T, 4, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 5: stockham_stage<T, 5, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 7: stockham_stage<T, 7, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 8: stockham_stage<T, 8, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 9: stockham_stage<T, 9, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 11: stockham_stage<T, 11, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 13: stockham_stage<T, 13, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 15: stockham_stage<T, 15, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 16: stockham_stage<T, 16, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 17: stockham_stage<T, 17, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 19: stockham_stage<T, 19, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 23: stockham_stage<T, 23, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 29: stockham_stage<T, 29, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 31: stockham_stage<T, 31, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
       default: break;  // the host planner only emits the radices above
     }
   }

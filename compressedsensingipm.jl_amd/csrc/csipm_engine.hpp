@@ -85,7 +85,7 @@ int chain_specs(const csipm_op* h, int which, PassSpec* s) {
 }
 
 // the batched kernel of one pass spec (the combinations the chains use)
-template <typename T, int NT>
+template <typename T, int NT, int E>
 int launch_spec(const PassSpec& s, int grid, size_t lds, hipStream_t st, const void* tabv,
                 BSeg seg) {
   const PassArgs<T>* tab = (const PassArgs<T>*)tabv;
@@ -97,46 +97,47 @@ int launch_spec(const PassSpec& s, int grid, size_t lds, hipStream_t st, const v
     return CSIPM_OK;                                                            \
   } while (0)
   if (s.kind == PK_LINES) {
-    if constexpr (NT == kNT || NT == kNTSmall) {
+    if constexpr (NT * E <= kTile) {
       if (s.D == 2 && s.src == SRC_U && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 2, SRC_U, DST_BUF, false>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 2, SRC_U, DST_BUF, false>));
       if (s.D == 2 && s.src == SRC_BUF && s.dst == DST_U && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 2, SRC_BUF, DST_U, true>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 2, SRC_BUF, DST_U, true>));
       if (s.D == 3 && s.src == SRC_U && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 3, SRC_U, DST_BUF, false>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_U, DST_BUF, false>));
       if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 3, SRC_BUF, DST_BUF, false>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_BUF, false>));
       if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_BUF && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 3, SRC_BUF, DST_BUF, true>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_BUF, true>));
       if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_U && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, kE, 3, SRC_BUF, DST_U, true>));
+        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_U, true>));
     }
-    return fail(CSIPM_ERR_UNSUPPORTED, "line pass with %d threads", NT);
   } else if (s.kind == PK_COL) {
-    if constexpr (NT != kNT) return fail(CSIPM_ERR_UNSUPPORTED, "column pass with %d threads", NT);
-    if (s.fm == C_FIRST) CSIPM_LAUNCH((kb_col<T, kNT, kE, SRC_U, DST_BUF, C_FIRST>));
-    if (s.fm == C_REAL_IN) CSIPM_LAUNCH((kb_col<T, kNT, kE, SRC_REAL, DST_BUF, C_REAL_IN>));
-    if (s.fm == C_MID) CSIPM_LAUNCH((kb_col<T, kNT, kE, SRC_BUF, DST_BUF, C_MID>));
-    if (s.fm == C_LAST) CSIPM_LAUNCH((kb_col<T, kNT, kE, SRC_BUF, DST_U, C_LAST>));
+    if constexpr (NT * E <= kTile) {
+    if (s.fm == C_FIRST) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_U, DST_BUF, C_FIRST>));
+    if (s.fm == C_REAL_IN) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_REAL, DST_BUF, C_REAL_IN>));
+    if (s.fm == C_MID) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_BUF, DST_BUF, C_MID>));
+    if (s.fm == C_LAST) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_BUF, DST_U, C_LAST>));
+    }
   } else if (s.kind == PK_ROW) {
-    if constexpr (NT != kNT) return fail(CSIPM_ERR_UNSUPPORTED, "row pass with %d threads", NT);
-    if (s.fm == R_MTM) CSIPM_LAUNCH((kb_row<T, kNT, kE, R_MTM>));
-    if (s.fm == R_R2C) CSIPM_LAUNCH((kb_row<T, kNT, kE, R_R2C>));
-    if (s.fm == R_CONV_INV) CSIPM_LAUNCH((kb_row<T, kNT, kE, R_CONV_INV>));
-    if (s.fm == R_CONV_FWD) CSIPM_LAUNCH((kb_row<T, kNT, kE, R_CONV_FWD>));
+    if constexpr (NT * E <= kTile) {
+    if (s.fm == R_MTM) CSIPM_LAUNCH((kb_row<T, NT, E, R_MTM>));
+    if (s.fm == R_R2C) CSIPM_LAUNCH((kb_row<T, NT, E, R_R2C>));
+    if (s.fm == R_CONV_INV) CSIPM_LAUNCH((kb_row<T, NT, E, R_CONV_INV>));
+    if (s.fm == R_CONV_FWD) CSIPM_LAUNCH((kb_row<T, NT, E, R_CONV_FWD>));
+    }
   } else {
     if (s.D == 1 && s.src == SRC_U && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 1, SRC_U, DST_U, MODE_MTM>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 1, SRC_U, DST_U, MODE_MTM>));
     if (s.D == 1 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 1, SRC_REAL, DST_U, MODE_R2C>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 1, SRC_REAL, DST_U, MODE_R2C>));
     if (s.D == 2 && s.src == SRC_BUF && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 2, SRC_BUF, DST_BUF, MODE_MTM>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 2, SRC_BUF, DST_BUF, MODE_MTM>));
     if (s.D == 2 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 2, SRC_REAL, DST_BUF, MODE_R2C>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 2, SRC_REAL, DST_BUF, MODE_R2C>));
     if (s.D == 3 && s.src == SRC_BUF && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 3, SRC_BUF, DST_BUF, MODE_MTM>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 3, SRC_BUF, DST_BUF, MODE_MTM>));
     if (s.D == 3 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, kE, 3, SRC_REAL, DST_BUF, MODE_R2C>));
+      CSIPM_LAUNCH((kb_dim1<T, NT, E, 3, SRC_REAL, DST_BUF, MODE_R2C>));
   }
 #undef CSIPM_LAUNCH
   return fail(CSIPM_ERR_UNSUPPORTED, "no batched kernel for pass (%d,%d,%d,%d,%d)", s.kind, s.D,
@@ -241,9 +242,12 @@ struct VsegOff {
 template <typename T>
 int launch_sub(const ChainSub& s, hipStream_t st) {
   BSeg seg{s.seg, s.seg + s.grid};
-  if (s.nt == kNT) return launch_spec<T, kNT>(s.spec, s.grid, s.lds, st, s.tab, seg);
-  if (s.nt == kNTSmall) return launch_spec<T, kNTSmall>(s.spec, s.grid, s.lds, st, s.tab, seg);
-  return launch_spec<T, kNTBig>(s.spec, s.grid, s.lds, st, s.tab, seg);
+  switch (s.nt) {
+    case 256: return launch_spec<T, 256, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
+    case 512: return launch_spec<T, 512, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
+    case 1024: return launch_spec<T, 1024, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
+    default: return launch_spec<T, 1024, 16>(s.spec, s.grid, s.lds, st, s.tab, seg);
+  }
 }
 
 template <typename T>
@@ -524,7 +528,6 @@ BatchCfg batch_cfg(csipm_op* h, int members) {
   if (h->big) {
     b.col = col_cfg(h->bA, h->bB, cs, target);
     b.row = row_cfg(h->bA, h->bB, cs, target);
-    b.d1.nt = kNT;
     return b;
   }
   const TuneVal t0 = tune_lookup(1, cs, h->plan[0].L, h->rows[0]);
@@ -535,20 +538,6 @@ BatchCfg batch_cfg(csipm_op* h, int members) {
     b.lines[a] = line_cfg(h->H1, h->plan[a].L, h->rows[a], h->n[a == 1 ? 2 : 1], cs, target,
                           ta[a].lg_cap);
   }
-  // a tile of at most kNTSmall*kE elements runs on kNTSmall threads: a stage
-  // of radix R has L*lines/R butterflies, and on 256 threads a 255-point
-  // tile of 8 lines (120 radix-17 butterflies) would leave half the lanes
-  // idle (a tuned choice replaces the rule where the tile fits it)
-  auto small = [](int64_t elems) { return elems <= (int64_t)kNTSmall * kE; };
-  auto pick = [&](int nt_rule, int64_t elems, const TuneVal& t) {
-    if (nt_rule == kNTBig) return nt_rule;
-    if (t.nt == kNTSmall && small(elems)) return kNTSmall;
-    if (t.nt == kNT) return kNT;
-    return small(elems) ? kNTSmall : kNT;
-  };
-  b.d1.nt = pick(b.d1.nt, (int64_t)h->plan[0].L << b.d1.lg, t0);
-  for (int a = 1; a < h->dim; ++a)
-    b.lines[a].nt = pick(kNT, (int64_t)h->plan[a].L << b.lines[a].lg, ta[a]);
   return b;
 }
 
@@ -618,7 +607,7 @@ int chain_call_args(Engine* E, int id, int call, int nb, const PassSpec& s,
 inline int pass_nt(const PassSpec& s, const BatchCfg& bc) {
   if (s.kind == PK_DIM1) return bc.d1.nt;
   if (s.kind == PK_LINES) return bc.lines[s.axis].nt;
-  return kNT;
+  return s.kind == PK_COL ? bc.col.nt : bc.row.nt;
 }
 
 template <typename T>
@@ -636,7 +625,7 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
                                specs);
     for (int p = 0; p < np; ++p) {
       const PassSpec& s = specs[p];
-      for (int nt : {kNTSmall, kNT, kNTBig}) {
+      for (int nt : {256, 512, 1024, kNTLong}) {
         std::vector<PassArgs<T>> tab;
         std::vector<int> grids;
         size_t lds = 0;
@@ -1282,11 +1271,7 @@ int engine_apply_timed(Engine* E, int64_t nrep, double* ms, double* bytes, std::
     HIPCHK(hipEventRecord(ev[0], E->stream));
     for (int k = 0; k < ns; ++k) {
       const ChainSub& sb = c.subs[(size_t)k];
-      BSeg seg{sb.seg, sb.seg + sb.grid};
-      if (sb.nt == kNT) CHK((launch_spec<TC, kNT>(sb.spec, sb.grid, sb.lds, E->stream, sb.tab, seg)));
-      else if (sb.nt == kNTSmall)
-        CHK((launch_spec<TC, kNTSmall>(sb.spec, sb.grid, sb.lds, E->stream, sb.tab, seg)));
-      else CHK((launch_spec<TC, kNTBig>(sb.spec, sb.grid, sb.lds, E->stream, sb.tab, seg)));
+      CHK(launch_sub<TC>(sb, E->stream));
       HIPCHK(hipEventRecord(ev[(size_t)k + 1], E->stream));
     }
     HIPCHK(hipEventSynchronize(ev[(size_t)ns]));

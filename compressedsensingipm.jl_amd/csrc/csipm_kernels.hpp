@@ -328,12 +328,16 @@ constexpr int stage_k() {
   return sizeof(T) == 4 ? 8 : 4;
 }
 
+// The members of a group past the end are skipped by a uniform branch: a small
+// tile otherwise spent most of its instructions on clamped repeats.
 template <int NT, int K, typename R, typename F, typename P>
 __device__ __forceinline__ void staged(int total, F&& fetch, P&& put) {
-  for (int i0 = threadIdx.x; i0 < total; i0 += K * NT) {
+  for (int g0 = 0; g0 < total; g0 += K * NT) {
+    const int i0 = g0 + (int)threadIdx.x;
     R r[K];
 #pragma unroll
-    for (int j = 0; j < K; ++j) r[j] = fetch(min(i0 + j * NT, total - 1));
+    for (int j = 0; j < K; ++j)
+      if (g0 + j * NT < total) r[j] = fetch(min(i0 + j * NT, total - 1));
 #pragma unroll
     for (int j = 0; j < K; ++j)
       if (i0 + j * NT < total) put(i0 + j * NT, r[j]);
@@ -377,8 +381,8 @@ enum { MODE_MTM = 0, MODE_C2R = 1, MODE_R2C = 2 };
 template <typename T>
 struct PassArgs {
   MapGeom g;
-  const FftPlan* plan;  // device-resident (read with uniform loads)
-  const cpx<T>* tw;
+  const FftPlan* plan;  // device-resident
+  const cpx<T>* tw;     // the plan's twiddles, stage by stage
   int axis;      // k_lines: 1 or 2
   int H1;
   int lg;        // log2 of lines (pairs) per workgroup
@@ -405,122 +409,110 @@ struct PassArgs {
   const cpx<T>* chirp;  // w_n = exp(-i pi n^2 / len), n < len
   const cpx<T>* bfw;    // FFT_M(b) / M of the forward kernel b = conj(w) (wrapped);
                         // Rader: FFT_{L-1}(b) / (L-1) of b_j = exp(-2 pi i g^-j / L)
-  const cpx<T>* binv;   // the same for the inverse kernel b = w (Rader: conj b)
   const int* rperm;     // Rader: [e] row of element e in the convolution order
                         // (e = 0: row L), [L + m] element g^-m mod L of output m
   // long 1D lines (four-step): the length-F transform (F = len, or the
   // Bluestein length when obs) as A columns x B rows, position col + A*row
   int A, B, F;
-  int obs;              // outer Bluestein: chirp / bfw / binv are of length len / F / F
+  int obs;              // outer Bluestein: chirp / bfw are of length len / F
   uint32_t am;          // ceil(2^32 / A)
   const cpx<T>* twF;    // exp(-2 pi i j / F), j < F
 };
 
-// DFT of length a.len of the 2^lg lines in LDS ([element][line], stride ps),
-// in place.  Direct: the Stockham plan.  Bluestein (lengths with a prime
-// factor above 17): X_k = w_k sum_n (x_n w_n) conj(w_{k-n}) (forward; the
-// inverse conjugates w), the convolution by FFT_M, pointwise product with the
-// precomputed kernel spectrum, inverse FFT_M.  LDS must hold M rows.
+// Forward DFT of length a.len of the 2^lg lines in LDS ([element][line],
+// stride ps), in place.  Direct: the Stockham plan.  Bluestein (lengths with a
+// prime factor above 31): X_k = w_k sum_n (x_n w_n) conj(w_{k-n}), the
+// convolution by FFT_M, pointwise product with the precomputed kernel
+// spectrum, inverse FFT_M.  LDS must hold M rows.
 // Rader (prime L = p, bs = 2), with g a primitive root mod p:
 //   X_0 = x_0 + sum_{n>0} x_n,   X_{g^-m} = x_0 + sum_q x_{g^q} w^{g^(q-m)}
-// (w = exp(-+2 pi i / p)), a cyclic convolution of length p - 1 of
+// (w = exp(-2 pi i / p)), a cyclic convolution of length p - 1 of
 // a_q = x_{g^q} with b_j = w^{g^-j}, done by FFT_{p-1}, the pointwise product
 // with the precomputed FFT_{p-1}(b) / (p - 1) and the inverse FFT_{p-1}.
 // LDS rows of a tile: 0..p-1 the line in natural order, p..2p-2 the
 // convolution (row p + q), 2p-1 x_0 and 2p X_0 (= x_0 + A_0, the DC term of
 // FFT_{p-1}(a)).  The two permutations move between disjoint rows, one
 // element at a time.
-template <typename T, int E, int NT, bool FWD>
-__device__ __forceinline__ void rader_dft(cpx<T>* lds, const PassArgs<T>& a, int lg, int ps) {
-  const int L = a.len, Lm = L - 1, nl = 1 << lg;
-  const int* __restrict__ perm = a.rperm;
-  cpx<T>* conv = lds + L * ps;
-  cpx<T>* x0row = lds + (2 * L - 1) * ps;
-  cpx<T>* X0row = lds + 2 * L * ps;
+//
+// One copy of the FFT per kernel: the inverse transforms (of a pass, and of
+// the convolutions) run the forward code on values with real and imaginary
+// part exchanged, and both transforms of a convolution are turns of one loop.
+// With an inlined copy for every direction and form (ten in the dimension-1
+// pass) a launch ran each copy once, cold: the short launches of single
+// problems waited for instruction fetches as much as for data.
+template <typename T, int E, int NT>
+__device__ __forceinline__ void line_dft(cpx<T>* lds, const PassArgs<T>& a, int pl, int lg,
+                                         int ps) {
+  const int L = a.len, M = plan_word(pl, 0), nl = 1 << lg;
+  constexpr int K = stage_k<T>();
+  cpx<T>* conv = lds;
   // the table loads of each phase are issued in groups (staged) so that a
   // thread has several in flight instead of waiting for each before its move
-  staged<NT, 8, int>(
-      L << lg, [&](int idx) { return perm[idx >> lg]; },   // e = 0: q = p - 1, the x_0 row
-      [&](int idx, int q) {
-        const int line = idx & (nl - 1), e = idx >> lg;
-        conv[q * ps + line] = lds[e * ps + line];
-      });
-  __syncthreads();
-  lds_fft<T, E, NT, true>(conv, *a.plan, lg, ps, a.tw);
-  const cpx<T>* __restrict__ B = FWD ? a.bfw : a.binv;
-  staged<NT, stage_k<T>(), cpx<T>>(
-      Lm << lg, [&](int idx) { return B[idx >> lg]; },
-      [&](int idx, const cpx<T>& bk) {
-        const int line = idx & (nl - 1), e = idx >> lg;
-        cpx<T>* q = conv + e * ps + line;
-        const cpx<T> v = *q;
-        if (e == 0) X0row[line] = cadd(x0row[line], v);
-        *q = cmul(v, bk);
-      });
-  __syncthreads();
-  lds_fft<T, E, NT, false>(conv, *a.plan, lg, ps, a.tw);
-  // X_{g^-m} = x_0 + c_m into row g^-m (1..p-1); the last index: X_0 into row 0
-  staged<NT, 8, int>(
-      L << lg, [&](int idx) { return perm[L + min(idx >> lg, Lm - 1)]; },
-      [&](int idx, int row) {
-        const int line = idx & (nl - 1), m = idx >> lg;
-        if (m < Lm)
-          lds[row * ps + line] = cadd(conv[m * ps + line], x0row[line]);
-        else
-          lds[line] = X0row[line];
-      });
-  __syncthreads();
-}
-
-template <typename T, int E, int NT, bool FWD>
-__device__ __forceinline__ void line_dft(cpx<T>* lds, const PassArgs<T>& a, int lg, int ps) {
-  if (!a.bs) {
-    lds_fft<T, E, NT, FWD>(lds, *a.plan, lg, ps, a.tw);
-    return;
+  if (a.bs == 2) {
+    conv = lds + L * ps;
+    const int* __restrict__ perm = a.rperm;
+    staged<NT, 8, int>(
+        L << lg, [&](int idx) { return perm[idx >> lg]; },   // e = 0: q = p - 1, the x_0 row
+        [&](int idx, int q) {
+          const int line = idx & (nl - 1), e = idx >> lg;
+          conv[q * ps + line] = lds[e * ps + line];
+        });
+    __syncthreads();
+  } else if (a.bs == 1) {
+    staged<NT, K, cpx<T>>(
+        M << lg, [&](int idx) { return a.chirp[min(idx >> lg, L - 1)]; },
+        [&](int idx, const cpx<T>& w) {
+          const int line = idx & (nl - 1), e = idx >> lg;
+          cpx<T>* q = lds + e * ps + line;
+          *q = e < L ? cmul(*q, w) : cpx<T>{(T)0, (T)0};
+        });
+    __syncthreads();
+  }
+  cpx<T>* x0row = lds + (2 * L - 1) * ps;   // Rader
+  cpx<T>* X0row = lds + 2 * L * ps;
+  const int turns = a.bs ? 2 : 1;
+#pragma unroll 1
+  for (int t = 0; t < turns; ++t) {
+    lds_fft<T, E, NT>(conv, pl, lg, ps, a.tw);
+    if (t == 0 && a.bs) {
+      // the product with the kernel spectrum, exchanged for the inverse FFT
+      const cpx<T>* __restrict__ B = a.bfw;
+      const bool rader = a.bs == 2;
+      staged<NT, K, cpx<T>>(
+          M << lg, [&](int idx) { return B[idx >> lg]; },
+          [&](int idx, const cpx<T>& bk) {
+            const int line = idx & (nl - 1), e = idx >> lg;
+            cpx<T>* q = conv + e * ps + line;
+            const cpx<T> v = *q;
+            if (rader && e == 0) X0row[line] = cadd(x0row[line], v);
+            *q = cswap(cmul(v, bk));
+          });
+      __syncthreads();
+    }
   }
   if (a.bs == 2) {
-    rader_dft<T, E, NT, FWD>(lds, a, lg, ps);
-    return;
+    // X_{g^-m} = x_0 + c_m into row g^-m (1..p-1); the last index: X_0 into row 0
+    const int* __restrict__ perm = a.rperm;
+    staged<NT, 8, int>(
+        L << lg, [&](int idx) { return perm[L + min(idx >> lg, L - 2)]; },
+        [&](int idx, int row) {
+          const int line = idx & (nl - 1), m = idx >> lg;
+          if (m < L - 1)
+            lds[row * ps + line] = cadd(cswap(conv[m * ps + line]), x0row[line]);
+          else
+            lds[line] = X0row[line];
+        });
+    __syncthreads();
+  } else if (a.bs == 1) {
+    staged<NT, K, cpx<T>>(
+        L << lg, [&](int idx) { return a.chirp[idx >> lg]; },
+        [&](int idx, const cpx<T>& w) {
+          const int line = idx & (nl - 1), e = idx >> lg;
+          cpx<T>* q = lds + e * ps + line;
+          *q = cmul(cswap(*q), w);
+        });
+    __syncthreads();
   }
-  const int L = a.len, M = uniform(a.plan->L), nl = 1 << lg;
-  constexpr int K = stage_k<T>();
-  // chirp and kernel-spectrum loads issued in groups (staged), as in the
-  // tile loads
-  staged<NT, K, cpx<T>>(
-      M << lg, [&](int idx) { return a.chirp[min(idx >> lg, L - 1)]; },
-      [&](int idx, const cpx<T>& wc) {
-        const int line = idx & (nl - 1), e = idx >> lg;
-        cpx<T>* q = lds + e * ps + line;
-        if (e < L) {
-          cpx<T> w = wc;
-          if (!FWD) w.y = -w.y;
-          *q = cmul(*q, w);
-        } else {
-          *q = {(T)0, (T)0};
-        }
-      });
-  __syncthreads();
-  lds_fft<T, E, NT, true>(lds, *a.plan, lg, ps, a.tw);
-  const cpx<T>* B = FWD ? a.bfw : a.binv;
-  staged<NT, K, cpx<T>>(
-      M << lg, [&](int idx) { return B[idx >> lg]; },
-      [&](int idx, const cpx<T>& bk) {
-        const int line = idx & (nl - 1), e = idx >> lg;
-        cpx<T>* q = lds + e * ps + line;
-        *q = cmul(*q, bk);
-      });
-  __syncthreads();
-  lds_fft<T, E, NT, false>(lds, *a.plan, lg, ps, a.tw);
-  staged<NT, K, cpx<T>>(
-      L << lg, [&](int idx) { return a.chirp[idx >> lg]; },
-      [&](int idx, const cpx<T>& wc) {
-        const int line = idx & (nl - 1), e = idx >> lg;
-        cpx<T>* q = lds + e * ps + line;
-        cpx<T> w = wc;
-        if (!FWD) w.y = -w.y;
-        *q = cmul(*q, w);
-      });
-  __syncthreads();
 }
 
 __device__ __forceinline__ int udiv(int a, int d, uint32_t m) { return d == 1 ? a : fdiv(a, m); }
@@ -563,6 +555,13 @@ __device__ __forceinline__ cpx<T> raw_value(const Raw<T>& r) {
   return SRC == SRC_U ? u_map(r.w, r.mode) : r.w;
 }
 
+// a value on its way into or out of the LDS tile of a pass whose transform is
+// forward (FWD) or inverse (held exchanged, see line_dft)
+template <bool FWD, typename T>
+__device__ __forceinline__ cpx<T> tile_value(cpx<T> v) {
+  return FWD ? v : cswap(v);
+}
+
 // a spectrum value read from LDS with its epilogue operands
 template <typename T>
 struct Fetched {
@@ -573,10 +572,12 @@ struct Fetched {
 // one workgroup's tile of a line pass (tile = its index within the pass)
 template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
 __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
+  static_assert(FWD || DST == DST_BUF, "inverse line passes end in the scratch spectrum");
   extern __shared__ unsigned char smem_raw[];
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
   // finished instances: the flag is read beside the loads, not before them
   const int dflag = a.done ? *a.done : 0;
+  const int pl = plan_load(a.plan);
   const int L = a.len;
   const int lg = a.lg, nl = 1 << lg;
   const int tile1 = tile % a.ntile1;
@@ -601,7 +602,7 @@ __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
           r.w = a.u_in[base + (line < nv ? line : 0) + el * sl];
           return r;
         },
-        [&](int idx, const Raw<T>& r) { lds[idx] = raw_value<T, SRC>(r); });
+        [&](int idx, const Raw<T>& r) { lds[idx] = tile_value<FWD>(raw_value<T, SRC>(r)); });
   } else {
   staged<NT, K, Raw<T>>(
       total,
@@ -624,15 +625,15 @@ __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
         if (!ok) r.mode = -1;
         return r;
       },
-      [&](int idx, const Raw<T>& r) { lds[idx] = raw_value<T, SRC>(r); });
+      [&](int idx, const Raw<T>& r) { lds[idx] = tile_value<FWD>(raw_value<T, SRC>(r)); });
   }
   if (dflag) return;
   __syncthreads();
-  line_dft<T, E, NT, FWD>(lds, a, lg, nl);
+  line_dft<T, E, NT>(lds, a, pl, lg, nl);
   double acc = 0.0;
   if (DST == DST_BUF) {
     staged<NT, K, cpx<T>>(
-        total, [&](int idx) { return lds[idx]; },
+        total, [&](int idx) { return tile_value<FWD>(lds[idx]); },
         [&](int idx, const cpx<T>& v) {
           const int line = idx & (nl - 1), el = idx >> lg;
           if (line < nv) a.buf[base + line + el * sl] = v;
@@ -688,7 +689,7 @@ __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
 }
 
 template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
-__global__ __launch_bounds__(NT) void k_lines(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_lines(PassArgs<T> a) {
   lines_body<T, NT, E, D, SRC, DST, FWD>(a, xcd_block());
 }
 
@@ -699,7 +700,7 @@ struct BSeg {
 };
 
 template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
-__global__ __launch_bounds__(NT) void kb_lines(const PassArgs<T>* __restrict__ tab, BSeg seg) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_lines(const PassArgs<T>* __restrict__ tab, BSeg seg) {
   const int b = xcd_block();
   const int i = uniform(seg.inst[b]);
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
@@ -734,22 +735,27 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
   extern __shared__ unsigned char smem_raw[];
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
   const int dflag = a.done ? *a.done : 0;   // read beside the loads
+  const int pl = plan_load(a.plan);
   const int N1 = a.len, H1 = a.H1;
   const int lg = a.lg, np = 1 << lg, ps = a.ps;
   const int p0 = tile << lg;
   const bool even = (N1 & 1) == 0;
   constexpr int K = stage_k<T>();
   const int nl1 = a.nlines - 1;
+  [[maybe_unused]] int W = 0;            // MODE_MTM, MODE_C2R: the staged mask
+  [[maybe_unused]] bool stage_mask = false;
+  [[maybe_unused]] uint32_t* mw = nullptr;
   if constexpr (MODE != MODE_R2C) {
     // the mask words of the tile's lines are loaded with the tile (into LDS)
     // rather than per element between the transforms: a line's N1 samples
     // span at most W words
     constexpr int kMaskWords = 640;
     constexpr int kMR = (kMaskWords + NT - 1) / NT;
-    __shared__ uint32_t mw[kMR * NT];
-    const int W = (N1 + 31) / 32 + 1;
+    __shared__ uint32_t mw_smem[kMR * NT];
+    mw = mw_smem;
+    W = (N1 + 31) / 32 + 1;
     const int nlt = 2 * np;
-    const bool stage_mask = a.miss && nlt * W <= kMaskWords;
+    stage_mask = a.miss && nlt * W <= kMaskWords;
     uint32_t mreg[kMR];
     if (stage_mask) {
       const int64_t nwords = ((int64_t)a.nlines * N1 + 31) >> 5;
@@ -795,16 +801,42 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
             A.y = 0;
             B.y = 0;
           }
-          lds[k * ps + p] = {A.x - B.y, A.y + B.x};
-          if (k > 0 && N1 - k != k) lds[(N1 - k) * ps + p] = {A.x + B.y, B.x - A.y};
+          // A + i B and its Hermitian partner, exchanged: the transform is inverse
+          lds[k * ps + p] = {A.y + B.x, A.x - B.y};
+          if (k > 0 && N1 - k != k) lds[(N1 - k) * ps + p] = {B.x - A.y, A.x + B.y};
         });
     if (stage_mask) {
 #pragma unroll
       for (int r = 0; r < kMR; ++r) mw[threadIdx.x + r * NT] = mreg[r];
     }
-    if (dflag) return;
-    __syncthreads();
-    line_dft<T, E, NT, false>(lds, a, lg, ps);
+  } else {
+    const int totr = N1 << lg;
+    staged<NT, K, cpx<T>>(
+        totr,
+        [&](int idx) {
+          const int p = udiv(idx, N1, a.n1m);
+          const int n = idx - p * N1;
+          const int la = 2 * (p0 + p);
+          return cpx<T>{a.real_in[(int64_t)min(la, nl1) * N1 + n],
+                        a.real_in[(int64_t)min(la + 1, nl1) * N1 + n]};
+        },
+        [&](int idx, const cpx<T>& r) {
+          const int p = udiv(idx, N1, a.n1m);
+          const int n = idx - p * N1;
+          const int la = 2 * (p0 + p), lb = la + 1;
+          const T xa = la < a.nlines ? r.x * a.scale : (T)0;
+          const T xb = lb < a.nlines ? r.y * a.scale : (T)0;
+          lds[n * ps + p] = {xa, xb};
+        });
+  }
+  if (dflag) return;
+  __syncthreads();
+  // the inverse (M^T M, C2R) and the forward transform (M^T M, R2C) are turns
+  // of one loop around one copy of the FFT
+#pragma unroll 1
+  for (int turn = 0;; ++turn) {
+    line_dft<T, E, NT>(lds, a, pl, lg, ps);
+    if (MODE == MODE_R2C || turn == 1) break;
     const int totr = N1 << lg;
     if (MODE == MODE_MTM && (stage_mask || !a.miss) && np <= NT) {
       // the mask in place from LDS: a thread keeps one line pair p (NT is a
@@ -827,10 +859,8 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
           if ((ra[ta >> 5] >> (ta & 31)) & 1u) sa = (T)0;
           if ((rb[tb >> 5] >> (tb & 31)) & 1u) sb = (T)0;
         }
-        cpx<T> z = *q;
-        z.x *= sa;
-        z.y *= sb;
-        *q = z;
+        const cpx<T> z = *q;   // (line b, line a): exchanged
+        *q = {z.y * sa, z.x * sb};
       }
     } else {
     staged<NT, K, Masked<T>>(
@@ -840,7 +870,7 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
           const int n = idx >> lg;
           const int la = 2 * (p0 + p);
           Masked<T> r;
-          r.z = lds[n * ps + p];
+          r.z = cswap(lds[n * ps + p]);
           r.wa = r.wb = 0u;
           if (stage_mask) {
             const int64_t sa = (int64_t)la * N1 + n, sb = sa + N1;
@@ -874,29 +904,7 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
     }
     if (MODE == MODE_C2R) return;
     __syncthreads();
-  } else {
-    const int totr = N1 << lg;
-    staged<NT, K, cpx<T>>(
-        totr,
-        [&](int idx) {
-          const int p = udiv(idx, N1, a.n1m);
-          const int n = idx - p * N1;
-          const int la = 2 * (p0 + p);
-          return cpx<T>{a.real_in[(int64_t)min(la, nl1) * N1 + n],
-                        a.real_in[(int64_t)min(la + 1, nl1) * N1 + n]};
-        },
-        [&](int idx, const cpx<T>& r) {
-          const int p = udiv(idx, N1, a.n1m);
-          const int n = idx - p * N1;
-          const int la = 2 * (p0 + p), lb = la + 1;
-          const T xa = la < a.nlines ? r.x * a.scale : (T)0;
-          const T xb = lb < a.nlines ? r.y * a.scale : (T)0;
-          lds[n * ps + p] = {xa, xb};
-        });
-    if (dflag) return;
-    __syncthreads();
   }
-  line_dft<T, E, NT, true>(lds, a, lg, ps);
   double acc = 0.0;
   const int tot = H1 << lg;
   const T half = (T)0.5;
@@ -958,12 +966,12 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
 }
 
 template <typename T, int NT, int E, int D, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT) void k_dim1(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_dim1(PassArgs<T> a) {
   dim1_body<T, NT, E, D, SRC, DST, MODE>(a, xcd_block());
 }
 
 template <typename T, int NT, int E, int D, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT) void kb_dim1(const PassArgs<T>* __restrict__ tab, BSeg seg) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_dim1(const PassArgs<T>* __restrict__ tab, BSeg seg) {
   const int b = xcd_block();
   const int i = uniform(seg.inst[b]);
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
@@ -980,7 +988,7 @@ __global__ __launch_bounds__(NT) void kb_dim1(const PassArgs<T>* __restrict__ ta
 //         index t = row + B*col, forward, twiddle)  col LAST (forward, epilogue)
 // Bluestein (F = M >= 2N - 1, chirp w_n = exp(-i pi n^2/N)):
 //   MTM   col FIRST (x conj(w), forward, twiddle)  row CONV_INV (forward,
-//         x FFT_M(w)/M, inverse, twiddle)  col MID (inverse, x conj(w), mask,
+//         x FFT_M(w)/M = conj(bfw), inverse, twiddle)  col MID (inverse, x conj(w), mask,
 //         x w, forward, twiddle)  row CONV_FWD  col LAST (inverse, x w, epilogue)
 // ===========================================================================
 enum { C_FIRST = 0, C_REAL_IN = 1, C_MID = 2, C_LAST = 3, C_MID_C2R = 4 };
@@ -1013,9 +1021,13 @@ __device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
   extern __shared__ unsigned char smem_raw[];
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
   if (a.done && *a.done) return;
+  const int pl = plan_load(a.plan);
   const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg;
   const int64_t N = a.len;
   const bool bs = a.obs != 0;
+  // the first transform is forward or inverse (then the tile holds exchanged
+  // values, see line_dft)
+  const bool fwd1 = MODE == C_FIRST ? bs : (MODE == C_REAL_IN ? true : (MODE == C_LAST ? !bs : false));
   const int c0 = tile << lg;
   const int nv = min(nl, A - c0);
   for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
@@ -1037,20 +1049,20 @@ __device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
         v = a.buf[n];
       }
     }
-    lds[r * nl + line] = v;
+    lds[r * nl + line] = fwd1 ? v : cswap(v);
   }
   __syncthreads();
-  const bool fwd1 = MODE == C_FIRST ? bs : (MODE == C_REAL_IN ? true : (MODE == C_LAST ? !bs : false));
-  if (fwd1) lds_fft<T, E, NT, true>(lds, *a.plan, lg, nl, a.tw);
-  else lds_fft<T, E, NT, false>(lds, *a.plan, lg, nl, a.tw);
-  if (MODE == C_MID || MODE == C_MID_C2R) {
+#pragma unroll 1
+  for (int turn = 0;; ++turn) {
+    lds_fft<T, E, NT>(lds, pl, lg, nl, a.tw);
+    if ((MODE != C_MID && MODE != C_MID_C2R) || turn == 1) break;
     // conv -> x_n = conj(w_n) conv_n, masked real part; then (MTM) x w for the forward
     for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
       const int line = idx & (nl - 1), r = idx >> lg;
       const int64_t n = c0 + line + (int64_t)A * r;
       cpx<T>* q = lds + r * nl + line;
       T xr = (T)0;
-      if (line < nv && n < N && !miss_bit(a.miss, n)) xr = cmul(*q, chirp_at(a, n, true)).x * a.scale;
+      if (line < nv && n < N && !miss_bit(a.miss, n)) xr = cmul(cswap(*q), chirp_at(a, n, true)).x * a.scale;
       if (MODE == C_MID_C2R) {
         if (line < nv && n < N) a.real_out[n] = xr;
       } else {
@@ -1060,14 +1072,15 @@ __device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
     }
     if (MODE == C_MID_C2R) return;
     __syncthreads();
-    lds_fft<T, E, NT, true>(lds, *a.plan, lg, nl, a.tw);
   }
+  const bool exchanged = MODE != C_MID && !fwd1;   // the last transform was inverse
   double acc = 0.0;
   for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
     const int line = idx & (nl - 1), r = idx >> lg;
     if (line >= nv) continue;
     const int col = c0 + line;
     cpx<T> v = lds[r * nl + line];
+    if (exchanged) v = cswap(v);
     if (MODE != C_LAST) {
       const bool inv = MODE == C_FIRST && !bs;
       v = cmul(v, twf(a, (int64_t)col * r, inv));
@@ -1088,6 +1101,8 @@ __device__ __forceinline__ void row_body(const PassArgs<T>& a, int tile) {
   extern __shared__ unsigned char smem_raw[];
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
   if (a.done && *a.done) return;
+  const int pl = plan_load(a.plan);
+  constexpr bool fwd1 = MODE == R_R2C || MODE == R_CONV_INV || MODE == R_CONV_FWD;
   const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg, ps = a.ps;
   const int r0 = tile << lg;
   const int nv = min(nl, B - r0);
@@ -1101,66 +1116,73 @@ __device__ __forceinline__ void row_body(const PassArgs<T>& a, int tile) {
       if (MODE == R_R2C) v = {a.real_in[row + (int64_t)B * c] * a.scale, (T)0};
       else v = a.buf[c + (int64_t)A * row];
     }
-    lds[c * ps + line] = v;
+    lds[c * ps + line] = fwd1 ? v : cswap(v);
   }
   __syncthreads();
-  const bool fwd1 = MODE == R_R2C || MODE == R_CONV_INV || MODE == R_CONV_FWD;
-  if (fwd1) lds_fft<T, E, NT, true>(lds, *a.plan, lg, ps, a.tw);
-  else lds_fft<T, E, NT, false>(lds, *a.plan, lg, ps, a.tw);
-  if (MODE == R_MTM || MODE == R_C2R) {
-    for (int idx = threadIdx.x; idx < tot; idx += NT) {
-      const int line = udiv(idx, A, a.am);
-      const int c = idx - line * A;
-      const int64_t t = r0 + line + (int64_t)B * c;
-      cpx<T>* q = lds + c * ps + line;
-      const T xr = (line < nv && !miss_bit(a.miss, t)) ? q->x * a.scale : (T)0;
-      if (MODE == R_C2R) {
-        if (line < nv) a.real_out[t] = xr;
-      } else {
-        *q = {xr, (T)0};
+#pragma unroll 1
+  for (int turn = 0;; ++turn) {
+    lds_fft<T, E, NT>(lds, pl, lg, ps, a.tw);
+    if (MODE == R_R2C || turn == 1) break;
+    if (MODE == R_MTM || MODE == R_C2R) {
+      for (int idx = threadIdx.x; idx < tot; idx += NT) {
+        const int line = udiv(idx, A, a.am);
+        const int c = idx - line * A;
+        const int64_t t = r0 + line + (int64_t)B * c;
+        cpx<T>* q = lds + c * ps + line;
+        const T xr = (line < nv && !miss_bit(a.miss, t)) ? q->y * a.scale : (T)0;   // exchanged
+        if (MODE == R_C2R) {
+          if (line < nv) a.real_out[t] = xr;
+        } else {
+          *q = {xr, (T)0};
+        }
+      }
+      if (MODE == R_C2R) return;
+    } else {
+      for (int idx = threadIdx.x; idx < tot; idx += NT) {
+        const int line = udiv(idx, A, a.am);
+        const int c = idx - line * A;
+        cpx<T>* q = lds + c * ps + line;
+        // the product with the kernel spectrum, exchanged for the inverse FFT
+        // (the inverse kernel is the conjugate of the forward one, and both
+        // are even, so its spectrum is the conjugate too)
+        if (line < nv) {
+          cpx<T> bk = a.bfw[r0 + line + (int64_t)B * c];
+          if (MODE == R_CONV_INV) bk.y = -bk.y;
+          *q = cswap(cmul(*q, bk));
+        }
       }
     }
-    if (MODE == R_C2R) return;
     __syncthreads();
-    lds_fft<T, E, NT, true>(lds, *a.plan, lg, ps, a.tw);
-  } else if (MODE == R_CONV_INV || MODE == R_CONV_FWD) {
-    const cpx<T>* Bh = MODE == R_CONV_FWD ? a.bfw : a.binv;
-    for (int idx = threadIdx.x; idx < tot; idx += NT) {
-      const int line = udiv(idx, A, a.am);
-      const int c = idx - line * A;
-      cpx<T>* q = lds + c * ps + line;
-      if (line < nv) *q = cmul(*q, Bh[r0 + line + (int64_t)B * c]);
-    }
-    __syncthreads();
-    lds_fft<T, E, NT, false>(lds, *a.plan, lg, ps, a.tw);
   }
-  const bool inv_tw = MODE == R_CONV_INV || MODE == R_CONV_FWD;
+  constexpr bool inv_tw = MODE == R_CONV_INV || MODE == R_CONV_FWD;
   for (int idx = threadIdx.x; idx < tot; idx += NT) {
     const int line = udiv(idx, A, a.am);
     const int c = idx - line * A;
     if (line >= nv) continue;
     const int row = r0 + line;
-    a.buf[c + (int64_t)A * row] = cmul(lds[c * ps + line], twf(a, (int64_t)row * c, inv_tw));
+    // (the second transform of a convolution is inverse)
+    const cpx<T> v = inv_tw ? cswap(lds[c * ps + line]) : lds[c * ps + line];
+    a.buf[c + (int64_t)A * row] = cmul(v, twf(a, (int64_t)row * c, inv_tw));
   }
 }
 
 template <typename T, int NT, int E, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT) void k_col(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_col(PassArgs<T> a) {
   col_body<T, NT, E, SRC, DST, MODE>(a, xcd_block());
 }
 template <typename T, int NT, int E, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT) void kb_col(const PassArgs<T>* __restrict__ tab, BSeg seg) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_col(const PassArgs<T>* __restrict__ tab, BSeg seg) {
   const int b = xcd_block();
   const int i = uniform(seg.inst[b]);
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
   col_body<T, NT, E, SRC, DST, MODE>(a, b - uniform(seg.first[i]));
 }
 template <typename T, int NT, int E, int MODE>
-__global__ __launch_bounds__(NT) void k_row(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_row(PassArgs<T> a) {
   row_body<T, NT, E, MODE>(a, xcd_block());
 }
 template <typename T, int NT, int E, int MODE>
-__global__ __launch_bounds__(NT) void kb_row(const PassArgs<T>* __restrict__ tab, BSeg seg) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_row(const PassArgs<T>* __restrict__ tab, BSeg seg) {
   const int b = xcd_block();
   const int i = uniform(seg.inst[b]);
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers

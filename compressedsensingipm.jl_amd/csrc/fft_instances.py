@@ -19,30 +19,32 @@ from __future__ import annotations
 import os
 
 # kernel -> template arguments after the precision
+_LINES = ["2 0 3 true", "2 3 0 false", "3 0 0 false", "3 0 0 true", "3 0 3 true", "3 3 0 false"]
+_LINES_BETA = ["2 0 1 true", "2 1 0 false", "3 0 1 true", "3 1 0 false"]
+_COL = ["0 0 2", "0 3 3", "2 0 1", "3 0 0"]
+_COL_BETA = ["0 1 3", "0 2 4", "1 0 0"]
+_ROW = ["0", "2", "3", "4"]
+_DIM1 = ["1 2 3 2", "1 3 3 0", "2 0 0 0", "2 2 0 2", "3 0 0 0", "3 2 0 2"]
+_DIM1_BETA = ["1 1 1 0", "1 1 2 1", "1 2 1 2", "2 0 2 1", "3 0 2 1"]
+# workgroup sizes with the elements per thread: of tiles up to 4096 elements,
+# and of the dimension-1 passes with longer lines
+_NT = ["256 8", "512 8"]
+_NT_DIM1 = _NT + ["1024 8", "1024 16"]
+
+
+def _rows(nts, rows):
+    return [f"{nt} {r}" for nt in nts for r in rows]
+
+
 TABLE = {
-    "k_col": ["256 16 0 0 2", "256 16 0 1 3", "256 16 0 2 4", "256 16 0 3 3", "256 16 1 0 0",
-              "256 16 2 0 1", "256 16 3 0 0"],
-    "k_dim1": ["1024 16 1 1 1 0", "1024 16 1 1 2 1", "1024 16 1 2 1 2", "1024 16 1 3 3 0",
-               "1024 16 2 0 0 0", "1024 16 2 0 2 1", "1024 16 2 2 0 2", "1024 16 3 0 0 0",
-               "1024 16 3 0 2 1", "1024 16 3 2 0 2", "256 16 1 1 1 0", "256 16 1 1 2 1",
-               "256 16 1 2 1 2", "256 16 1 3 3 0", "256 16 2 0 0 0", "256 16 2 0 2 1",
-               "256 16 2 2 0 2", "256 16 3 0 0 0", "256 16 3 0 2 1", "256 16 3 2 0 2"],
-    "k_lines": ["256 16 2 0 1 true", "256 16 2 0 3 true", "256 16 2 1 0 false",
-                "256 16 2 3 0 false", "256 16 3 0 0 false", "256 16 3 0 0 true",
-                "256 16 3 0 1 true", "256 16 3 0 3 true", "256 16 3 1 0 false",
-                "256 16 3 3 0 false"],
-    "k_row": ["256 16 0", "256 16 1", "256 16 2", "256 16 3", "256 16 4"],
-    "kb_col": ["256 16 0 0 2", "256 16 0 3 3", "256 16 2 0 1", "256 16 3 0 0"],
-    "kb_dim1": ["1024 16 1 2 3 2", "1024 16 1 3 3 0", "1024 16 2 0 0 0", "1024 16 2 2 0 2",
-                "1024 16 3 0 0 0", "1024 16 3 2 0 2", "256 16 1 2 3 2", "256 16 1 3 3 0",
-                "256 16 2 0 0 0", "256 16 2 2 0 2", "256 16 3 0 0 0", "256 16 3 2 0 2",
-                "128 16 1 2 3 2", "128 16 1 3 3 0", "128 16 2 0 0 0", "128 16 2 2 0 2",
-                "128 16 3 0 0 0", "128 16 3 2 0 2"],
-    "kb_lines": ["256 16 2 0 3 true", "256 16 2 3 0 false", "256 16 3 0 0 false",
-                 "256 16 3 0 0 true", "256 16 3 0 3 true", "256 16 3 3 0 false",
-                 "128 16 2 0 3 true", "128 16 2 3 0 false", "128 16 3 0 0 false",
-                 "128 16 3 0 0 true", "128 16 3 0 3 true", "128 16 3 3 0 false"],
-    "kb_row": ["256 16 0", "256 16 2", "256 16 3", "256 16 4"],
+    "k_col": _rows(_NT, _COL + _COL_BETA),
+    "k_row": _rows(_NT, _ROW + ["1"]),
+    "k_lines": _rows(_NT, _LINES + _LINES_BETA),
+    "k_dim1": _rows(_NT_DIM1, _DIM1[1:] + _DIM1_BETA),
+    "kb_col": _rows(_NT, _COL),
+    "kb_row": _rows(_NT, _ROW),
+    "kb_lines": _rows(_NT, _LINES),
+    "kb_dim1": _rows(_NT_DIM1, _DIM1),
 }
 
 

@@ -128,9 +128,9 @@ int csipm_op_fft_shape(csipm_op_t h, int axis, int* fft_len, int* rows, int* mod
 /* Autotuned launch shapes of the batch engine's FFT passes (no counterpart
  * in the reference): for pass kind 0 (line pass) or 1 (dimension-1 pass),
  * complex element size 8 (FP32) or 16 (FP64), FFT length and LDS rows, cap
- * the tile at 2^lg_cap lines (line pairs) per workgroup and run it on nt
- * threads (128 or 256; 0 keeps the built-in choice); lg_cap < 0 removes the
- * entry.  csipm.tune measures the candidates and writes the committed
+ * the tile at 2^lg_cap lines (line pairs) per workgroup; lg_cap < 0 removes
+ * the entry.  nt (0, 128 or 256) is kept for callers and has no effect: the
+ * workgroup size follows from the tile.  csipm.tune measures the candidates and writes the committed
  * table the package loads at start-up.  Takes effect at the next table
  * rebuild of an engine (a new batch, or the next change of its instances). */
 int csipm_tune_set(int kind, int elem_bytes, int fft_len, int rows, int lg_cap, int nt);

@@ -218,3 +218,25 @@ def test_complex_path_operator(cuda, dims):
     assert np.array_equal(v, maps.beta_to_dft(x, dims, rdft=False))
     assert np.array_equal(DFT_to_beta(o, torch.from_numpy(v).to(cuda)).cpu().numpy(),
                           maps.dft_to_beta(v, dims))
+
+
+# the workgroup size follows from the tile: 256 threads up to 2048 elements,
+# 512 to 4096, 1024 to 8192 and, 16 elements each, beyond (dimension 1);
+# sizes on both sides of each line, in every pass kind (4091: Bluestein of
+# about 8190; 65536 = 256 x 256 and 4608 = 64 x 72 four-step)
+@pytest.mark.parametrize("dims", [(2048,), (2058,), (4096,), (4091,), (9000, 2), (4104, 3),
+                                  (2, 2048), (6, 2058), (6, 4096), (4608,), (3, 5, 2058)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_workgroup_sizes(cuda, dims, dtype):
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("workgroups", dims, dtype, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 3)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    tol = TOL64 if dtype == torch.float64 else TOL32
+    o = _make(dims, miss, dtype)
+    xt = torch.from_numpy(x).to(cuda, dtype)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
