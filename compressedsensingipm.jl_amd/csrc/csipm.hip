@@ -26,9 +26,7 @@
 #include "csipm_batch.hpp"
 // the FFT pass kernels are compiled in separate translation units when the
 // build provides their declarations
-#if __has_include("fft_extern.inc")
 #include "fft_extern.inc"
-#endif
 
 using namespace csipm;
 
@@ -1035,21 +1033,117 @@ PassArgs<T> dim1_args(csipm_op* h, const void* src, const T* real_in, T* real_ou
   return a;
 }
 
-#define CSIPM_PASS(NT, kern)                                                 \
-  do {                                                                       \
-    auto kern_ = kern;                                                       \
-    CHK(allow_lds(kern_, c.lds));                                            \
-    hipLaunchKernelGGL(kern_, dim3(c.grid), dim3(NT), c.lds, h->stream, a);  \
-    HIPCHK(hipGetLastError());                                               \
-    return CSIPM_OK;                                                         \
+enum { PK_LINES = 0, PK_DIM1 = 1, PK_COL = 2, PK_ROW = 3 };
+struct PassSpec {
+  int kind, D, src, dst, fm, axis;  // fm: FWD (lines), MODE (dim1, col, row)
+};
+
+// the load, middle step and store of pass s (obs: outer Bluestein)
+template <typename T>
+void set_steps(PassArgs<T>& a, const PassSpec& s, bool obs) {
+  a.mid = MID_NONE;
+  if (s.kind == PK_LINES) {
+    const bool two = s.D == 2;
+    a.ld = s.src == SRC_BUF ? (s.fm ? LD_LINES_BUF_FWD : LD_LINES_BUF_INV)
+           : s.src == SRC_U ? (two ? LD_LINES_U2 : LD_LINES_U3)
+                            : (two ? LD_LINES_BETA2 : LD_LINES_BETA3);
+    a.st = s.dst == DST_BUF ? (s.fm ? ST_LINES_BUF_FWD : ST_LINES_BUF_INV)
+           : s.dst == DST_U ? (two ? ST_LINES_U2 : ST_LINES_U3)
+                            : (two ? ST_LINES_BETA2 : ST_LINES_BETA3);
+  } else if (s.kind == PK_DIM1) {
+    a.ld = s.src == SRC_BUF ? LD_DIM1_BUF : s.src == SRC_U ? LD_DIM1_U
+           : s.src == SRC_BETA ? LD_DIM1_BETA : LD_DIM1_REAL;
+    a.st = s.dst == DST_BUF ? ST_DIM1_BUF : s.dst == DST_U ? ST_DIM1_U
+           : s.dst == DST_BETA ? ST_DIM1_BETA : ST_DIM1_REAL;
+    if (s.fm == MODE_MTM) a.mid = MID_DIM1_MASK;
+  } else if (s.kind == PK_COL) {
+    // a direct transform starts inverse and ends forward, an outer Bluestein
+    // one the other way round
+    switch (s.fm) {
+      case C_FIRST:
+        a.ld = s.src == SRC_BETA ? LD_COL_FIRST_BETA : LD_COL_FIRST_U;
+        a.st = obs ? ST_COL_BUF_FWD : ST_COL_BUF_INV;
+        break;
+      case C_REAL_IN:
+        a.ld = LD_COL_REAL;
+        a.st = ST_COL_BUF_FWD;
+        break;
+      case C_MID:
+        a.ld = LD_COL_BUF_INV;
+        a.mid = MID_COL;
+        a.st = ST_COL_BUF_FWD;
+        break;
+      case C_MID_C2R:
+        a.ld = LD_COL_BUF_INV;
+        a.st = ST_COL_REAL;
+        break;
+      default:   // C_LAST
+        a.ld = obs ? LD_COL_BUF_INV : LD_COL_BUF_FWD;
+        a.st = s.dst == DST_BETA ? ST_COL_BETA : ST_COL_U;
+    }
+  } else {
+    switch (s.fm) {
+      case R_MTM:
+        a.ld = LD_ROW_INV;
+        a.mid = MID_ROW_MASK;
+        a.st = ST_ROW_FWD;
+        break;
+      case R_C2R:
+        a.ld = LD_ROW_INV;
+        a.st = ST_ROW_REAL;
+        break;
+      case R_R2C:
+        a.ld = LD_ROW_REAL;
+        a.st = ST_ROW_FWD;
+        break;
+      default:   // R_CONV_INV, R_CONV_FWD
+        a.ld = LD_ROW_FWD;
+        a.mid = s.fm == R_CONV_INV ? MID_ROW_CONV_INV : MID_ROW_CONV_FWD;
+        a.st = ST_ROW_INV;
+    }
+  }
+}
+
+// one pass of one instance: grid tiles on workgroups sized nt (tile_nt)
+template <typename T>
+int launch_pass(csipm_op* h, const PassArgs<T>& a, int grid, int nt, size_t lds) {
+#define CSIPM_PASS(NT, E, LD, MID, ST)                                           \
+  do {                                                                           \
+    auto kern = k_pass<T, NT, E, LD, MID, ST>;                                   \
+    CHK(allow_lds(kern, lds));                                                   \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, h->stream, a);           \
+    HIPCHK(hipGetLastError());                                                   \
+    return CSIPM_OK;                                                             \
   } while (0)
+#define CSIPM_IS(LD, MID, ST) a.ld == LD && a.mid == MID && a.st == ST
+#define CSIPM_SHORT(LD, MID, ST)                          \
+  if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
+    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
+  }
+#define CSIPM_DIM1(LD, MID, ST)                           \
+  CSIPM_SHORT(LD, MID, ST)                                \
+  if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST);    \
+    CSIPM_PASS(1024, 16, LD, MID, ST);                    \
+  }
+  CSIPM_CHAIN_DIM1(CSIPM_DIM1)
+  CSIPM_ENTRY_DIM1(CSIPM_DIM1)
+  CSIPM_CHAIN_SHORT(CSIPM_SHORT)
+  CSIPM_ENTRY_SHORT(CSIPM_SHORT)
+#undef CSIPM_PASS
+#undef CSIPM_SHORT
+#undef CSIPM_DIM1
+  return fail(CSIPM_ERR_UNSUPPORTED, "no kernel for pass (%d, %d, %d) on %d threads", a.ld, a.mid,
+              a.st, nt);
+}
 
 template <typename T, int D, int SRC, int DST, bool FWD>
 int launch_lines(csipm_op* h, int axis, const void* src, const Epi<T>& epi, const int* done) {
   const LineCfg& c = h->ps<T>().lines[axis];
   PassArgs<T> a = lines_args<T>(h, axis, src, epi, done);
-  if (c.nt == 256) CSIPM_PASS(256, (k_lines<T, 256, kE, D, SRC, DST, FWD>));
-  CSIPM_PASS(512, (k_lines<T, 512, kE, D, SRC, DST, FWD>));
+  set_steps(a, {PK_LINES, D, SRC, DST, FWD ? 1 : 0, axis}, false);
+  return launch_pass(h, a, c.grid, c.nt, c.lds);
 }
 
 template <typename T, int D, int SRC, int DST, int MODE>
@@ -1057,12 +1151,9 @@ int launch_dim1(csipm_op* h, const void* src, const T* real_in, T* real_out, con
                 T scale, const int* done) {
   const Dim1Cfg& c = h->ps<T>().d1;
   PassArgs<T> a = dim1_args<T>(h, src, real_in, real_out, epi, scale, done);
-  switch (c.nt) {
-    case 256: CSIPM_PASS(256, (k_dim1<T, 256, kE, D, SRC, DST, MODE>));
-    case 512: CSIPM_PASS(512, (k_dim1<T, 512, kE, D, SRC, DST, MODE>));
-    case 1024: CSIPM_PASS(1024, (k_dim1<T, 1024, kE, D, SRC, DST, MODE>));
-    default: CSIPM_PASS(1024, (k_dim1<T, 1024, 16, D, SRC, DST, MODE>));
-  }
+  set_steps(a, {PK_DIM1, D, MODE == MODE_R2C ? SRC_REAL : SRC, MODE == MODE_C2R ? DST_REAL : DST, MODE, 0},
+            false);
+  return launch_pass(h, a, c.grid, c.nt, c.lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1103,11 +1194,6 @@ PassArgs<T> big_args(csipm_op* h, bool col, const void* src, const T* real_in, T
   a.done = done;
   return a;
 }
-
-enum { PK_LINES = 0, PK_DIM1 = 1, PK_COL = 2, PK_ROW = 3 };
-struct PassSpec {
-  int kind, D, src, dst, fm, axis;  // fm: FWD (lines), MODE (dim1, col, row)
-};
 
 // pass sequence of a long 1D line.  which: 0 M^T M (+ epilogue), 1 M^T z from
 // real samples, 2 M beta to real samples
@@ -1150,48 +1236,6 @@ int big_specs(const csipm_op* h, int which, int src, int dst, PassSpec* s) {
   return 3;
 }
 
-// one four-step pass of a single instance
-template <typename T>
-int launch_big_pass(csipm_op* h, const PassSpec& sp, const PassArgs<T>& a) {
-  const PrecState& ps = h->ps<T>();
-  const int grid = sp.kind == PK_COL ? ps.col.grid : ps.row.grid;
-  const size_t lds = sp.kind == PK_COL ? ps.col.lds : ps.row.lds;
-  const int nt = sp.kind == PK_COL ? ps.col.nt : ps.row.nt;
-#define CSIPM_BIG(K, ...)                                                    \
-  do {                                                                       \
-    auto kern = nt == 256 ? K<T, 256, kE, __VA_ARGS__> : K<T, 512, kE, __VA_ARGS__>; \
-    CHK(allow_lds(kern, lds));                                               \
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, h->stream, a);       \
-    HIPCHK(hipGetLastError());                                               \
-    return CSIPM_OK;                                                         \
-  } while (0)
-  if (sp.kind == PK_COL) {
-    switch (sp.fm) {
-      case C_FIRST:
-        if (sp.src == SRC_BETA) CSIPM_BIG(k_col, SRC_BETA, DST_BUF, C_FIRST);
-        CSIPM_BIG(k_col, SRC_U, DST_BUF, C_FIRST);
-      case C_REAL_IN: CSIPM_BIG(k_col, SRC_REAL, DST_BUF, C_REAL_IN);
-      case C_MID: CSIPM_BIG(k_col, SRC_BUF, DST_BUF, C_MID);
-      case C_MID_C2R: CSIPM_BIG(k_col, SRC_BUF, DST_REAL, C_MID_C2R);
-      case C_LAST:
-        if (sp.dst == DST_BETA) CSIPM_BIG(k_col, SRC_BUF, DST_BETA, C_LAST);
-        CSIPM_BIG(k_col, SRC_BUF, DST_U, C_LAST);
-      default: break;
-    }
-  } else {
-    switch (sp.fm) {
-      case R_MTM: CSIPM_BIG(k_row, R_MTM);
-      case R_C2R: CSIPM_BIG(k_row, R_C2R);
-      case R_R2C: CSIPM_BIG(k_row, R_R2C);
-      case R_CONV_INV: CSIPM_BIG(k_row, R_CONV_INV);
-      case R_CONV_FWD: CSIPM_BIG(k_row, R_CONV_FWD);
-      default: break;
-    }
-  }
-#undef CSIPM_BIG
-  return fail(CSIPM_ERR_UNSUPPORTED, "no four-step kernel for pass (%d, %d)", sp.kind, sp.fm);
-}
-
 // run a four-step pass sequence on one instance; ev: an event after every pass
 template <typename T>
 int run_big(csipm_op* h, int which, int src, int dst, const void* x, const T* real_in,
@@ -1201,7 +1245,10 @@ int run_big(csipm_op* h, int which, int src, int dst, const void* x, const T* re
   for (int k = 0; k < np; ++k) {
     const bool col = sp[k].kind == PK_COL;
     PassArgs<T> a = big_args<T>(h, col, x, real_in, real_out, epi, scale, done);
-    CHK(launch_big_pass<T>(h, sp[k], a));
+    set_steps(a, sp[k], h->obs);
+    const PrecState& ps = h->ps<T>();
+    CHK(launch_pass(h, a, col ? ps.col.grid : ps.row.grid, col ? ps.col.nt : ps.row.nt,
+                    col ? ps.col.lds : ps.row.lds));
     if (ev) HIPCHK(hipEventRecord(ev[k], h->stream));
   }
   return CSIPM_OK;

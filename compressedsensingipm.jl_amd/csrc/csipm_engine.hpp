@@ -84,66 +84,6 @@ int chain_specs(const csipm_op* h, int which, PassSpec* s) {
   return 3;
 }
 
-// the batched kernel of one pass spec (the combinations the chains use)
-template <typename T, int NT, int E>
-int launch_spec(const PassSpec& s, int grid, size_t lds, hipStream_t st, const void* tabv,
-                BSeg seg) {
-  const PassArgs<T>* tab = (const PassArgs<T>*)tabv;
-#define CSIPM_LAUNCH(kern)                                                      \
-  do {                                                                          \
-    CHK(allow_lds(kern, lds));                                                  \
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, st, tab, seg);          \
-    HIPCHK(hipGetLastError());                                                  \
-    return CSIPM_OK;                                                            \
-  } while (0)
-  if (s.kind == PK_LINES) {
-    if constexpr (NT * E <= kTile) {
-      if (s.D == 2 && s.src == SRC_U && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 2, SRC_U, DST_BUF, false>));
-      if (s.D == 2 && s.src == SRC_BUF && s.dst == DST_U && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 2, SRC_BUF, DST_U, true>));
-      if (s.D == 3 && s.src == SRC_U && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_U, DST_BUF, false>));
-      if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_BUF && !s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_BUF, false>));
-      if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_BUF && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_BUF, true>));
-      if (s.D == 3 && s.src == SRC_BUF && s.dst == DST_U && s.fm)
-        CSIPM_LAUNCH((kb_lines<T, NT, E, 3, SRC_BUF, DST_U, true>));
-    }
-  } else if (s.kind == PK_COL) {
-    if constexpr (NT * E <= kTile) {
-    if (s.fm == C_FIRST) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_U, DST_BUF, C_FIRST>));
-    if (s.fm == C_REAL_IN) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_REAL, DST_BUF, C_REAL_IN>));
-    if (s.fm == C_MID) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_BUF, DST_BUF, C_MID>));
-    if (s.fm == C_LAST) CSIPM_LAUNCH((kb_col<T, NT, E, SRC_BUF, DST_U, C_LAST>));
-    }
-  } else if (s.kind == PK_ROW) {
-    if constexpr (NT * E <= kTile) {
-    if (s.fm == R_MTM) CSIPM_LAUNCH((kb_row<T, NT, E, R_MTM>));
-    if (s.fm == R_R2C) CSIPM_LAUNCH((kb_row<T, NT, E, R_R2C>));
-    if (s.fm == R_CONV_INV) CSIPM_LAUNCH((kb_row<T, NT, E, R_CONV_INV>));
-    if (s.fm == R_CONV_FWD) CSIPM_LAUNCH((kb_row<T, NT, E, R_CONV_FWD>));
-    }
-  } else {
-    if (s.D == 1 && s.src == SRC_U && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 1, SRC_U, DST_U, MODE_MTM>));
-    if (s.D == 1 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 1, SRC_REAL, DST_U, MODE_R2C>));
-    if (s.D == 2 && s.src == SRC_BUF && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 2, SRC_BUF, DST_BUF, MODE_MTM>));
-    if (s.D == 2 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 2, SRC_REAL, DST_BUF, MODE_R2C>));
-    if (s.D == 3 && s.src == SRC_BUF && s.fm == MODE_MTM)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 3, SRC_BUF, DST_BUF, MODE_MTM>));
-    if (s.D == 3 && s.src == SRC_REAL && s.fm == MODE_R2C)
-      CSIPM_LAUNCH((kb_dim1<T, NT, E, 3, SRC_REAL, DST_BUF, MODE_R2C>));
-  }
-#undef CSIPM_LAUNCH
-  return fail(CSIPM_ERR_UNSUPPORTED, "no batched kernel for pass (%d,%d,%d,%d,%d)", s.kind, s.D,
-              s.src, s.dst, s.fm);
-}
-
 // Launch tables of a rebuild (chain pass arguments, block -> instance maps,
 // vector segments) are staged on the host, packed into one pinned buffer and
 // copied to one device buffer by a single asynchronous copy on the engine's
@@ -200,17 +140,18 @@ struct TableArena {
   }
 };
 
-// one launch of a chain: a pass over a subset of instances
+// one launch of a chain: the passes at one position of the chains of the
+// instances whose workgroups have one size there
 struct ChainSub {
-  PassSpec spec;
-  int pass = 0;          // index of the pass in its chain
+  int pass = 0;          // position in the chains
   std::vector<int> ids;  // member instance ids
+  bool side = false;     // only whole 1D lines of long transforms: independent of the rest
+  int ld = -1, mid = -1, st = -1;   // the members' steps, -1 when they differ
   int nt = kNT, grid = 0;
   size_t lds = 0;
-  void* tab = nullptr;   // device PassArgs<T>[members] (in a table arena)
-  int* seg = nullptr;    // device: block -> member, then member -> first block
-  size_t tab_off = 0, seg_off = 0;   // their offsets in the arena
-  int members = 0;
+  void* tab = nullptr;        // device PassArgs<T>[members] (in a table arena)
+  BlockMap* map = nullptr;    // device: block -> (member, tile)
+  size_t tab_off = 0, map_off = 0;   // their offsets in the arena
 };
 
 struct Chain {
@@ -221,7 +162,7 @@ struct Chain {
   void bind(char* base) {
     for (ChainSub& s : subs) {
       s.tab = base + s.tab_off;
-      s.seg = (int*)(base + s.seg_off);
+      s.map = (BlockMap*)(base + s.map_off);
     }
   }
 };
@@ -240,42 +181,59 @@ struct VsegOff {
 };
 
 template <typename T>
-int launch_sub(const ChainSub& s, hipStream_t st) {
-  BSeg seg{s.seg, s.seg + s.grid};
-  switch (s.nt) {
-    case 256: return launch_spec<T, 256, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
-    case 512: return launch_spec<T, 512, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
-    case 1024: return launch_spec<T, 1024, kE>(s.spec, s.grid, s.lds, st, s.tab, seg);
-    default: return launch_spec<T, 1024, 16>(s.spec, s.grid, s.lds, st, s.tab, seg);
+int launch_sub(const ChainSub& a, hipStream_t st) {
+  const int nt = a.nt;
+#define CSIPM_PASS(NT, E, LD, MID, ST)                                                \
+  do {                                                                                \
+    auto kern = kb_pass<T, NT, E, LD, MID, ST>;                                       \
+    CHK(allow_lds(kern, a.lds));                                                      \
+    hipLaunchKernelGGL(kern, dim3(a.grid), dim3(NT), a.lds, st, (const PassArgs<T>*)a.tab, \
+                       a.map);                                                        \
+    HIPCHK(hipGetLastError());                                                        \
+    return CSIPM_OK;                                                                  \
+  } while (0)
+#define CSIPM_SHORT(LD, MID, ST)                          \
+  if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
+    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
   }
+#define CSIPM_DIM1(LD, MID, ST)                           \
+  CSIPM_SHORT(LD, MID, ST)                                \
+  if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST);    \
+    CSIPM_PASS(1024, 16, LD, MID, ST);                    \
+  }
+  CSIPM_DIM1(-1, -1, -1)
+  CSIPM_CHAIN_DIM1(CSIPM_DIM1)
+  CSIPM_CHAIN_SHORT(CSIPM_SHORT)
+#undef CSIPM_PASS
+#undef CSIPM_SHORT
+#undef CSIPM_DIM1
+#undef CSIPM_IS
+  return fail(CSIPM_ERR_UNSUPPORTED, "no batched kernel for pass (%d, %d, %d) on %d threads", a.ld,
+              a.mid, a.st, nt);
 }
 
+// A chain's launches in order on `st`, those of long 1D lines (one workgroup
+// of 1024 threads per instance, about 40 us) beside them on `side`: a fork
+// from `st` and a join back into it, which a graph capture of `st` records as
+// two branches.
 template <typename T>
-int run_chain(const Chain& c, hipStream_t st) {
-  for (const ChainSub& s : c.subs) CHK(launch_sub<T>(s, st));
-  return CSIPM_OK;
-}
-
-// the same with the passes of the 1D and 2D instances on `side`, concurrent
-// with those of the 3D instances on `st` (the instances of a launch are
-// independent; each dimensionality keeps its pass order): a fork from `st`
-// and a join back into it, which a graph capture of `st` records as two
-// branches.  The small instances' passes, latency-bound launches of few
-// workgroups, then fill the CUs the 3D passes leave idle.
-template <typename T>
-int run_chain_par(const Chain& c, hipStream_t st, hipStream_t side, hipEvent_t fork_ev,
-                  hipEvent_t join_ev) {
-  bool big = false, small = false;
-  for (const ChainSub& s : c.subs) (s.spec.D == 3 ? big : small) = true;
-  if (!big || !small || !side) return run_chain<T>(c, st);
-  HIPCHK(hipEventRecord(fork_ev, st));
-  HIPCHK(hipStreamWaitEvent(side, fork_ev, 0));
+int run_chain(const Chain& c, hipStream_t st, hipStream_t side, hipEvent_t fork_ev,
+              hipEvent_t join_ev) {
+  bool fork = false, rest = false;
+  for (const ChainSub& s : c.subs) (s.side ? fork : rest) = true;
+  fork = fork && rest;
+  if (fork) {
+    HIPCHK(hipEventRecord(fork_ev, st));
+    HIPCHK(hipStreamWaitEvent(side, fork_ev, 0));
+    for (const ChainSub& s : c.subs)
+      if (s.side) CHK(launch_sub<T>(s, side));
+    HIPCHK(hipEventRecord(join_ev, side));
+  }
   for (const ChainSub& s : c.subs)
-    if (s.spec.D != 3) CHK(launch_sub<T>(s, side));
-  HIPCHK(hipEventRecord(join_ev, side));
-  for (const ChainSub& s : c.subs)
-    if (s.spec.D == 3) CHK(launch_sub<T>(s, st));
-  HIPCHK(hipStreamWaitEvent(st, join_ev, 0));
+    if (!fork || !s.side) CHK(launch_sub<T>(s, st));
+  if (fork) HIPCHK(hipStreamWaitEvent(st, join_ev, 0));
   return CSIPM_OK;
 }
 
@@ -304,9 +262,9 @@ struct Engine {
   hipStream_t stream = nullptr;   // the engine's own stream (all its work)
   hipStream_t user = nullptr;     // the caller's stream, ordered around every call
   hipEvent_t ev = nullptr;
-  // a second stream: an apply's passes of the 1D and 2D instances run on it
-  // beside those of the 3D instances (forked from and joined back into
-  // `stream`, also inside the captured CG chunks)
+  // a second stream: an apply's launches of long 1D lines run on it beside
+  // the others (forked from and joined back into `stream`, also inside the
+  // captured CG chunks)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   bool use_graphs = true;         // CG chunks replayed as captured HIP graphs
@@ -600,6 +558,7 @@ int chain_call_args(Engine* E, int id, int call, int nb, const PassSpec& s,
   if (s.kind == PK_LINES) a = lines_args<T>(h, s.axis, src, e, done, &bc.lines[s.axis]);
   else if (s.kind == PK_DIM1) a = dim1_args<T>(h, src, real_in, nullptr, e, scale, done, &bc.d1);
   else a = big_args<T>(h, s.kind == PK_COL, src, real_in, nullptr, e, scale, done, &bc.col, &bc.row);
+  set_steps(a, s, h->obs);
   return CSIPM_OK;
 }
 
@@ -610,76 +569,95 @@ inline int pass_nt(const PassSpec& s, const BatchCfg& bc) {
   return s.kind == PK_COL ? bc.col.nt : bc.row.nt;
 }
 
+// Block map of a launch over members with `grids` tiles each.  Block b runs on
+// XCD b % 8, each XCD with its own L2: a member's tiles go to the XCDs in
+// eight consecutive ranges (adjacent tiles share cache lines), the few tiles
+// of a small member to one XCD after another, and the members follow each
+// other on every XCD in their order.  The lists are evened out by fillers.
+std::vector<BlockMap> block_map(const std::vector<int>& grids) {
+  constexpr int kXcd = 8;
+  std::vector<BlockMap> list[kXcd];
+  int next = 0;
+  for (int m = 0; m < (int)grids.size(); ++m) {
+    const int64_t g = grids[(size_t)m];
+    if (g < kXcd) {
+      for (int t = 0; t < g; ++t) list[next++ % kXcd].push_back({m, t});
+      continue;
+    }
+    for (int x = 0; x < kXcd; ++x)
+      for (int64_t t = x * g / kXcd; t < (x + 1) * g / kXcd; ++t)
+        list[(x + next) % kXcd].push_back({m, (int)t});
+    ++next;
+  }
+  size_t len = 0;
+  for (const auto& l : list) len = std::max(len, l.size());
+  std::vector<BlockMap> map;
+  map.reserve(len * kXcd);
+  for (size_t r = 0; r < len; ++r)
+    for (const auto& l : list) map.push_back(r < l.size() ? l[r] : BlockMap{-1, 0});
+  while (!map.empty() && map.back().member < 0) map.pop_back();
+  return map;
+}
+
 template <typename T>
 int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call, int nb,
                 Chain& out) {
   out.release();
   out.esize = sizeof(T);
-  for (int key : {1, 2, 3, 10, 11}) {
-    std::vector<int> mem;
-    for (int id : ids)
-      if (chain_key(E->inst[(size_t)id].h) == key) mem.push_back(id);
-    if (mem.empty()) continue;
+  struct Member {
+    int id, np;
     PassSpec specs[8];
-    const int np = chain_specs(E->inst[(size_t)mem[0]].h, call == CALL_MTZ ? CH_MTZ : CH_MTM,
-                               specs);
-    for (int p = 0; p < np; ++p) {
-      const PassSpec& s = specs[p];
-      for (int nt : {256, 512, 1024, kNTLong}) {
-        std::vector<PassArgs<T>> tab;
-        std::vector<int> grids;
-        size_t lds = 0;
-        for (int id : mem) {
-          csipm_op* h = E->inst[(size_t)id].h;
-          const BatchCfg bc = batch_cfg<T>(h, (int)ids.size());
-          const int want = pass_nt(s, bc);
-          if (want != nt) continue;
-          PassArgs<T> a{};
-          CHK(chain_call_args<T>(E, id, call, nb, s, bc, a));
-          tab.push_back(a);
-          if (s.kind == PK_LINES) {
-            grids.push_back(bc.lines[s.axis].grid);
-            lds = std::max(lds, bc.lines[s.axis].lds);
-          } else if (s.kind == PK_DIM1) {
-            grids.push_back(bc.d1.grid);
-            lds = std::max(lds, bc.d1.lds);
-          } else if (s.kind == PK_COL) {
-            grids.push_back(bc.col.grid);
-            lds = std::max(lds, bc.col.lds);
-          } else {
-            grids.push_back(bc.row.grid);
-            lds = std::max(lds, bc.row.lds);
-          }
-        }
-        if (tab.empty()) continue;
-        ChainSub sub;
-        sub.spec = s;
-        sub.pass = p;
-        for (int id : mem) {
-          csipm_op* hm = E->inst[(size_t)id].h;
-          const int want = pass_nt(s, batch_cfg<T>(hm, (int)ids.size()));
-          if (want == nt) sub.ids.push_back(id);
-        }
-        sub.nt = nt;
-        sub.lds = lds;
-        sub.members = (int)tab.size();
-        std::vector<int> segv;
-        std::vector<int> first;
-        int tot = 0;
-        for (size_t m = 0; m < tab.size(); ++m) {
-          first.push_back(tot);
-          for (int b = 0; b < grids[m]; ++b) segv.push_back((int)m);
-          tot += grids[m];
-        }
-        first.push_back(tot);
-        sub.grid = tot;
-        segv.insert(segv.end(), first.begin(), first.end());
-        sub.tab_off = A.put(tab.data(), sizeof(PassArgs<T>) * tab.size());
-        sub.seg_off = A.put(segv.data(), sizeof(int) * segv.size());
-        out.subs.push_back(sub);
-      }
+    BatchCfg bc;
+  };
+  // whole 1D lines first: their workgroups run longest
+  std::vector<Member> mem;
+  for (bool line : {true, false})
+    for (int id : ids) {
+      csipm_op* h = E->inst[(size_t)id].h;
+      if ((chain_key(h) == 1) != line) continue;
+      Member m;
+      m.id = id;
+      m.np = chain_specs(h, call == CALL_MTZ ? CH_MTZ : CH_MTM, m.specs);
+      m.bc = batch_cfg<T>(h, (int)ids.size());
+      mem.push_back(m);
     }
-  }
+  for (int p = 0; p < 8; ++p)
+    for (int nt : {kNTLong, 1024, 512, 256}) {
+      ChainSub sub;
+      sub.pass = p;
+      sub.nt = nt;
+      sub.side = nt >= 1024;
+      std::vector<PassArgs<T>> tab;
+      std::vector<int> grids;
+      for (const Member& m : mem) {
+        if (p >= m.np || pass_nt(m.specs[p], m.bc) != nt) continue;
+        const PassSpec& s = m.specs[p];
+        PassArgs<T> a{};
+        CHK(chain_call_args<T>(E, m.id, call, nb, s, m.bc, a));
+        const bool same = tab.empty() || (sub.ld == a.ld && sub.mid == a.mid && sub.st == a.st);
+        sub.ld = same ? a.ld : -1;
+        sub.mid = same ? a.mid : -1;
+        sub.st = same ? a.st : -1;
+        tab.push_back(a);
+        sub.ids.push_back(m.id);
+        if (m.np > 1) sub.side = false;
+        if (s.kind == PK_LINES || s.kind == PK_COL) {
+          const LineCfg& c = s.kind == PK_LINES ? m.bc.lines[s.axis] : m.bc.col;
+          grids.push_back(c.grid);
+          sub.lds = std::max(sub.lds, c.lds);
+        } else {
+          const Dim1Cfg& c = s.kind == PK_DIM1 ? m.bc.d1 : m.bc.row;
+          grids.push_back(c.grid);
+          sub.lds = std::max(sub.lds, c.lds);
+        }
+      }
+      if (tab.empty()) continue;
+      const std::vector<BlockMap> map = block_map(grids);
+      sub.grid = (int)map.size();
+      sub.tab_off = A.put(tab.data(), sizeof(PassArgs<T>) * tab.size());
+      sub.map_off = A.put(map.data(), sizeof(BlockMap) * map.size());
+      out.subs.push_back(sub);
+    }
   return CSIPM_OK;
 }
 
@@ -911,7 +889,7 @@ int engine_init_fresh(Engine* E) {
     mtz.bind(base);
     vs.bind(base, &seg, &ids);
     grid = vs.grid;
-    if ((rc = run_chain<double>(mtz, E->stream)) != CSIPM_OK) break;
+    if ((rc = run_chain<double>(mtz, E->stream, E->side, E->fork_ev, E->join_ev)) != CSIPM_OK) break;
     hipLaunchKernelGGL(bk_absmax, dim3(grid), dim3(kNT), 0, E->stream, seg, E->info, E->flags,
                        E->W(V_B), E->part);
     if ((rc = finalize(E, seg, ids, (int)fresh.size(), {1}, 0, S_BNORM, 0, 0, 0)) != CSIPM_OK)
@@ -944,13 +922,13 @@ int cg_iteration(Engine* E, int nb, bool reliable) {
   TC *z = E->C2<TC>(C2_Z), *p = E->C2<TC>(C2_P), *q = E->C2<TC>(C2_Q);
   TC *P11 = E->C<TC>(C_P11), *P12 = E->C<TC>(C_P12), *P22 = E->C<TC>(C_P22);
   hipStream_t st = E->stream;
-  CHK(run_chain_par<TC>(E->chains[CALL_CGA], st, E->side, E->fork_ev, E->join_ev));
+  CHK(run_chain<TC>(E->chains[CALL_CGA], st, E->side, E->fork_ev, E->join_ev));
   hipLaunchKernelGGL((bk_cg_update<TC>), dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info,
                      E->cg, x, r, z, p, q, P11, P12, P22, nb, E->part);
   hipLaunchKernelGGL(bk_cg_gamma, dim3(na), dim3(kNT), 0, st, E->vseg, E->ids, E->info, E->cg,
                      E->part);
   if (reliable) {
-    CHK(run_chain_par<TC>(E->chains[CALL_CGR], st, E->side, E->fork_ev, E->join_ev));
+    CHK(run_chain<TC>(E->chains[CALL_CGR], st, E->side, E->fork_ev, E->join_ev));
     hipLaunchKernelGGL((bk_cg_residual<TC>), dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info,
                        E->cg, b, q, r, z, P11, P12, P22, nb, E->part);
     hipLaunchKernelGGL(bk_cg_regamma, dim3(na), dim3(kNT), 0, st, E->vseg, E->ids, E->info,
@@ -1084,7 +1062,7 @@ int engine_newton(Engine* E, double atol, double rtol, int reliable, bool refine
                      E->flags, E->C2<TC>(C2_D), E->W2(V2_DD), 1);
   hipLaunchKernelGGL((bk_convert<double, double>), dim3(E->vgrid), dim3(kNT), 0, st, sg, E->info,
                      E->flags, E->W2(V2_RHSD), E->W2(V2_TMP), 1);
-  CHK(run_chain_par<double>(E->chains[CALL_REF], st, E->side, E->fork_ev, E->join_ev));
+  CHK(run_chain<double>(E->chains[CALL_REF], st, E->side, E->fork_ev, E->join_ev));
   hipLaunchKernelGGL((bk_convert<double, TC>), dim3(E->vgrid), dim3(kNT), 0, st, sg, E->info,
                      E->flags, E->W2(V2_TMP), E->C2<TC>(C2_RHS), 1);
   HIPCHK(hipGetLastError());
@@ -1133,7 +1111,7 @@ int engine_step(Engine* E, double tol, int max_iter, double cg_atol, double cg_r
   // the correction is a 1e-5 part of d, so FP64-level accuracy)
   TC* rhs = E->C2<TC>(C2_RHS);
   double* rhsd = E->mixed ? E->W2(V2_RHSD) : nullptr;
-  if (!E->mixed) CHK(run_chain<double>(E->chains[CALL_QB], st));
+  if (!E->mixed) CHK(run_chain<double>(E->chains[CALL_QB], st, E->side, E->fork_ev, E->join_ev));
   // mixed: the reduced system comes from the residual kernel's own loads
   if (E->mixed)
     hipLaunchKernelGGL((bk_ipm_resid_prep_red<TC>), dim3(g), dim3(kNT), 0, st, sg, E->info,
@@ -1288,22 +1266,23 @@ int engine_apply_timed(Engine* E, int64_t nrep, double* ms, double* bytes, std::
     double b = 0;
     const char* nm[8];
     double by[8];
+    // "<dim>d:<pass>" of each kind of member, joined by '+'
+    std::string name;
     for (int id : sb.ids) {
+      const csipm_op* h = E->inst[(size_t)id].h;
       kkt_pass_info(E->inst[(size_t)id].h, layout, nm, by);
       b += by[sb.pass];
+      const std::string one = std::to_string(h->dim) + (h->big ? "d-4step:" : "d:") + nm[sb.pass];
+      if (("+" + name + "+").find("+" + one + "+") == std::string::npos)
+        name += (name.empty() ? "" : "+") + one;
     }
-    kkt_pass_info(E->inst[(size_t)sb.ids[0]].h, layout, nm, by);
     ms[k] = acc[(size_t)k] / (double)nrep;
     bytes[k] = b;
-    names[k] = std::to_string(sb.spec.D) + (sb.spec.kind >= PK_COL ? "d-4step:" : "d:") +
-               nm[sb.pass];
-    // a pass split over several launches: each name carries its workgroup
-    // size and LDS bytes
+    names[k] = name;
+    // a position split over several launches: each name carries its
+    // workgroup size and LDS bytes
     int same = 0;
-    for (const ChainSub& o : c.subs)
-      if (o.pass == sb.pass && o.spec.D == sb.spec.D && o.spec.kind == sb.spec.kind &&
-          o.spec.axis == sb.spec.axis)
-        ++same;
+    for (const ChainSub& o : c.subs) same += o.pass == sb.pass;
     if (same > 1)
       names[k] += "@nt" + std::to_string(sb.nt) + "/lds" + std::to_string(sb.lds);
   }
@@ -1341,7 +1320,7 @@ int engine_admm_init_fresh(Engine* E, double rho) {
     mtz.bind(base);
     vs.bind(base, &seg, &ids);
     grid = vs.grid;
-    if ((rc = run_chain<double>(mtz, E->stream))) break;
+    if ((rc = run_chain<double>(mtz, E->stream, E->side, E->fork_ev, E->join_ev))) break;
     for (int id : fresh) {
       Engine::Inst& in = E->inst[(size_t)id];
       double* ones = E->W(V_DT1) + in.off;   // beta-layout scratch (N <= U slots)

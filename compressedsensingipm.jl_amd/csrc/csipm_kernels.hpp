@@ -366,10 +366,21 @@ __device__ __forceinline__ void store_partial(double* part, double acc, int idx)
 
 // ===========================================================================
 // FFT passes over the (H1, N2, N3) half spectrum.
-//  k_lines: lines along dimension 2 (axis 1) or 3 (axis 2); a workgroup takes
-//           2^lg lines with consecutive k1, so global accesses are contiguous.
-//  k_dim1:  dimension 1; two real lines per complex FFT of length N1
-//           (z = x_a + i x_b), 2^lg pairs per workgroup.
+//  lines: along dimension 2 (axis 1) or 3 (axis 2); a workgroup takes 2^lg
+//         lines with consecutive k1, so global accesses are contiguous.
+//  dim1:  dimension 1; two real lines per complex FFT of length N1
+//         (z = x_a + i x_b), 2^lg pairs per workgroup.
+//  col, row: the four-step passes of long 1D lines, below.
+// One body runs them all (pass_body): a pass is a load, one or two turns of
+// the line transform with a step between them, and a store.  Kernels exist for
+// each combination the single-instance passes and the batched chains use, and
+// one that takes the steps from PassArgs: a batch of several dimensionalities
+// runs the passes at one position of all its chains in one launch of that
+// kernel, side by side instead of one after another.  It is the slower one for
+// passes of one kind (registers and branches of all steps: 255 x 255 FP64 31.9
+// against 39.4 us an apply, 49999 FP32 45 against 59 us) and much the faster
+// one for a mix (48 requests of the serving stream's mix, launches of one kind
+// on two streams 70 ms a solve, mixed launches 57 ms).
 // Sources: SRC_BUF (scratch spectrum), SRC_BETA (gather from beta through the
 // packing map), SRC_U (spectrum-ordered beta), SRC_REAL (real samples, dim 1).
 // Destinations likewise, the beta / u ones with the epilogue Epi.
@@ -377,9 +388,30 @@ __device__ __forceinline__ void store_partial(double* part, double acc, int idx)
 enum { SRC_BUF = 0, SRC_BETA = 1, SRC_REAL = 2, SRC_U = 3 };
 enum { DST_BUF = 0, DST_BETA = 1, DST_REAL = 2, DST_U = 3 };
 enum { MODE_MTM = 0, MODE_C2R = 1, MODE_R2C = 2 };
+// four-step passes (see below)
+enum { C_FIRST = 0, C_REAL_IN = 1, C_MID = 2, C_LAST = 3, C_MID_C2R = 4 };
+enum { R_MTM = 0, R_C2R = 1, R_R2C = 2, R_CONV_INV = 3, R_CONV_FWD = 4 };
+
+// the steps of a pass
+enum {   // load
+  LD_LINES_BUF_FWD, LD_LINES_BUF_INV, LD_LINES_U2, LD_LINES_U3, LD_LINES_BETA2, LD_LINES_BETA3,
+  LD_DIM1_BUF, LD_DIM1_U, LD_DIM1_BETA, LD_DIM1_REAL,
+  LD_COL_FIRST_U, LD_COL_FIRST_BETA, LD_COL_REAL, LD_COL_BUF_FWD, LD_COL_BUF_INV,
+  LD_ROW_FWD, LD_ROW_INV, LD_ROW_REAL
+};
+enum {   // between the two turns (MID_NONE: one turn)
+  MID_NONE, MID_DIM1_MASK, MID_COL, MID_ROW_MASK, MID_ROW_CONV_INV, MID_ROW_CONV_FWD
+};
+enum {   // store
+  ST_LINES_BUF_FWD, ST_LINES_BUF_INV, ST_LINES_U2, ST_LINES_U3, ST_LINES_BETA2, ST_LINES_BETA3,
+  ST_DIM1_BUF, ST_DIM1_U, ST_DIM1_BETA, ST_DIM1_REAL,
+  ST_COL_BUF_FWD, ST_COL_BUF_INV, ST_COL_U, ST_COL_BETA, ST_COL_REAL,
+  ST_ROW_FWD, ST_ROW_INV, ST_ROW_REAL
+};
 
 template <typename T>
 struct PassArgs {
+  int ld, mid, st;      // the pass (LD_*, MID_*, ST_*)
   MapGeom g;
   const FftPlan* plan;  // device-resident
   const cpx<T>* tw;     // the plan's twiddles, stage by stage
@@ -569,15 +601,15 @@ struct Fetched {
   EpiOps<T> ops;
 };
 
-// one workgroup's tile of a line pass (tile = its index within the pass)
-template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
-__device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
-  static_assert(FWD || DST == DST_BUF, "inverse line passes end in the scratch spectrum");
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  // finished instances: the flag is read beside the loads, not before them
-  const int dflag = a.done ? *a.done : 0;
-  const int pl = plan_load(a.plan);
+// block -> instance map of a vector launch over several instances
+struct BSeg {
+  const int* inst;   // instance of each block
+  const int* first;  // first block of each instance (n + 1 entries)
+};
+
+// the tile of a line pass (tile = its index within the pass) into LDS
+template <typename T, int NT, int D, int SRC, bool FWD>
+__device__ __forceinline__ void lines_load(const PassArgs<T>& a, cpx<T>* lds, int tile) {
   const int L = a.len;
   const int lg = a.lg, nl = 1 << lg;
   const int tile1 = tile % a.ntile1;
@@ -627,9 +659,25 @@ __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
       },
       [&](int idx, const Raw<T>& r) { lds[idx] = tile_value<FWD>(raw_value<T, SRC>(r)); });
   }
-  if (dflag) return;
-  __syncthreads();
-  line_dft<T, E, NT>(lds, a, pl, lg, nl);
+}
+
+// ... and out of it; returns the thread's share of x'y
+template <typename T, int NT, int D, int DST, bool FWD>
+__device__ __forceinline__ double lines_store(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int L = a.len;
+  const int lg = a.lg, nl = 1 << lg;
+  const int tile1 = tile % a.ntile1;
+  const int o = tile / a.ntile1;
+  const int k10 = tile1 << lg;
+  const int nv = min(nl, a.H1 - k10);
+  const int64_t s2 = a.H1, s3 = (int64_t)a.H1 * a.g.n[1];
+  const int64_t sl = a.axis == 1 ? s2 : s3;
+  const int64_t base = k10 + (a.axis == 1 ? (int64_t)o * s3 : (int64_t)o * s2);
+  const int total = L << lg;
+  constexpr int K = stage_k<T>();
+  // a tile whose k1 are all representatives (1 <= k1 <= P1) reads and writes
+  // u at the scratch index with the plain sqrt2 scalings of u_to_v / v_to_u
+  const bool interior = k10 >= 1 && k10 + nv - 1 <= a.g.P[0];
   double acc = 0.0;
   if (DST == DST_BUF) {
     staged<NT, K, cpx<T>>(
@@ -685,26 +733,7 @@ __device__ __forceinline__ void lines_body(const PassArgs<T>& a, int tile) {
       acc += spec_store<D, T, DST>(a, k10 + line, k2, k3, lds[idx]);
     }
   }
-  if (DST != DST_BUF && a.epi.dot_part) store_partial(a.epi.dot_part, acc, tile);
-}
-
-template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_lines(PassArgs<T> a) {
-  lines_body<T, NT, E, D, SRC, DST, FWD>(a, xcd_block());
-}
-
-// block -> (instance, tile) map of a launch over several instances
-struct BSeg {
-  const int* inst;   // instance of each block
-  const int* first;  // first block of each instance (n + 1 entries)
-};
-
-template <typename T, int NT, int E, int D, int SRC, int DST, bool FWD>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_lines(const PassArgs<T>* __restrict__ tab, BSeg seg) {
-  const int b = xcd_block();
-  const int i = uniform(seg.inst[b]);
-  const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
-  lines_body<T, NT, E, D, SRC, DST, FWD>(a, b - uniform(seg.first[i]));
+  return acc;
 }
 
 __device__ __forceinline__ bool miss_bit(const uint32_t* m, int64_t s) {
@@ -730,181 +759,209 @@ struct Fetched2 {
   EpiOps<T> ops;
 };
 
-template <typename T, int NT, int E, int D, int SRC, int DST, int MODE>
-__device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  const int dflag = a.done ? *a.done : 0;   // read beside the loads
-  const int pl = plan_load(a.plan);
+// the mask words of a dimension-1 tile's lines are loaded with the tile (into
+// LDS) rather than per element between the transforms: a line's N1 samples
+// span at most mask_row(N1) words
+constexpr int kMaskWords = 640;
+__device__ __forceinline__ int mask_row(int N1) { return (N1 + 31) / 32 + 1; }
+template <typename T>
+__device__ __forceinline__ bool mask_staged(const PassArgs<T>& a) {
+  return a.miss && (2 << a.lg) * mask_row(a.len) <= kMaskWords;
+}
+
+// the tile of a dimension-1 pass from the spectrum, exchanged (the first
+// transform is inverse), and its mask words
+template <typename T, int NT, int D, int SRC>
+__device__ __forceinline__ void dim1_load(const PassArgs<T>& a, cpx<T>* lds, uint32_t* mw,
+                                          int tile) {
   const int N1 = a.len, H1 = a.H1;
   const int lg = a.lg, np = 1 << lg, ps = a.ps;
   const int p0 = tile << lg;
-  const bool even = (N1 & 1) == 0;
-  constexpr int K = stage_k<T>();
   const int nl1 = a.nlines - 1;
-  [[maybe_unused]] int W = 0;            // MODE_MTM, MODE_C2R: the staged mask
-  [[maybe_unused]] bool stage_mask = false;
-  [[maybe_unused]] uint32_t* mw = nullptr;
-  if constexpr (MODE != MODE_R2C) {
-    // the mask words of the tile's lines are loaded with the tile (into LDS)
-    // rather than per element between the transforms: a line's N1 samples
-    // span at most W words
-    constexpr int kMaskWords = 640;
-    constexpr int kMR = (kMaskWords + NT - 1) / NT;
-    __shared__ uint32_t mw_smem[kMR * NT];
-    mw = mw_smem;
-    W = (N1 + 31) / 32 + 1;
-    const int nlt = 2 * np;
-    stage_mask = a.miss && nlt * W <= kMaskWords;
-    uint32_t mreg[kMR];
-    if (stage_mask) {
-      const int64_t nwords = ((int64_t)a.nlines * N1 + 31) >> 5;
+  constexpr int K = stage_k<T>();
+  (void)np, (void)nl1, (void)N1, (void)H1;
+  const bool even = (N1 & 1) == 0;
+  // the mask words of the tile's lines are loaded with the tile (into LDS)
+  // rather than per element between the transforms: a line's N1 samples
+  // span at most W words
+  constexpr int kMR = (kMaskWords + NT - 1) / NT;
+  const int W = mask_row(N1);
+  const int nlt = 2 * np;
+  const bool stage_mask = mask_staged(a);
+  uint32_t mreg[kMR];
+  if (stage_mask) {
+    const int64_t nwords = ((int64_t)a.nlines * N1 + 31) >> 5;
 #pragma unroll
-      for (int r = 0; r < kMR; ++r) {
-        const int i = threadIdx.x + r * NT;
-        const int ll = i / W, j = i - ll * W;
-        const int64_t l = 2 * (int64_t)p0 + ll;
-        const int64_t w = ((l * N1) >> 5) + j;
-        const bool ok = i < nlt * W && l < a.nlines && w < nwords;
-        const uint32_t v = a.miss[ok ? w : 0];
-        mreg[r] = ok ? v : 0u;
-      }
+    for (int r = 0; r < kMR; ++r) {
+      const int i = threadIdx.x + r * NT;
+      const int ll = i / W, j = i - ll * W;
+      const int64_t l = 2 * (int64_t)p0 + ll;
+      const int64_t w = ((l * N1) >> 5) + j;
+      const bool ok = i < nlt * W && l < a.nlines && w < nwords;
+      const uint32_t v = a.miss[ok ? w : 0];
+      mreg[r] = ok ? v : 0u;
     }
-    const int tot = H1 << lg;
-    staged<NT, K, Pair<T>>(
-        tot,
-        [&](int idx) {
-          const int p = udiv(idx, H1, a.h1m);
-          const int k = idx - p * H1;
-          const int la = 2 * (p0 + p);
-          Pair<T> r;
-          r.mode = 0;
-          r.B = {(T)0, (T)0};
-          if (SRC == SRC_BUF) {
-            r.A = a.buf[(int64_t)min(la, nl1) * H1 + k];
-            r.B = a.buf[(int64_t)min(la + 1, nl1) * H1 + k];
-          } else if (SRC == SRC_U) {
-            r.A = a.u_in[u_src<D>(k, 0, 0, a.g, a.H1, r.mode)];   // 1D: a single line
-          } else {
-            r.A = spec_load<D, T, SRC>(a, k, 0, 0);
-          }
-          return r;
-        },
-        [&](int idx, const Pair<T>& r) {
-          const int p = udiv(idx, H1, a.h1m);
-          const int k = idx - p * H1;
-          const int la = 2 * (p0 + p), lb = la + 1;
-          const cpx<T> zero = {(T)0, (T)0};
-          cpx<T> A = la < a.nlines ? (SRC == SRC_U ? u_map(r.A, r.mode) : r.A) : zero;
-          cpx<T> B = (SRC == SRC_BUF && lb < a.nlines) ? r.B : zero;
-          if (k == 0 || (even && k == H1 - 1)) {  // DC / Nyquist of a real line are real
-            A.y = 0;
-            B.y = 0;
-          }
-          // A + i B and its Hermitian partner, exchanged: the transform is inverse
-          lds[k * ps + p] = {A.y + B.x, A.x - B.y};
-          if (k > 0 && N1 - k != k) lds[(N1 - k) * ps + p] = {B.x - A.y, A.x + B.y};
-        });
-    if (stage_mask) {
-#pragma unroll
-      for (int r = 0; r < kMR; ++r) mw[threadIdx.x + r * NT] = mreg[r];
-    }
-  } else {
-    const int totr = N1 << lg;
-    staged<NT, K, cpx<T>>(
-        totr,
-        [&](int idx) {
-          const int p = udiv(idx, N1, a.n1m);
-          const int n = idx - p * N1;
-          const int la = 2 * (p0 + p);
-          return cpx<T>{a.real_in[(int64_t)min(la, nl1) * N1 + n],
-                        a.real_in[(int64_t)min(la + 1, nl1) * N1 + n]};
-        },
-        [&](int idx, const cpx<T>& r) {
-          const int p = udiv(idx, N1, a.n1m);
-          const int n = idx - p * N1;
-          const int la = 2 * (p0 + p), lb = la + 1;
-          const T xa = la < a.nlines ? r.x * a.scale : (T)0;
-          const T xb = lb < a.nlines ? r.y * a.scale : (T)0;
-          lds[n * ps + p] = {xa, xb};
-        });
   }
-  if (dflag) return;
-  __syncthreads();
-  // the inverse (M^T M, C2R) and the forward transform (M^T M, R2C) are turns
-  // of one loop around one copy of the FFT
-#pragma unroll 1
-  for (int turn = 0;; ++turn) {
-    line_dft<T, E, NT>(lds, a, pl, lg, ps);
-    if (MODE == MODE_R2C || turn == 1) break;
-    const int totr = N1 << lg;
-    if (MODE == MODE_MTM && (stage_mask || !a.miss) && np <= NT) {
-      // the mask in place from LDS: a thread keeps one line pair p (NT is a
-      // multiple of np), so its lines, their staged mask rows and the bit
-      // offset of sample 0 in their first word are fixed; per sample only
-      // the word and bit of o + n are formed
-      const int p = (int)threadIdx.x & (np - 1);
-      const int dn = NT >> lg;
-      const int la = 2 * (p0 + p), lb = la + 1;
-      const T sa0 = la < a.nlines ? a.scale : (T)0;
-      const T sb0 = lb < a.nlines ? a.scale : (T)0;
-      const int oa = (int)(((int64_t)la * N1) & 31), ob = (int)(((int64_t)lb * N1) & 31);
-      const uint32_t* ra = mw + (2 * p) * W;
-      const uint32_t* rb = ra + W;
-      cpx<T>* q = lds + ((int)threadIdx.x >> lg) * ps + p;
-      for (int n = (int)threadIdx.x >> lg; n < N1; n += dn, q += dn * ps) {
-        T sa = sa0, sb = sb0;
-        if (stage_mask) {
-          const int ta = oa + n, tb = ob + n;
-          if ((ra[ta >> 5] >> (ta & 31)) & 1u) sa = (T)0;
-          if ((rb[tb >> 5] >> (tb & 31)) & 1u) sb = (T)0;
+  const int tot = H1 << lg;
+  staged<NT, K, Pair<T>>(
+      tot,
+      [&](int idx) {
+        const int p = udiv(idx, H1, a.h1m);
+        const int k = idx - p * H1;
+        const int la = 2 * (p0 + p);
+        Pair<T> r;
+        r.mode = 0;
+        r.B = {(T)0, (T)0};
+        if (SRC == SRC_BUF) {
+          r.A = a.buf[(int64_t)min(la, nl1) * H1 + k];
+          r.B = a.buf[(int64_t)min(la + 1, nl1) * H1 + k];
+        } else if (SRC == SRC_U) {
+          r.A = a.u_in[u_src<D>(k, 0, 0, a.g, a.H1, r.mode)];   // 1D: a single line
+        } else {
+          r.A = spec_load<D, T, SRC>(a, k, 0, 0);
         }
-        const cpx<T> z = *q;   // (line b, line a): exchanged
-        *q = {z.y * sa, z.x * sb};
-      }
-    } else {
-    staged<NT, K, Masked<T>>(
-        totr,
-        [&](int idx) {
-          const int p = idx & (np - 1);
-          const int n = idx >> lg;
-          const int la = 2 * (p0 + p);
-          Masked<T> r;
-          r.z = cswap(lds[n * ps + p]);
-          r.wa = r.wb = 0u;
-          if (stage_mask) {
-            const int64_t sa = (int64_t)la * N1 + n, sb = sa + N1;
-            r.wa = mw[(2 * p) * W + (int)((sa >> 5) - (((int64_t)la * N1) >> 5))];
-            r.wb = mw[(2 * p + 1) * W + (int)((sb >> 5) - (((int64_t)(la + 1) * N1) >> 5))];
-          } else if (a.miss) {
-            r.wa = a.miss[((int64_t)min(la, nl1) * N1 + n) >> 5];
-            r.wb = a.miss[((int64_t)min(la + 1, nl1) * N1 + n) >> 5];
-          }
-          return r;
-        },
-        [&](int idx, const Masked<T>& r) {
-          const int p = idx & (np - 1);
-          const int n = idx >> lg;
-          const int la = 2 * (p0 + p), lb = la + 1;
-          const int64_t sa_i = (int64_t)la * N1 + n, sb_i = (int64_t)lb * N1 + n;
-          const bool ma = (r.wa >> (sa_i & 31)) & 1u;
-          const bool mb = (r.wb >> (sb_i & 31)) & 1u;
-          const T sa = (la < a.nlines && !ma) ? a.scale : (T)0;
-          const T sb = (lb < a.nlines && !mb) ? a.scale : (T)0;
-          cpx<T> z = r.z;
-          z.x *= sa;
-          z.y *= sb;
-          if (MODE == MODE_C2R) {
-            if (la < a.nlines) a.real_out[sa_i] = z.x;
-            if (lb < a.nlines) a.real_out[sb_i] = z.y;
-          } else {
-            lds[n * ps + p] = z;
-          }
-        });
-    }
-    if (MODE == MODE_C2R) return;
-    __syncthreads();
+        return r;
+      },
+      [&](int idx, const Pair<T>& r) {
+        const int p = udiv(idx, H1, a.h1m);
+        const int k = idx - p * H1;
+        const int la = 2 * (p0 + p), lb = la + 1;
+        const cpx<T> zero = {(T)0, (T)0};
+        cpx<T> A = la < a.nlines ? (SRC == SRC_U ? u_map(r.A, r.mode) : r.A) : zero;
+        cpx<T> B = (SRC == SRC_BUF && lb < a.nlines) ? r.B : zero;
+        if (k == 0 || (even && k == H1 - 1)) {  // DC / Nyquist of a real line are real
+          A.y = 0;
+          B.y = 0;
+        }
+        // A + i B and its Hermitian partner, exchanged: the transform is inverse
+        lds[k * ps + p] = {A.y + B.x, A.x - B.y};
+        if (k > 0 && N1 - k != k) lds[(N1 - k) * ps + p] = {B.x - A.y, A.x + B.y};
+      });
+  if (stage_mask) {
+#pragma unroll
+    for (int r = 0; r < kMR; ++r)
+      if ((int)threadIdx.x + r * NT < kMaskWords) mw[threadIdx.x + r * NT] = mreg[r];
   }
+}
+
+// ... from real samples
+template <typename T, int NT>
+__device__ __forceinline__ void dim1_load_real(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int N1 = a.len, H1 = a.H1;
+  const int lg = a.lg, np = 1 << lg, ps = a.ps;
+  const int p0 = tile << lg;
+  const int nl1 = a.nlines - 1;
+  constexpr int K = stage_k<T>();
+  (void)np, (void)nl1, (void)N1, (void)H1;
+  const int totr = N1 << lg;
+  staged<NT, K, cpx<T>>(
+      totr,
+      [&](int idx) {
+        const int p = udiv(idx, N1, a.n1m);
+        const int n = idx - p * N1;
+        const int la = 2 * (p0 + p);
+        return cpx<T>{a.real_in[(int64_t)min(la, nl1) * N1 + n],
+                      a.real_in[(int64_t)min(la + 1, nl1) * N1 + n]};
+      },
+      [&](int idx, const cpx<T>& r) {
+        const int p = udiv(idx, N1, a.n1m);
+        const int n = idx - p * N1;
+        const int la = 2 * (p0 + p), lb = la + 1;
+        const T xa = la < a.nlines ? r.x * a.scale : (T)0;
+        const T xb = lb < a.nlines ? r.y * a.scale : (T)0;
+        lds[n * ps + p] = {xa, xb};
+      });
+}
+
+// the samples after the inverse transform (exchanged in LDS), masked and
+// scaled: in place and unexchanged for the forward transform, or (C2R) out
+template <typename T, int NT, bool C2R>
+__device__ __forceinline__ void dim1_mask(const PassArgs<T>& a, cpx<T>* lds, const uint32_t* mw,
+                                          int tile) {
+  const int N1 = a.len, H1 = a.H1;
+  const int lg = a.lg, np = 1 << lg, ps = a.ps;
+  const int p0 = tile << lg;
+  const int nl1 = a.nlines - 1;
+  constexpr int K = stage_k<T>();
+  (void)np, (void)nl1, (void)N1, (void)H1;
+  const int W = mask_row(N1);
+  const bool stage_mask = mask_staged(a);
+  const int totr = N1 << lg;
+  if (!C2R && (stage_mask || !a.miss) && np <= NT) {
+    // the mask in place from LDS: a thread keeps one line pair p (NT is a
+    // multiple of np), so its lines, their staged mask rows and the bit
+    // offset of sample 0 in their first word are fixed; per sample only
+    // the word and bit of o + n are formed
+    const int p = (int)threadIdx.x & (np - 1);
+    const int dn = NT >> lg;
+    const int la = 2 * (p0 + p), lb = la + 1;
+    const T sa0 = la < a.nlines ? a.scale : (T)0;
+    const T sb0 = lb < a.nlines ? a.scale : (T)0;
+    const int oa = (int)(((int64_t)la * N1) & 31), ob = (int)(((int64_t)lb * N1) & 31);
+    const uint32_t* ra = mw + (2 * p) * W;
+    const uint32_t* rb = ra + W;
+    cpx<T>* q = lds + ((int)threadIdx.x >> lg) * ps + p;
+    for (int n = (int)threadIdx.x >> lg; n < N1; n += dn, q += dn * ps) {
+      T sa = sa0, sb = sb0;
+      if (stage_mask) {
+        const int ta = oa + n, tb = ob + n;
+        if ((ra[ta >> 5] >> (ta & 31)) & 1u) sa = (T)0;
+        if ((rb[tb >> 5] >> (tb & 31)) & 1u) sb = (T)0;
+      }
+      const cpx<T> z = *q;   // (line b, line a): exchanged
+      *q = {z.y * sa, z.x * sb};
+    }
+    return;
+  }
+staged<NT, K, Masked<T>>(
+    totr,
+    [&](int idx) {
+      const int p = idx & (np - 1);
+      const int n = idx >> lg;
+      const int la = 2 * (p0 + p);
+      Masked<T> r;
+      r.z = cswap(lds[n * ps + p]);
+      r.wa = r.wb = 0u;
+      if (stage_mask) {
+        const int64_t sa = (int64_t)la * N1 + n, sb = sa + N1;
+        r.wa = mw[(2 * p) * W + (int)((sa >> 5) - (((int64_t)la * N1) >> 5))];
+        r.wb = mw[(2 * p + 1) * W + (int)((sb >> 5) - (((int64_t)(la + 1) * N1) >> 5))];
+      } else if (a.miss) {
+        r.wa = a.miss[((int64_t)min(la, nl1) * N1 + n) >> 5];
+        r.wb = a.miss[((int64_t)min(la + 1, nl1) * N1 + n) >> 5];
+      }
+      return r;
+    },
+    [&](int idx, const Masked<T>& r) {
+      const int p = idx & (np - 1);
+      const int n = idx >> lg;
+      const int la = 2 * (p0 + p), lb = la + 1;
+      const int64_t sa_i = (int64_t)la * N1 + n, sb_i = (int64_t)lb * N1 + n;
+      const bool ma = (r.wa >> (sa_i & 31)) & 1u;
+      const bool mb = (r.wb >> (sb_i & 31)) & 1u;
+      const T sa = (la < a.nlines && !ma) ? a.scale : (T)0;
+      const T sb = (lb < a.nlines && !mb) ? a.scale : (T)0;
+      cpx<T> z = r.z;
+      z.x *= sa;
+      z.y *= sb;
+      if (C2R) {
+        if (la < a.nlines) a.real_out[sa_i] = z.x;
+        if (lb < a.nlines) a.real_out[sb_i] = z.y;
+      } else {
+        lds[n * ps + p] = z;
+      }
+    });
+}
+
+// the forward transform's two real lines out of the tile
+template <typename T, int NT, int D, int DST>
+__device__ __forceinline__ double dim1_store(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int N1 = a.len, H1 = a.H1;
+  const int lg = a.lg, np = 1 << lg, ps = a.ps;
+  const int p0 = tile << lg;
+  const int nl1 = a.nlines - 1;
+  constexpr int K = stage_k<T>();
+  (void)np, (void)nl1, (void)N1, (void)H1;
   double acc = 0.0;
   const int tot = H1 << lg;
   const T half = (T)0.5;
@@ -962,20 +1019,7 @@ __device__ __forceinline__ void dim1_body(const PassArgs<T>& a, int tile) {
       acc += spec_store<D, T, DST>(a, k, 0, 0, Va);   // 1D: line 0 only
     }
   }
-  if (DST != DST_BUF && a.epi.dot_part) store_partial(a.epi.dot_part, acc, tile);
-}
-
-template <typename T, int NT, int E, int D, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_dim1(PassArgs<T> a) {
-  dim1_body<T, NT, E, D, SRC, DST, MODE>(a, xcd_block());
-}
-
-template <typename T, int NT, int E, int D, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_dim1(const PassArgs<T>* __restrict__ tab, BSeg seg) {
-  const int b = xcd_block();
-  const int i = uniform(seg.inst[b]);
-  const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
-  dim1_body<T, NT, E, D, SRC, DST, MODE>(a, b - uniform(seg.first[i]));
+  return acc;
 }
 
 // ===========================================================================
@@ -991,9 +1035,6 @@ __global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_dim1(const PassA
 //         x FFT_M(w)/M = conj(bfw), inverse, twiddle)  col MID (inverse, x conj(w), mask,
 //         x w, forward, twiddle)  row CONV_FWD  col LAST (inverse, x w, epilogue)
 // ===========================================================================
-enum { C_FIRST = 0, C_REAL_IN = 1, C_MID = 2, C_LAST = 3, C_MID_C2R = 4 };
-enum { R_MTM = 0, R_C2R = 1, R_R2C = 2, R_CONV_INV = 3, R_CONV_FWD = 4 };
-
 template <typename T>
 __device__ __forceinline__ cpx<T> twf(const PassArgs<T>& a, int64_t j, bool inv) {
   cpx<T> w = a.twF[j];
@@ -1016,18 +1057,13 @@ __device__ __forceinline__ cpx<T> half_load(const PassArgs<T>& a, int64_t k) {
   return {v.x, -v.y};
 }
 
-template <typename T, int NT, int E, int SRC, int DST, int MODE>
-__device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  if (a.done && *a.done) return;
-  const int pl = plan_load(a.plan);
+// FWD: the pass's first transform is forward (else the tile holds exchanged
+// values, see line_dft)
+template <typename T, int NT, int MODE, int SRC, bool FWD>
+__device__ __forceinline__ void col_load(const PassArgs<T>& a, cpx<T>* lds, int tile) {
   const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg;
   const int64_t N = a.len;
   const bool bs = a.obs != 0;
-  // the first transform is forward or inverse (then the tile holds exchanged
-  // values, see line_dft)
-  const bool fwd1 = MODE == C_FIRST ? bs : (MODE == C_REAL_IN ? true : (MODE == C_LAST ? !bs : false));
   const int c0 = tile << lg;
   const int nv = min(nl, A - c0);
   for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
@@ -1038,7 +1074,7 @@ __device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
       if (MODE == C_FIRST) {
         if (n < N) {
           v = half_load<T, SRC>(a, n);
-          if (bs) v = cmul(v, chirp_at(a, n, true));
+          v = bs ? cmul(v, chirp_at(a, n, true)) : cswap(v);   // direct: inverse first
         }
       } else if (MODE == C_REAL_IN) {
         if (n < N) {
@@ -1046,147 +1082,253 @@ __device__ __forceinline__ void col_body(const PassArgs<T>& a, int tile) {
           if (bs) v = cmul(v, chirp_at(a, n, false));
         }
       } else {
-        v = a.buf[n];
+        v = tile_value<FWD>(a.buf[n]);
       }
     }
-    lds[r * nl + line] = fwd1 ? v : cswap(v);
+    lds[r * nl + line] = v;
   }
-  __syncthreads();
-#pragma unroll 1
-  for (int turn = 0;; ++turn) {
-    lds_fft<T, E, NT>(lds, pl, lg, nl, a.tw);
-    if ((MODE != C_MID && MODE != C_MID_C2R) || turn == 1) break;
-    // conv -> x_n = conj(w_n) conv_n, masked real part; then (MTM) x w for the forward
-    for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
-      const int line = idx & (nl - 1), r = idx >> lg;
-      const int64_t n = c0 + line + (int64_t)A * r;
-      cpx<T>* q = lds + r * nl + line;
-      T xr = (T)0;
-      if (line < nv && n < N && !miss_bit(a.miss, n)) xr = cmul(cswap(*q), chirp_at(a, n, true)).x * a.scale;
-      if (MODE == C_MID_C2R) {
-        if (line < nv && n < N) a.real_out[n] = xr;
-      } else {
-        const cpx<T> w = n < N ? chirp_at(a, n, false) : cpx<T>{(T)0, (T)0};
-        *q = {xr * w.x, xr * w.y};
-      }
+}
+
+// outer Bluestein, between the convolutions (exchanged values in LDS):
+// conv -> x_n = conj(w_n) conv_n, masked real part; then x w for the forward
+// transform, or (C2R) out
+template <typename T, int NT, bool C2R>
+__device__ __forceinline__ void col_mid(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg;
+  const int64_t N = a.len;
+  const int c0 = tile << lg;
+  const int nv = min(nl, A - c0);
+  for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
+    const int line = idx & (nl - 1), r = idx >> lg;
+    const int64_t n = c0 + line + (int64_t)A * r;
+    cpx<T>* q = lds + r * nl + line;
+    T xr = (T)0;
+    if (line < nv && n < N && !miss_bit(a.miss, n))
+      xr = cmul(cswap(*q), chirp_at(a, n, true)).x * a.scale;
+    if (C2R) {
+      if (line < nv && n < N) a.real_out[n] = xr;
+    } else {
+      const cpx<T> w = n < N ? chirp_at(a, n, false) : cpx<T>{(T)0, (T)0};
+      *q = {xr * w.x, xr * w.y};
     }
-    if (MODE == C_MID_C2R) return;
-    __syncthreads();
   }
-  const bool exchanged = MODE != C_MID && !fwd1;   // the last transform was inverse
+}
+
+// FWD: the pass's last transform was forward.  Into the scratch spectrum (with
+// the four-step twiddle: conjugate after an inverse transform) or, the last
+// pass, into beta / u
+template <typename T, int NT, int DST, bool FWD>
+__device__ __forceinline__ double col_store(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg;
+  const bool bs = a.obs != 0;
+  const int c0 = tile << lg;
+  const int nv = min(nl, A - c0);
   double acc = 0.0;
   for (int idx = threadIdx.x; idx < (B << lg); idx += NT) {
     const int line = idx & (nl - 1), r = idx >> lg;
     if (line >= nv) continue;
     const int col = c0 + line;
-    cpx<T> v = lds[r * nl + line];
-    if (exchanged) v = cswap(v);
-    if (MODE != C_LAST) {
-      const bool inv = MODE == C_FIRST && !bs;
-      v = cmul(v, twf(a, (int64_t)col * r, inv));
+    cpx<T> v = tile_value<FWD>(lds[r * nl + line]);
+    if (DST == DST_BUF) {
+      v = cmul(v, twf(a, (int64_t)col * r, !FWD));
       a.buf[col + (int64_t)A * r] = v;
     } else {
       const int64_t k = col + (int64_t)A * r;
       if (k < a.H1) {
-        if (bs) v = cmul(v, chirp_at(a, k, false));
+        if (bs) v = cmul(cswap(v), chirp_at(a, k, false));   // ends in the inverse transform
         acc += spec_store<1, T, DST>(a, (int)k, 0, 0, v);
       }
     }
   }
-  if (MODE == C_LAST && a.epi.dot_part) store_partial(a.epi.dot_part, acc, tile);
+  return acc;
 }
 
-template <typename T, int NT, int E, int MODE>
-__device__ __forceinline__ void row_body(const PassArgs<T>& a, int tile) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  if (a.done && *a.done) return;
-  const int pl = plan_load(a.plan);
-  constexpr bool fwd1 = MODE == R_R2C || MODE == R_CONV_INV || MODE == R_CONV_FWD;
+template <typename T, int NT, bool REAL, bool FWD>
+__device__ __forceinline__ void row_load(const PassArgs<T>& a, cpx<T>* lds, int tile) {
   const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg, ps = a.ps;
   const int r0 = tile << lg;
   const int nv = min(nl, B - r0);
-  const int tot = A << lg;
-  for (int idx = threadIdx.x; idx < tot; idx += NT) {
+  for (int idx = threadIdx.x; idx < (A << lg); idx += NT) {
     const int line = udiv(idx, A, a.am);
     const int c = idx - line * A;
     const int row = r0 + line;
     cpx<T> v = {(T)0, (T)0};
     if (line < nv) {
-      if (MODE == R_R2C) v = {a.real_in[row + (int64_t)B * c] * a.scale, (T)0};
+      if (REAL) v = {a.real_in[row + (int64_t)B * c] * a.scale, (T)0};
       else v = a.buf[c + (int64_t)A * row];
     }
-    lds[c * ps + line] = fwd1 ? v : cswap(v);
+    lds[c * ps + line] = tile_value<FWD>(v);
   }
-  __syncthreads();
-#pragma unroll 1
-  for (int turn = 0;; ++turn) {
-    lds_fft<T, E, NT>(lds, pl, lg, ps, a.tw);
-    if (MODE == R_R2C || turn == 1) break;
-    if (MODE == R_MTM || MODE == R_C2R) {
-      for (int idx = threadIdx.x; idx < tot; idx += NT) {
-        const int line = udiv(idx, A, a.am);
-        const int c = idx - line * A;
-        const int64_t t = r0 + line + (int64_t)B * c;
-        cpx<T>* q = lds + c * ps + line;
-        const T xr = (line < nv && !miss_bit(a.miss, t)) ? q->y * a.scale : (T)0;   // exchanged
-        if (MODE == R_C2R) {
-          if (line < nv) a.real_out[t] = xr;
-        } else {
-          *q = {xr, (T)0};
-        }
-      }
-      if (MODE == R_C2R) return;
+}
+
+// direct: the samples after the inverse transform (exchanged), masked
+template <typename T, int NT, bool C2R>
+__device__ __forceinline__ void row_mask(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg, ps = a.ps;
+  const int r0 = tile << lg;
+  const int nv = min(nl, B - r0);
+  for (int idx = threadIdx.x; idx < (A << lg); idx += NT) {
+    const int line = udiv(idx, A, a.am);
+    const int c = idx - line * A;
+    const int64_t t = r0 + line + (int64_t)B * c;
+    cpx<T>* q = lds + c * ps + line;
+    const T xr = (line < nv && !miss_bit(a.miss, t)) ? q->y * a.scale : (T)0;
+    if (C2R) {
+      if (line < nv) a.real_out[t] = xr;
     } else {
-      for (int idx = threadIdx.x; idx < tot; idx += NT) {
-        const int line = udiv(idx, A, a.am);
-        const int c = idx - line * A;
-        cpx<T>* q = lds + c * ps + line;
-        // the product with the kernel spectrum, exchanged for the inverse FFT
-        // (the inverse kernel is the conjugate of the forward one, and both
-        // are even, so its spectrum is the conjugate too)
-        if (line < nv) {
-          cpx<T> bk = a.bfw[r0 + line + (int64_t)B * c];
-          if (MODE == R_CONV_INV) bk.y = -bk.y;
-          *q = cswap(cmul(*q, bk));
-        }
-      }
+      *q = {xr, (T)0};
     }
-    __syncthreads();
   }
-  constexpr bool inv_tw = MODE == R_CONV_INV || MODE == R_CONV_FWD;
-  for (int idx = threadIdx.x; idx < tot; idx += NT) {
+}
+
+// the product with the kernel spectrum, exchanged for the inverse FFT (the
+// inverse kernel is the conjugate of the forward one, and both are even, so
+// its spectrum is the conjugate too)
+template <typename T, int NT, bool INV>
+__device__ __forceinline__ void row_conv(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg, ps = a.ps;
+  const int r0 = tile << lg;
+  const int nv = min(nl, B - r0);
+  for (int idx = threadIdx.x; idx < (A << lg); idx += NT) {
+    const int line = udiv(idx, A, a.am);
+    const int c = idx - line * A;
+    cpx<T>* q = lds + c * ps + line;
+    if (line < nv) {
+      cpx<T> bk = a.bfw[r0 + line + (int64_t)B * c];
+      if (INV) bk.y = -bk.y;
+      *q = cswap(cmul(*q, bk));
+    }
+  }
+}
+
+// FWD as in col_store
+template <typename T, int NT, bool FWD>
+__device__ __forceinline__ void row_store(const PassArgs<T>& a, cpx<T>* lds, int tile) {
+  const int A = a.A, B = a.B, lg = a.lg, nl = 1 << lg, ps = a.ps;
+  const int r0 = tile << lg;
+  const int nv = min(nl, B - r0);
+  for (int idx = threadIdx.x; idx < (A << lg); idx += NT) {
     const int line = udiv(idx, A, a.am);
     const int c = idx - line * A;
     if (line >= nv) continue;
     const int row = r0 + line;
-    // (the second transform of a convolution is inverse)
-    const cpx<T> v = inv_tw ? cswap(lds[c * ps + line]) : lds[c * ps + line];
-    a.buf[c + (int64_t)A * row] = cmul(v, twf(a, (int64_t)row * c, inv_tw));
+    const cpx<T> v = tile_value<FWD>(lds[c * ps + line]);
+    a.buf[c + (int64_t)A * row] = cmul(v, twf(a, (int64_t)row * c, !FWD));
   }
 }
 
-template <typename T, int NT, int E, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_col(PassArgs<T> a) {
-  col_body<T, NT, E, SRC, DST, MODE>(a, xcd_block());
+// one workgroup's tile of a pass; LD, MID, ST < 0: the steps PassArgs names
+template <typename T, int NT, int E, int LD, int MID, int ST>
+__device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
+  const int ld = LD < 0 ? a.ld : LD, mid = MID < 0 ? a.mid : MID, st = ST < 0 ? a.st : ST;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
+  __shared__ uint32_t mw[kMaskWords];
+  // finished instances: the flag is read beside the loads, not before them
+  const int dflag = a.done ? *a.done : 0;
+  const int pl = plan_load(a.plan);
+  constexpr bool kShort = NT * E <= 4096;   // line, column and row tiles
+  switch (ld) {
+    case LD_DIM1_BUF: dim1_load<T, NT, 2, SRC_BUF>(a, lds, mw, tile); break;
+    case LD_DIM1_U: dim1_load<T, NT, 1, SRC_U>(a, lds, mw, tile); break;
+    case LD_DIM1_BETA: dim1_load<T, NT, 1, SRC_BETA>(a, lds, mw, tile); break;
+    case LD_DIM1_REAL: dim1_load_real<T, NT>(a, lds, tile); break;
+    default:
+      if constexpr (kShort) {
+        switch (ld) {
+          case LD_LINES_BUF_FWD: lines_load<T, NT, 3, SRC_BUF, true>(a, lds, tile); break;
+          case LD_LINES_BUF_INV: lines_load<T, NT, 3, SRC_BUF, false>(a, lds, tile); break;
+          case LD_LINES_U2: lines_load<T, NT, 2, SRC_U, false>(a, lds, tile); break;
+          case LD_LINES_U3: lines_load<T, NT, 3, SRC_U, false>(a, lds, tile); break;
+          case LD_LINES_BETA2: lines_load<T, NT, 2, SRC_BETA, false>(a, lds, tile); break;
+          case LD_LINES_BETA3: lines_load<T, NT, 3, SRC_BETA, false>(a, lds, tile); break;
+          case LD_COL_FIRST_U: col_load<T, NT, C_FIRST, SRC_U, false>(a, lds, tile); break;
+          case LD_COL_FIRST_BETA: col_load<T, NT, C_FIRST, SRC_BETA, false>(a, lds, tile); break;
+          case LD_COL_REAL: col_load<T, NT, C_REAL_IN, SRC_REAL, true>(a, lds, tile); break;
+          case LD_COL_BUF_FWD: col_load<T, NT, C_LAST, SRC_BUF, true>(a, lds, tile); break;
+          case LD_COL_BUF_INV: col_load<T, NT, C_LAST, SRC_BUF, false>(a, lds, tile); break;
+          case LD_ROW_FWD: row_load<T, NT, false, true>(a, lds, tile); break;
+          case LD_ROW_INV: row_load<T, NT, false, false>(a, lds, tile); break;
+          case LD_ROW_REAL: row_load<T, NT, true, true>(a, lds, tile); break;
+          default: break;
+        }
+      }
+  }
+  if (dflag) return;
+  __syncthreads();
+#pragma unroll 1
+  for (int turn = 0;; ++turn) {
+    if constexpr (LD >= LD_COL_FIRST_U)   // four-step passes transform directly
+      lds_fft<T, E, NT>(lds, pl, a.lg, a.ps, a.tw);
+    else
+      line_dft<T, E, NT>(lds, a, pl, a.lg, a.ps);
+    if (turn == 1 || mid == MID_NONE) break;
+    switch (mid) {
+      case MID_DIM1_MASK: dim1_mask<T, NT, false>(a, lds, mw, tile); break;
+      default:
+        if constexpr (kShort) {
+          switch (mid) {
+            case MID_COL: col_mid<T, NT, false>(a, lds, tile); break;
+            case MID_ROW_MASK: row_mask<T, NT, false>(a, lds, tile); break;
+            case MID_ROW_CONV_INV: row_conv<T, NT, true>(a, lds, tile); break;
+            case MID_ROW_CONV_FWD: row_conv<T, NT, false>(a, lds, tile); break;
+            default: break;
+          }
+        }
+    }
+    __syncthreads();
+  }
+  double acc = 0.0;
+  switch (st) {
+    case ST_DIM1_BUF: dim1_store<T, NT, 2, DST_BUF>(a, lds, tile); return;
+    case ST_DIM1_REAL: dim1_mask<T, NT, true>(a, lds, mw, tile); return;
+    case ST_DIM1_U: acc = dim1_store<T, NT, 1, DST_U>(a, lds, tile); break;
+    case ST_DIM1_BETA: acc = dim1_store<T, NT, 1, DST_BETA>(a, lds, tile); break;
+    default:
+      if constexpr (kShort) {
+        switch (st) {
+          case ST_LINES_BUF_FWD: lines_store<T, NT, 3, DST_BUF, true>(a, lds, tile); return;
+          case ST_LINES_BUF_INV: lines_store<T, NT, 3, DST_BUF, false>(a, lds, tile); return;
+          case ST_LINES_U2: acc = lines_store<T, NT, 2, DST_U, true>(a, lds, tile); break;
+          case ST_LINES_U3: acc = lines_store<T, NT, 3, DST_U, true>(a, lds, tile); break;
+          case ST_LINES_BETA2: acc = lines_store<T, NT, 2, DST_BETA, true>(a, lds, tile); break;
+          case ST_LINES_BETA3: acc = lines_store<T, NT, 3, DST_BETA, true>(a, lds, tile); break;
+          case ST_COL_BUF_FWD: col_store<T, NT, DST_BUF, true>(a, lds, tile); return;
+          case ST_COL_BUF_INV: col_store<T, NT, DST_BUF, false>(a, lds, tile); return;
+          case ST_COL_U: acc = col_store<T, NT, DST_U, true>(a, lds, tile); break;
+          case ST_COL_BETA: acc = col_store<T, NT, DST_BETA, true>(a, lds, tile); break;
+          case ST_COL_REAL: col_mid<T, NT, true>(a, lds, tile); return;
+          case ST_ROW_FWD: row_store<T, NT, true>(a, lds, tile); return;
+          case ST_ROW_INV: row_store<T, NT, false>(a, lds, tile); return;
+          case ST_ROW_REAL: row_mask<T, NT, true>(a, lds, tile); return;
+          default: break;
+        }
+      }
+  }
+  if (a.epi.dot_part) store_partial(a.epi.dot_part, acc, tile);
 }
-template <typename T, int NT, int E, int SRC, int DST, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_col(const PassArgs<T>* __restrict__ tab, BSeg seg) {
-  const int b = xcd_block();
-  const int i = uniform(seg.inst[b]);
+
+// a pass of one instance
+template <typename T, int NT, int E, int LD, int MID, int ST>
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_pass(PassArgs<T> a) {
+  pass_body<T, NT, E, LD, MID, ST>(a, xcd_block());
+}
+
+// member and tile of a block of a launch over several instances; member < 0:
+// a filler
+struct BlockMap {
+  int member, tile;
+};
+
+// passes of several instances (LD < 0: each its own kind): the host's block map keeps
+// adjacent tiles of an instance on one XCD (block b runs on XCD b % 8)
+template <typename T, int NT, int E, int LD, int MID, int ST>
+__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_pass(
+    const PassArgs<T>* __restrict__ tab, const BlockMap* __restrict__ map) {
+  const int i = uniform(map[blockIdx.x].member), tile = uniform(map[blockIdx.x].tile);
+  if (i < 0) return;
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
-  col_body<T, NT, E, SRC, DST, MODE>(a, b - uniform(seg.first[i]));
-}
-template <typename T, int NT, int E, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_row(PassArgs<T> a) {
-  row_body<T, NT, E, MODE>(a, xcd_block());
-}
-template <typename T, int NT, int E, int MODE>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_row(const PassArgs<T>* __restrict__ tab, BSeg seg) {
-  const int b = xcd_block();
-  const int i = uniform(seg.inst[b]);
-  const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
-  row_body<T, NT, E, MODE>(a, b - uniform(seg.first[i]));
+  pass_body<T, NT, E, LD, MID, ST>(a, tile);
 }
 
 // beta <-> u (exact: a signed permutation), one thread per half-spectrum element.

@@ -2,12 +2,12 @@
 instantiate them.
 
 The pass kernels (csipm_kernels.hpp) are templates over the precision, the
-workgroup size, the spectrum dimensionality and the source / destination /
-mode of a pass; every combination the host code launches is listed here.
+workgroup size and the steps of a pass; every combination the host code launches is listed here.
 `write(outdir, nunits)` writes
 
   fft_extern.inc      explicit instantiation declarations, included by
                       csipm.hip so that its own compilation skips them, and
+                      the combinations as X-macros for its dispatch, and
   fft_inst_<k>.hip    nunits translation units holding the definitions,
 
 so that the kernels compile in parallel.  A combination missing from the
@@ -18,54 +18,66 @@ from __future__ import annotations
 
 import os
 
-# kernel -> template arguments after the precision
-_LINES = ["2 0 3 true", "2 3 0 false", "3 0 0 false", "3 0 0 true", "3 0 3 true", "3 3 0 false"]
-_LINES_BETA = ["2 0 1 true", "2 1 0 false", "3 0 1 true", "3 1 0 false"]
-_COL = ["0 0 2", "0 3 3", "2 0 1", "3 0 0"]
-_COL_BETA = ["0 1 3", "0 2 4", "1 0 0"]
-_ROW = ["0", "2", "3", "4"]
-_DIM1 = ["1 2 3 2", "1 3 3 0", "2 0 0 0", "2 2 0 2", "3 0 0 0", "3 2 0 2"]
-_DIM1_BETA = ["1 1 1 0", "1 1 2 1", "1 2 1 2", "2 0 2 1", "3 0 2 1"]
+# the steps (load, middle, store) of the passes: of the batched chains, on the
+# spectrum order, and of the entry points besides
+CHAIN_SHORT = [
+    "LD_LINES_U2 MID_NONE ST_LINES_BUF_INV", "LD_LINES_U3 MID_NONE ST_LINES_BUF_INV",
+    "LD_LINES_BUF_INV MID_NONE ST_LINES_BUF_INV", "LD_LINES_BUF_FWD MID_NONE ST_LINES_BUF_FWD",
+    "LD_LINES_BUF_FWD MID_NONE ST_LINES_U2", "LD_LINES_BUF_FWD MID_NONE ST_LINES_U3",
+    "LD_COL_FIRST_U MID_NONE ST_COL_BUF_INV", "LD_COL_FIRST_U MID_NONE ST_COL_BUF_FWD",
+    "LD_COL_REAL MID_NONE ST_COL_BUF_FWD", "LD_COL_BUF_INV MID_COL ST_COL_BUF_FWD",
+    "LD_COL_BUF_FWD MID_NONE ST_COL_U", "LD_COL_BUF_INV MID_NONE ST_COL_U",
+    "LD_ROW_INV MID_ROW_MASK ST_ROW_FWD", "LD_ROW_REAL MID_NONE ST_ROW_FWD",
+    "LD_ROW_FWD MID_ROW_CONV_INV ST_ROW_INV", "LD_ROW_FWD MID_ROW_CONV_FWD ST_ROW_INV",
+]
+CHAIN_DIM1 = [
+    "LD_DIM1_U MID_DIM1_MASK ST_DIM1_U", "LD_DIM1_BUF MID_DIM1_MASK ST_DIM1_BUF",
+    "LD_DIM1_REAL MID_NONE ST_DIM1_U", "LD_DIM1_REAL MID_NONE ST_DIM1_BUF",
+]
+ENTRY_SHORT = [
+    "LD_LINES_BETA2 MID_NONE ST_LINES_BUF_INV", "LD_LINES_BETA3 MID_NONE ST_LINES_BUF_INV",
+    "LD_LINES_BUF_FWD MID_NONE ST_LINES_BETA2", "LD_LINES_BUF_FWD MID_NONE ST_LINES_BETA3",
+    "LD_COL_FIRST_BETA MID_NONE ST_COL_BUF_INV", "LD_COL_FIRST_BETA MID_NONE ST_COL_BUF_FWD",
+    "LD_COL_BUF_INV MID_NONE ST_COL_REAL", "LD_COL_BUF_FWD MID_NONE ST_COL_BETA",
+    "LD_COL_BUF_INV MID_NONE ST_COL_BETA", "LD_ROW_INV MID_NONE ST_ROW_REAL",
+]
+ENTRY_DIM1 = [
+    "LD_DIM1_BETA MID_DIM1_MASK ST_DIM1_BETA", "LD_DIM1_BETA MID_NONE ST_DIM1_REAL",
+    "LD_DIM1_BUF MID_NONE ST_DIM1_REAL", "LD_DIM1_REAL MID_NONE ST_DIM1_BETA",
+]
 # workgroup sizes with the elements per thread: of tiles up to 4096 elements,
-# and of the dimension-1 passes with longer lines
-_NT = ["256 8", "512 8"]
-_NT_DIM1 = _NT + ["1024 8", "1024 16"]
-
-
-def _rows(nts, rows):
-    return [f"{nt} {r}" for nt in nts for r in rows]
-
-
-TABLE = {
-    "k_col": _rows(_NT, _COL + _COL_BETA),
-    "k_row": _rows(_NT, _ROW + ["1"]),
-    "k_lines": _rows(_NT, _LINES + _LINES_BETA),
-    "k_dim1": _rows(_NT_DIM1, _DIM1[1:] + _DIM1_BETA),
-    "kb_col": _rows(_NT, _COL),
-    "kb_row": _rows(_NT, _ROW),
-    "kb_lines": _rows(_NT, _LINES),
-    "kb_dim1": _rows(_NT_DIM1, _DIM1),
-}
-
-
-def _params(kernel, t):
-    return f"const PassArgs<{t}>*, BSeg" if kernel.startswith("kb_") else f"PassArgs<{t}>"
+# and of longer lines (dimension 1 only)
+NT_SHORT = ["256 8", "512 8"]
+NT_LONG = ["1024 8", "1024 16"]
+MIXED = "-1 -1 -1"
 
 
 def instances():
+    def rows(nts, steps):
+        return [f"{n} {s}" for n in nts for s in steps]
+    table = {
+        "k_pass": rows(NT_SHORT + NT_LONG, CHAIN_DIM1 + ENTRY_DIM1) +
+        rows(NT_SHORT, CHAIN_SHORT + ENTRY_SHORT),
+        "kb_pass": rows(NT_SHORT + NT_LONG, CHAIN_DIM1 + [MIXED]) + rows(NT_SHORT, CHAIN_SHORT),
+    }
     out = []
     for t in ("float", "double"):
-        for k, rows in TABLE.items():
-            for r in rows:
-                args = ", ".join([t] + r.split())
-                out.append(f"void {k}<{args}>({_params(k, t)})")
+        for k, rs in table.items():
+            p = f"PassArgs<{t}>" if k == "k_pass" else f"const PassArgs<{t}>*, const BlockMap*"
+            out += [f"void {k}<{', '.join([t] + r.split())}>({p})" for r in rs]
     return out
 
 
 def write(outdir, nunits):
     os.makedirs(outdir, exist_ok=True)
     inst = instances()
-    ext = ["// generated by fft_instances.py", "namespace csipm {"]
+    ext = ["// generated by fft_instances.py"]
+    # the steps as X-macros, for the host's dispatch
+    for name, steps in (("CHAIN_SHORT", CHAIN_SHORT), ("CHAIN_DIM1", CHAIN_DIM1),
+                        ("ENTRY_SHORT", ENTRY_SHORT), ("ENTRY_DIM1", ENTRY_DIM1)):
+        ext += [f"#define CSIPM_{name}(X) " +
+                " ".join("X(" + ", ".join(s.split()) + ")" for s in steps)]
+    ext += ["namespace csipm {"]
     ext += [f"extern template __global__ {s};" for s in inst]
     ext += ["}  // namespace csipm", ""]
     _put(os.path.join(outdir, "fft_extern.inc"), "\n".join(ext))
