@@ -219,6 +219,54 @@ __host__ __device__ __forceinline__ bool scatter_targets(int k1, int k2, int k3,
   return true;
 }
 
+// The same for the interior of dimension 1 (1 <= k1 <= P1, D >= 2), a row
+// (k2, k3) at a time: every such element reads / feeds two beta entries, at
+//   re + s * k1  and  d further,
+// with the imaginary part negated when neg (the mirror blocks, where k1 runs
+// backwards).  32-bit arithmetic: beta has at most 2^31 entries.
+struct BetaRow {
+  uint32_t re, d;
+  int s;
+  bool neg;
+};
+
+template <int D>
+__host__ __device__ __forceinline__ BetaRow beta_row(int k2, int k3, const MapGeom& g) {
+  const uint32_t P1 = (uint32_t)g.P[0], P2 = (uint32_t)g.P[1];
+  const Cat c2 = cat_of(k2, g, 1);
+  uint32_t v2 = (uint32_t)c2.v;
+  if (D == 2) {
+    if (c2.c == 0) return {(uint32_t)g.off[2] + 2u * v2 * P1 - 1u, P1, 1, false};
+    return {(uint32_t)g.off[3] + (c2.c == 2 ? 2u * (uint32_t)g.P12 : 0u) + P1 * v2 - 1u,
+            (uint32_t)g.P12, 1, false};
+  }
+  const uint32_t P3 = (uint32_t)g.P[2];
+  const Cat c3 = cat_of(k3, g, 2);
+  uint32_t v3 = (uint32_t)c3.v;
+  const bool neg = c3.c == 2 || (c3.c == 0 && c2.c == 2);
+  // the class of the representative (the mirror element's when neg)
+  const bool h2 = neg ? c2.c == 1 : c2.c == 2;   // dimension 2 in its second half
+  if (neg && c2.c != 0) v2 = P2 - 1u - v2;
+  if (neg && c3.c != 0) v3 = P3 - 1u - v3;
+  uint32_t base, d;
+  if (c2.c == 0 && c3.c == 0) {
+    d = P1;
+    base = (uint32_t)g.off[3] + 2u * (v2 * (uint32_t)g.S[2] + v3) * P1;
+  } else if (c2.c == 0) {
+    d = (uint32_t)g.P13;
+    base = (uint32_t)g.off[5] + (4u * v2 + (neg ? 2u : 0u)) * d + P1 * v3;
+  } else if (c3.c == 0) {
+    d = (uint32_t)g.P12;
+    base = (uint32_t)g.off[6] + (4u * v3 + (neg ? 2u : 0u)) * d + P1 * v2;
+  } else {
+    d = (uint32_t)g.P123;
+    base = (uint32_t)g.off[7] + 2u * ((neg ? 1u : 0u) + (h2 ? 2u : 0u)) * d + P1 * (v2 + P2 * v3);
+  }
+  // k1 - 1 forwards, P1 - 1 - (k1 - 1) backwards
+  if (neg) return {base + P1, d, -1, true};
+  return {base - 1u, d, 1, false};
+}
+
 // ---------------------------------------------------------------------------
 // Radix-R DFT butterflies on registers, forward: exp(-2 pi i jk/R).  There is
 // no inverse form: inverse = swap . forward . swap with swap exchanging real
@@ -636,6 +684,15 @@ __host__ __device__ __forceinline__ cpx<T> u_map(cpx<T> w, int mode) {
   const T x = w.x / sq2, y = w.y / sq2;
   if (mode == 1) return {w.x, (T)0};
   return {x, mode == 2 ? -y : y};
+}
+
+// u_map on the way into a pass, with one multiplication instead of the
+// division (as exact: the constant and the product are rounded once each)
+template <typename T>
+__device__ __forceinline__ cpx<T> u_scale(cpx<T> w, int mode) {
+  const T h = (T)0.70710678118654752440;
+  if (mode == 1) return {w.x, (T)0};
+  return {w.x * h, mode == 2 ? -(w.y * h) : w.y * h};
 }
 
 // sqrt2 * v, v_to_u of a representative element (kept apart from any

@@ -190,75 +190,6 @@ struct Epi {
   double* dot_part;     // per-block partial sums of x'y (CG p'q), or null
 };
 
-// writes value m of beta index i; returns its contribution to x'y
-template <typename T>
-__device__ __forceinline__ double epi_apply(const Epi<T>& e, int64_t i, T m) {
-  if (e.kind == 0) {
-    e.out[i] = m;
-    return 0.0;
-  }
-  if (e.kind == 2) {
-    if (e.out) e.out[i] = m;
-    const T xb = e.xb[i];
-    T qb = e.alpha * (m + e.L1[i] * xb);
-    if (e.beta != (T)0) qb += e.beta * e.yb[i];
-    e.yb[i] = qb;
-    return (double)xb * (double)qb;
-  }
-  const T xb = e.xb[i], xz = e.xz[i], l1 = e.L1[i], l2 = e.L2[i];
-  T qb = e.alpha * (m + l1 * xb + l2 * xz);
-  T qz = e.alpha * (l2 * xb + l1 * xz);
-  if (e.beta != (T)0) {
-    qb += e.beta * e.yb[i];
-    qz += e.beta * e.yz[i];
-  }
-  e.yb[i] = qb;
-  e.yz[i] = qz;
-  return (double)xb * (double)qb + (double)xz * (double)qz;
-}
-
-// the same on the two slots (re, im) of u-space element e, as one vector access
-template <typename T>
-__device__ __forceinline__ double epi_apply_u(const Epi<T>& e, int64_t el, cpx<T> m) {
-  if (e.kind == 0) {
-    reinterpret_cast<cpx<T>*>(e.out)[el] = m;
-    return 0.0;
-  }
-  if (e.kind == 2) {
-    if (e.out) reinterpret_cast<cpx<T>*>(e.out)[el] = m;
-    const cpx<T> xb = reinterpret_cast<const cpx<T>*>(e.xb)[el];
-    const cpx<T> dg = reinterpret_cast<const cpx<T>*>(e.L1)[el];
-    cpx<T> qb = {e.alpha * (m.x + dg.x * xb.x), e.alpha * (m.y + dg.y * xb.y)};
-    cpx<T>* yb = reinterpret_cast<cpx<T>*>(e.yb);
-    if (e.beta != (T)0) {
-      const cpx<T> ob = yb[el];
-      qb.x += e.beta * ob.x;
-      qb.y += e.beta * ob.y;
-    }
-    yb[el] = qb;
-    return (double)xb.x * qb.x + (double)xb.y * qb.y;
-  }
-  const cpx<T> xb = reinterpret_cast<const cpx<T>*>(e.xb)[el];
-  const cpx<T> xz = reinterpret_cast<const cpx<T>*>(e.xz)[el];
-  const cpx<T> l1 = reinterpret_cast<const cpx<T>*>(e.L1)[el];
-  const cpx<T> l2 = reinterpret_cast<const cpx<T>*>(e.L2)[el];
-  cpx<T> qb = {e.alpha * (m.x + l1.x * xb.x + l2.x * xz.x),
-               e.alpha * (m.y + l1.y * xb.y + l2.y * xz.y)};
-  cpx<T> qz = {e.alpha * (l2.x * xb.x + l1.x * xz.x), e.alpha * (l2.y * xb.y + l1.y * xz.y)};
-  cpx<T>* yb = reinterpret_cast<cpx<T>*>(e.yb);
-  cpx<T>* yz = reinterpret_cast<cpx<T>*>(e.yz);
-  if (e.beta != (T)0) {
-    const cpx<T> ob = yb[el], oz = yz[el];
-    qb.x += e.beta * ob.x;
-    qb.y += e.beta * ob.y;
-    qz.x += e.beta * oz.x;
-    qz.y += e.beta * oz.y;
-  }
-  yb[el] = qb;
-  yz[el] = qz;
-  return (double)xb.x * qb.x + (double)xb.y * qb.y + (double)xz.x * qz.x + (double)xz.y * qz.y;
-}
-
 // The epilogue of a u-space element in two steps, so that a thread can issue
 // the operand loads of several elements before it consumes any of them:
 // epi_fetch_u loads what kind `e.kind` reads (always in range for el < U),
@@ -284,7 +215,6 @@ __device__ __forceinline__ EpiOps<T> epi_fetch_u(const Epi<T>& e, int64_t el) {
   return o;
 }
 
-// the arithmetic of epi_apply_u, on fetched operands
 template <typename T>
 __device__ __forceinline__ double epi_commit_u(const Epi<T>& e, int64_t el, cpx<T> m,
                                                const EpiOps<T>& o) {
@@ -344,17 +274,92 @@ __device__ __forceinline__ void staged(int total, F&& fetch, P&& put) {
   }
 }
 
-// value v of half-spectrum element (k1,k2,k3) -> the beta entries reading it
+// The same for the beta entries an element of the half spectrum feeds (none
+// of them: an element that beta does not hold).
+template <typename T>
+struct BetaOps {
+  EpiOps<T> o;        // operands of the real-part entry (.x) and the other (.y)
+  uint32_t re, im;
+  bool hit, vertex, neg;
+};
+
+// interior: 1 <= k1 <= P1 and D >= 2
 template <int D, typename T>
-__device__ __forceinline__ double scatter_elem(const Epi<T>& e, int k1, int k2, int k3,
-                                               cpx<T> v, const MapGeom& g) {
-  int64_t re, im;
-  bool vertex, neg;
-  if (!scatter_targets<D>(k1, k2, k3, g, re, im, vertex, neg)) return 0.0;
+__device__ __forceinline__ BetaOps<T> epi_fetch_beta(const Epi<T>& e, int k1, int k2, int k3,
+                                                     const MapGeom& g, bool interior) {
+  BetaOps<T> r;
+  r.hit = true;
+  r.vertex = false;
+  if (D >= 2 && interior) {
+    const BetaRow w = beta_row<D>(k2, k3, g);
+    r.re = w.re + (uint32_t)(w.s * k1);
+    r.im = r.re + w.d;
+    r.neg = w.neg;
+  } else {
+    int64_t re, im;
+    r.hit = scatter_targets<D>(k1, k2, k3, g, re, im, r.vertex, r.neg);
+    r.re = r.hit ? (uint32_t)re : 0u;
+    r.im = r.hit && !r.vertex ? (uint32_t)im : r.re;
+  }
+  const cpx<T> z = {(T)0, (T)0};
+  r.o.xb = r.o.xz = r.o.l1 = r.o.l2 = r.o.ob = r.o.oz = z;
+  if (e.kind == 0) return r;
+  r.o.xb = {e.xb[r.re], e.xb[r.im]};
+  r.o.l1 = {e.L1[r.re], e.L1[r.im]};
+  if (e.beta != (T)0) r.o.ob = {e.yb[r.re], e.yb[r.im]};
+  if (e.kind == 2) return r;
+  r.o.xz = {e.xz[r.re], e.xz[r.im]};
+  r.o.l2 = {e.L2[r.re], e.L2[r.im]};
+  if (e.beta != (T)0) r.o.oz = {e.yz[r.re], e.yz[r.im]};
+  return r;
+}
+
+// v: the spectrum value
+template <typename T>
+__device__ __forceinline__ double epi_commit_beta(const Epi<T>& e, cpx<T> v, const BetaOps<T>& r) {
+  if (!r.hit) return 0.0;
   const T sq2 = (T)1.4142135623730951;
-  if (vertex) return epi_apply(e, re, v.x);
-  double acc = epi_apply(e, re, sq2 * v.x);
-  acc += epi_apply(e, im, (neg ? -sq2 : sq2) * v.y);
+  const EpiOps<T>& o = r.o;
+  cpx<T> m = {sq2 * v.x, sq2 * v.y};
+  if (r.neg) m.y = -m.y;
+  if (r.vertex) m.x = v.x;
+  if (e.kind == 0) {
+    e.out[r.re] = m.x;
+    if (!r.vertex) e.out[r.im] = m.y;
+    return 0.0;
+  }
+  if (e.kind == 2) {
+    if (e.out) {
+      e.out[r.re] = m.x;
+      if (!r.vertex) e.out[r.im] = m.y;
+    }
+    cpx<T> qb = {e.alpha * (m.x + o.l1.x * o.xb.x), e.alpha * (m.y + o.l1.y * o.xb.y)};
+    if (e.beta != (T)0) {
+      qb.x += e.beta * o.ob.x;
+      qb.y += e.beta * o.ob.y;
+    }
+    e.yb[r.re] = qb.x;
+    if (!r.vertex) e.yb[r.im] = qb.y;
+    return (double)o.xb.x * qb.x + (r.vertex ? 0.0 : (double)o.xb.y * qb.y);
+  }
+  cpx<T> qb = {e.alpha * (m.x + o.l1.x * o.xb.x + o.l2.x * o.xz.x),
+               e.alpha * (m.y + o.l1.y * o.xb.y + o.l2.y * o.xz.y)};
+  cpx<T> qz = {e.alpha * (o.l2.x * o.xb.x + o.l1.x * o.xz.x),
+               e.alpha * (o.l2.y * o.xb.y + o.l1.y * o.xz.y)};
+  if (e.beta != (T)0) {
+    qb.x += e.beta * o.ob.x;
+    qb.y += e.beta * o.ob.y;
+    qz.x += e.beta * o.oz.x;
+    qz.y += e.beta * o.oz.y;
+  }
+  e.yb[r.re] = qb.x;
+  e.yz[r.re] = qz.x;
+  double acc = (double)o.xb.x * qb.x + (double)o.xz.x * qz.x;
+  if (!r.vertex) {
+    e.yb[r.im] = qb.y;
+    e.yz[r.im] = qz.y;
+    acc += (double)o.xb.y * qb.y + (double)o.xz.y * qz.y;
+  }
   return acc;
 }
 
@@ -549,20 +554,6 @@ __device__ __forceinline__ void line_dft(cpx<T>* lds, const PassArgs<T>& a, int 
 
 __device__ __forceinline__ int udiv(int a, int d, uint32_t m) { return d == 1 ? a : fdiv(a, m); }
 
-template <int D, typename T, int SRC>
-__device__ __forceinline__ cpx<T> spec_load(const PassArgs<T>& a, int k1, int k2, int k3) {
-  if (SRC == SRC_BETA) return beta_to_dft_elem<D, T>(a.beta_in, k1, k2, k3, a.g);
-  return u_to_v<D, T>(a.u_in, k1, k2, k3, a.g, a.H1);
-}
-
-template <int D, typename T, int DST>
-__device__ __forceinline__ double spec_store(const PassArgs<T>& a, int k1, int k2, int k3,
-                                             cpx<T> v) {
-  if (DST == DST_BETA) return scatter_elem<D, T>(a.epi, k1, k2, k3, v, a.g);
-  const int64_t el = k1 + (int64_t)a.H1 * (k2 + (int64_t)a.g.n[1] * k3);
-  return epi_apply_u(a.epi, el, v_to_u<D, T>(v, k1, k2, k3, a.g));
-}
-
 // Workgroups are dispatched to the 8 XCDs round robin (block b on XCD b % 8),
 // each XCD with its own L2.  xcd_block() numbers the blocks so that blocks
 // b, b + 8, b + 16, .. (one XCD) take consecutive numbers: adjacent tiles,
@@ -574,7 +565,7 @@ __device__ __forceinline__ int xcd_block() {
 }
 
 // a fetched source value: mode -1 = outside the tile (zero), otherwise the
-// u_src map of an SRC_U load (other sources: the value as loaded)
+// u_scale map of an SRC_U or SRC_BETA load (SRC_BUF: the value as loaded)
 template <typename T>
 struct Raw {
   cpx<T> w;
@@ -584,7 +575,43 @@ struct Raw {
 template <typename T, int SRC>
 __device__ __forceinline__ cpx<T> raw_value(const Raw<T>& r) {
   if (r.mode < 0) return {(T)0, (T)0};
-  return SRC == SRC_U ? u_map(r.w, r.mode) : r.w;
+  return SRC == SRC_BUF ? r.w : u_scale(r.w, r.mode);
+}
+
+// the source value of element (k1, k2, k3); interior: 1 <= k1 <= P1 and D >= 2
+template <int D, typename T, int SRC>
+__device__ __forceinline__ Raw<T> spec_fetch(const PassArgs<T>& a, int k1, int k2, int k3,
+                                             bool interior) {
+  Raw<T> r;
+  if (SRC == SRC_U) {
+    r.w = a.u_in[u_src<D>(k1, k2, k3, a.g, a.H1, r.mode)];
+    return r;
+  }
+  if (D >= 2 && interior) {
+    const BetaRow w = beta_row<D>(k2, k3, a.g);
+    const uint32_t re = w.re + (uint32_t)(w.s * k1);
+    r.mode = w.neg ? 2 : 0;
+    r.w = {a.beta_in[re], a.beta_in[re + w.d]};
+    return r;
+  }
+  // beta_to_dft_elem's entries (an element that beta does not hold reads its
+  // partner's, conjugate)
+  Cat c1 = cat_of(k1, a.g, 0);
+  Cat c2 = D >= 2 ? cat_of(k2, a.g, 1) : Cat{0, 0};
+  Cat c3 = D >= 3 ? cat_of(k3, a.g, 2) : Cat{0, 0};
+  r.mode = 0;
+  if (!is_rep<D>(c1, c2, c3)) {
+    c1 = cat_mirror(c1, a.g.P[0]);
+    c2 = cat_mirror(c2, a.g.P[1]);
+    c3 = cat_mirror(c3, a.g.P[2]);
+    r.mode = 2;
+  }
+  int64_t bs;
+  bool vertex;
+  const int64_t re = rep_index<D>(c1, c2, c3, a.g, bs, vertex);
+  if (vertex) r.mode = 1;
+  r.w = {a.beta_in[re], a.beta_in[re + (vertex ? 0 : bs)]};
+  return r;
 }
 
 // a value on its way into or out of the LDS tile of a pass whose transform is
@@ -599,6 +626,11 @@ template <typename T>
 struct Fetched {
   cpx<T> m;
   EpiOps<T> ops;
+};
+template <typename T>
+struct FetchedBeta {
+  cpx<T> m;
+  BetaOps<T> ops;
 };
 
 // block -> instance map of a vector launch over several instances
@@ -616,9 +648,10 @@ __device__ __forceinline__ void lines_load(const PassArgs<T>& a, cpx<T>* lds, in
   const int o = tile / a.ntile1;
   const int k10 = tile1 << lg;
   const int nv = min(nl, a.H1 - k10);
-  const int64_t s2 = a.H1, s3 = (int64_t)a.H1 * a.g.n[1];
-  const int64_t sl = a.axis == 1 ? s2 : s3;
-  const int64_t base = k10 + (a.axis == 1 ? (int64_t)o * s3 : (int64_t)o * s2);
+  // element indexes of the half spectrum fit 31 bits
+  const int s2 = a.H1, s3 = a.H1 * a.g.n[1];
+  const int sl = a.axis == 1 ? s2 : s3;
+  const int base = k10 + (a.axis == 1 ? o * s3 : o * s2);
   const int total = L << lg;
   constexpr int K = stage_k<T>();
   // a tile whose k1 are all representatives (1 <= k1 <= P1) reads and writes
@@ -649,10 +682,7 @@ __device__ __forceinline__ void lines_load(const PassArgs<T>& a, cpx<T>* lds, in
         } else {
           const int k2 = a.axis == 1 ? el : o;
           const int k3 = a.axis == 1 ? o : el;
-          if (SRC == SRC_U)
-            r.w = a.u_in[u_src<D>(k1, k2, k3, a.g, a.H1, r.mode)];
-          else
-            r.w = spec_load<D, T, SRC>(a, k1, k2, k3);
+          r = spec_fetch<D, T, SRC>(a, k1, k2, k3, interior);
         }
         if (!ok) r.mode = -1;
         return r;
@@ -670,9 +700,10 @@ __device__ __forceinline__ double lines_store(const PassArgs<T>& a, cpx<T>* lds,
   const int o = tile / a.ntile1;
   const int k10 = tile1 << lg;
   const int nv = min(nl, a.H1 - k10);
-  const int64_t s2 = a.H1, s3 = (int64_t)a.H1 * a.g.n[1];
-  const int64_t sl = a.axis == 1 ? s2 : s3;
-  const int64_t base = k10 + (a.axis == 1 ? (int64_t)o * s3 : (int64_t)o * s2);
+  // element indexes of the half spectrum fit 31 bits
+  const int s2 = a.H1, s3 = a.H1 * a.g.n[1];
+  const int sl = a.axis == 1 ? s2 : s3;
+  const int base = k10 + (a.axis == 1 ? o * s3 : o * s2);
   const int total = L << lg;
   constexpr int K = stage_k<T>();
   // a tile whose k1 are all representatives (1 <= k1 <= P1) reads and writes
@@ -711,7 +742,7 @@ __device__ __forceinline__ double lines_store(const PassArgs<T>& a, cpx<T>* lds,
           const int k3 = a.axis == 1 ? o : el;
           Fetched<T> f;
           f.m = lds[idx];
-          f.ops = epi_fetch_u(a.epi, k1 + (int64_t)a.H1 * (k2 + (int64_t)a.g.n[1] * k3));
+          f.ops = epi_fetch_u(a.epi, k1 + a.H1 * (k2 + a.g.n[1] * k3));
           return f;
         },
         [&](int idx, const Fetched<T>& f) {
@@ -720,24 +751,28 @@ __device__ __forceinline__ double lines_store(const PassArgs<T>& a, cpx<T>* lds,
           const int k1 = k10 + line;
           const int k2 = a.axis == 1 ? el : o;
           const int k3 = a.axis == 1 ? o : el;
-          const int64_t e = k1 + (int64_t)a.H1 * (k2 + (int64_t)a.g.n[1] * k3);
+          const int e = k1 + a.H1 * (k2 + a.g.n[1] * k3);
           acc += epi_commit_u(a.epi, e, v_to_u<D, T>(f.m, k1, k2, k3, a.g), f.ops);
         });
   } else {
-    for (int idx = threadIdx.x; idx < total; idx += NT) {
-      const int line = idx & (nl - 1);
-      const int el = idx >> lg;
-      if (line >= nv) continue;
-      const int k2 = a.axis == 1 ? el : o;
-      const int k3 = a.axis == 1 ? o : el;
-      acc += spec_store<D, T, DST>(a, k10 + line, k2, k3, lds[idx]);
-    }
+    staged<NT, (K > 2 ? K / 2 : 1), FetchedBeta<T>>(
+        total,
+        [&](int idx) {
+          const int line = idx & (nl - 1), el = idx >> lg;
+          const int k1 = k10 + (line < nv ? line : 0);
+          const int k2 = a.axis == 1 ? el : o;
+          const int k3 = a.axis == 1 ? o : el;
+          FetchedBeta<T> f;
+          f.m = lds[idx];
+          f.ops = epi_fetch_beta<D>(a.epi, k1, k2, k3, a.g, interior);
+          return f;
+        },
+        [&](int idx, const FetchedBeta<T>& f) {
+          const int line = idx & (nl - 1);
+          if (line < nv) acc += epi_commit_beta(a.epi, f.m, f.ops);
+        });
   }
   return acc;
-}
-
-__device__ __forceinline__ bool miss_bit(const uint32_t* m, int64_t s) {
-  return m && ((m[s >> 5] >> (s & 31)) & 1u);
 }
 
 // staged values of the dim-1 pass
@@ -813,12 +848,12 @@ __device__ __forceinline__ void dim1_load(const PassArgs<T>& a, cpx<T>* lds, uin
         r.mode = 0;
         r.B = {(T)0, (T)0};
         if (SRC == SRC_BUF) {
-          r.A = a.buf[(int64_t)min(la, nl1) * H1 + k];
-          r.B = a.buf[(int64_t)min(la + 1, nl1) * H1 + k];
-        } else if (SRC == SRC_U) {
-          r.A = a.u_in[u_src<D>(k, 0, 0, a.g, a.H1, r.mode)];   // 1D: a single line
-        } else {
-          r.A = spec_load<D, T, SRC>(a, k, 0, 0);
+          r.A = a.buf[min(la, nl1) * H1 + k];
+          r.B = a.buf[min(la + 1, nl1) * H1 + k];
+        } else {   // 1D: a single line
+          const Raw<T> w = spec_fetch<D, T, SRC>(a, k, 0, 0, false);
+          r.A = w.w;
+          r.mode = w.mode;
         }
         return r;
       },
@@ -827,7 +862,7 @@ __device__ __forceinline__ void dim1_load(const PassArgs<T>& a, cpx<T>* lds, uin
         const int k = idx - p * H1;
         const int la = 2 * (p0 + p), lb = la + 1;
         const cpx<T> zero = {(T)0, (T)0};
-        cpx<T> A = la < a.nlines ? (SRC == SRC_U ? u_map(r.A, r.mode) : r.A) : zero;
+        cpx<T> A = la < a.nlines ? (SRC == SRC_BUF ? r.A : u_scale(r.A, r.mode)) : zero;
         cpx<T> B = (SRC == SRC_BUF && lb < a.nlines) ? r.B : zero;
         if (k == 0 || (even && k == H1 - 1)) {  // DC / Nyquist of a real line are real
           A.y = 0;
@@ -985,8 +1020,8 @@ __device__ __forceinline__ double dim1_store(const PassArgs<T>& a, cpx<T>* lds, 
           const cpx<T> X = r.A, Y = r.B;
           const cpx<T> Va = {half * (X.x + Y.x), half * (X.y - Y.y)};
           const cpx<T> Vb = {half * (X.y + Y.y), half * (Y.x - X.x)};
-          a.buf[(int64_t)la * H1 + k] = Va;
-          if (lb < a.nlines) a.buf[(int64_t)lb * H1 + k] = Vb;
+          a.buf[la * H1 + k] = Va;
+          if (lb < a.nlines) a.buf[lb * H1 + k] = Vb;
         });
   } else if (DST == DST_U) {   // 1D: line 0 only
     staged<NT, (K > 2 ? K / 2 : 1), Fetched2<T>>(
@@ -1007,17 +1042,21 @@ __device__ __forceinline__ double dim1_store(const PassArgs<T>& a, cpx<T>* lds, 
           const cpx<T> Va = {half * (f.X.x + f.Y.x), half * (f.X.y - f.Y.y)};
           acc += epi_commit_u(a.epi, k, v_to_u<D, T>(Va, k, 0, 0, a.g), f.ops);
         });
-  } else {
-    for (int idx = threadIdx.x; idx < tot; idx += NT) {
-      const int p = udiv(idx, H1, a.h1m);
-      const int k = idx - p * H1;
-      const int la = 2 * (p0 + p);
-      if (la >= a.nlines) continue;
-      const cpx<T> X = lds[k * ps + p];
-      const cpx<T> Y = lds[(k == 0 ? 0 : N1 - k) * ps + p];
-      const cpx<T> Va = {half * (X.x + Y.x), half * (X.y - Y.y)};
-      acc += spec_store<D, T, DST>(a, k, 0, 0, Va);   // 1D: line 0 only
-    }
+  } else {   // 1D: line 0 only
+    staged<NT, (K > 2 ? K / 2 : 1), FetchedBeta<T>>(
+        tot,
+        [&](int idx) {
+          const int p = udiv(idx, H1, a.h1m);
+          const int k = idx - p * H1;
+          const cpx<T> X = lds[k * ps + p], Y = lds[(k == 0 ? 0 : N1 - k) * ps + p];
+          FetchedBeta<T> f;
+          f.m = {half * (X.x + Y.x), half * (X.y - Y.y)};
+          f.ops = epi_fetch_beta<D>(a.epi, k, 0, 0, a.g, false);
+          return f;
+        },
+        [&](int idx, const FetchedBeta<T>& f) {
+          if (2 * (p0 + udiv(idx, H1, a.h1m)) < a.nlines) acc += epi_commit_beta(a.epi, f.m, f.ops);
+        });
   }
   return acc;
 }
@@ -1035,6 +1074,12 @@ __device__ __forceinline__ double dim1_store(const PassArgs<T>& a, cpx<T>* lds, 
 //         x FFT_M(w)/M = conj(bfw), inverse, twiddle)  col MID (inverse, x conj(w), mask,
 //         x w, forward, twiddle)  row CONV_FWD  col LAST (inverse, x w, epilogue)
 // ===========================================================================
+// (unstaged: groups of loads held in registers were slower here, 44 -> 48 us
+// for 49999 samples in FP32 and 57 -> 66 ms for a mixed batch)
+__device__ __forceinline__ bool miss_bit(const uint32_t* m, int64_t s) {
+  return m && ((m[s >> 5] >> (s & 31)) & 1u);
+}
+
 template <typename T>
 __device__ __forceinline__ cpx<T> twf(const PassArgs<T>& a, int64_t j, bool inv) {
   cpx<T> w = a.twF[j];
@@ -1052,9 +1097,10 @@ __device__ __forceinline__ cpx<T> chirp_at(const PassArgs<T>& a, int64_t n, bool
 // spectrum value k (< N) of a Hermitian line held as its half (k < H1)
 template <typename T, int SRC>
 __device__ __forceinline__ cpx<T> half_load(const PassArgs<T>& a, int64_t k) {
-  if (k < a.H1) return spec_load<1, T, SRC>(a, (int)k, 0, 0);
-  const cpx<T> v = spec_load<1, T, SRC>(a, (int)(a.len - k), 0, 0);
-  return {v.x, -v.y};
+  const bool far = k >= a.H1;
+  const cpx<T> v =
+      raw_value<T, SRC>(spec_fetch<1, T, SRC>(a, (int)(far ? a.len - k : k), 0, 0, false));
+  return {v.x, far ? -v.y : v.y};
 }
 
 // FWD: the pass's first transform is forward (else the tile holds exchanged
@@ -1136,7 +1182,10 @@ __device__ __forceinline__ double col_store(const PassArgs<T>& a, cpx<T>* lds, i
       const int64_t k = col + (int64_t)A * r;
       if (k < a.H1) {
         if (bs) v = cmul(cswap(v), chirp_at(a, k, false));   // ends in the inverse transform
-        acc += spec_store<1, T, DST>(a, (int)k, 0, 0, v);
+        if constexpr (DST == DST_U)
+          acc += epi_commit_u(a.epi, k, v_to_u<1, T>(v, (int)k, 0, 0, a.g), epi_fetch_u(a.epi, k));
+        else
+          acc += epi_commit_beta(a.epi, v, epi_fetch_beta<1>(a.epi, (int)k, 0, 0, a.g, false));
       }
     }
   }

@@ -42,9 +42,30 @@ void sc(const MapGeom& g, int64_t* re, int64_t* im, int8_t* flags, int H1) {
         flags[t] = (int8_t)((hit ? 1 : 0) | (vertex ? 2 : 0) | (neg ? 4 : 0));
       }
 }
+// interior elements (1 <= k1 <= P1) whose beta_row differs from scatter_targets
+template <int D>
+int64_t rows_off(const MapGeom& g) {
+  int64_t bad = 0;
+  for (int k3 = 0; k3 < g.n[2]; ++k3)
+    for (int k2 = 0; k2 < g.n[1]; ++k2) {
+      const BetaRow w = beta_row<D>(k2, k3, g);
+      for (int k1 = 1; k1 <= g.P[0]; ++k1) {
+        int64_t re = -1, im = -1;
+        bool vertex = false, neg = false;
+        const bool hit = scatter_targets<D>(k1, k2, k3, g, re, im, vertex, neg);
+        const uint32_t r = w.re + (uint32_t)(w.s * k1);
+        bad += !(hit && !vertex && (int64_t)r == re && (int64_t)(r + w.d) == im && w.neg == neg);
+      }
+    }
+  return bad;
+}
 }  // namespace
 
 extern "C" {
+int64_t geomchk_rows(int dim, const int64_t* sizes) {
+  const MapGeom g = geom(dim, sizes);
+  return dim == 2 ? rows_off<2>(g) : rows_off<3>(g);
+}
 // the geometry fields, for comparison with the oracle: n, M, P, S (3 each),
 // N, P12, P13, P23, P123, off[8]
 void geomchk_info(int dim, const int64_t* sizes, int64_t* out) {

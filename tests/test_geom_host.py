@@ -116,3 +116,14 @@ def test_spectrum_order_is_exact(glib, dims):
     want = maps.beta_to_dft(beta, dims, rdft=True)
     assert np.array_equal(v[0::2], want.real) and np.array_equal(v[1::2], want.imag)
     assert np.array_equal(back, maps.dft_to_beta(spec, dims))
+
+
+# the passes' row form of the beta indices (interior of dimension 1) against
+# the per-element form, over odd, even and tiny sizes of every class
+@pytest.mark.parametrize("dims", [d for d in SHAPES if len(d) >= 2] +
+                         [(3, 2), (4, 3), (5, 1 + 1), (3, 3, 2), (4, 2, 3), (3, 4, 5), (9, 2, 2),
+                          (6, 7, 4), (7, 5, 6)])
+def test_rows_equal_elements(glib, dims):
+    glib.geomchk_rows.restype = ctypes.c_int64
+    sz = _sizes(dims)
+    assert glib.geomchk_rows(len(dims), _p(sz)) == 0
