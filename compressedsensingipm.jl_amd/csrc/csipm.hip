@@ -291,27 +291,54 @@ static void release_pending() {
 namespace {
 
 constexpr int kNT = 256;      // threads per workgroup of the vector kernels
-// FFT passes: kE complex elements of the tile per thread, so the workgroup
-// size follows from the tile (tile_nt): 256 or 512 threads up to kTile
-// elements, 1024 up to 8192 and, sized kNTLong, 1024 threads of 16 elements up
-// to kTileLong (dimension-1 passes only)
+// FFT passes: a thread holds kE complex elements of the tile in a stage, or
+// one butterfly of a radix above that.  kTile: the largest tile of a line,
+// column or row pass; dimension-1 passes go on to kTileLong with kNTLong (a name
+// for 1024 threads of 16 elements).
 constexpr int kE = 8;
 constexpr int kTile = 4096;
-// tiles grow to kTileGrow elements (256 threads), and beyond only while a row
-// of the tile spans less than 64 bytes: several small workgroups on a CU
-// overlap one's loads with another's transform
-constexpr int kTileGrow = 2048;
-inline bool tile_grows(int lg, int W, size_t cs) {
-  const int64_t e = (int64_t)(2 << lg) * W;
-  return e <= kTileGrow || (e <= kTile && ((size_t)1 << lg) * cs < 64);
-}
 constexpr int kTileLong = 16384;
-constexpr int kNTLong = 2048;   // names the last: 1024 threads, 16 elements each
-inline int tile_nt(int64_t elems) {
-  return elems <= 256 * kE ? 256 : elems <= 512 * kE ? 512 : elems <= 1024 * kE ? 1024 : kNTLong;
-}
+constexpr int kNTLong = 2048;
 constexpr size_t kLdsSmall = 64 * 1024;
 constexpr size_t kLdsMax = 160 * 1024;
+// elements a thread takes through the stages of a plan
+inline int plan_cap(const FftPlan& p) {
+  int cap = 2 * kE;
+  for (int s = 0; s < p.nstages; ++s) {
+    const int R = p.st[s].radix;
+    cap = std::min(cap, R * ((kE + R - 1) / R));
+  }
+  return cap;
+}
+inline int tile_threads(int64_t elems, const FftPlan& p) {
+  const int cap = plan_cap(p);
+  return (int)((elems + cap - 1) / cap);
+}
+// workgroup size of a tile: as many threads as the stages keep busy, but 256
+// for tiles of up to 1024 elements (more loads in flight where the launch is
+// short) and where 128 would move 16 elements each through the global phases
+// (256^3 FP64: 617 us on 256 threads, 652 on 128).  391 = 23 x 17 points in 4
+// lines keep 92 threads busy.
+inline int tile_nt(int64_t elems, const FftPlan& p) {
+  const int t = tile_threads(elems, p);
+  if (t <= 128 && elems > 1024 && elems <= 14 * 128) return 128;
+  return t <= 256 ? 256 : t <= 512 ? 512 : t <= 1024 ? 1024 : kNTLong;
+}
+// A tile of 2^lg lines (rows LDS rows each) is doubled while 256 threads and 32
+// KB hold it, and up to 512 threads only while its rows span less than 32
+// bytes: several small workgroups on a CU overlap one's loads with another's
+// transform.  185^3 in FP32 (391 rows): 414 us with four lines on 256 threads,
+// 453 with eight on 512.  mixed: a launch of several kinds of passes, whose
+// workgroups all hold the LDS of the largest tile: 2048 elements (48 requests,
+// 56.6 against 59.6 ms).
+inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed) {
+  const int64_t e = (int64_t)(2 << lg) * p.L;
+  const int t = tile_threads(e, p);
+  if (e > kTile) return false;
+  if (mixed && e > kTile / 2 && ((size_t)1 << lg) * cs >= 64) return false;
+  return (t <= 256 && ((size_t)2 << lg) * rows * cs <= 32 * 1024) ||
+         (t <= 512 && ((size_t)1 << lg) * cs < 32);
+}
 
 struct LineCfg {
   int lg = 0, ntile1 = 0, grid = 0;
@@ -872,17 +899,15 @@ static int min_tile_lg(size_t cs) {
   return lg;
 }
 
-// line FFTs along dim 2/3: 2^lg lines per workgroup, as many as the
-// registers (lines * W <= NT*E for the FFT length W) and 64 KB of LDS (lines *
-// R rows) allow, fewer when that
-// would leave the launch with under min_grid workgroups (1024 for one
-// instance; a batch shares the target among its instances)
-
-static LineCfg line_cfg(int H1, int W, int R, int64_t others, size_t cs,
-                        int min_grid = 1024, int lg_cap = 30) {
+// line FFTs along dim 2/3: 2^lg lines per workgroup, as many as tile_grows
+// allows, fewer when that would leave the launch with under min_grid
+// workgroups (1024 for one instance; a batch shares the target among its
+// instances)
+static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size_t cs,
+                        int min_grid = 1024, int lg_cap = 30, bool mixed = false) {
   LineCfg c{};
   int lg = 0;
-  while (tile_grows(lg, W, cs) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
+  while (tile_grows(lg, plan, R, cs, mixed) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
          lg < lg_cap)
     ++lg;
   // below 64-byte rows only while the launch would not even give a
@@ -895,15 +920,17 @@ static LineCfg line_cfg(int H1, int W, int R, int64_t others, size_t cs,
   c.ntile1 = (H1 + (1 << lg) - 1) >> lg;
   c.grid = (int)(c.ntile1 * others);
   c.lds = (size_t)(1 << lg) * R * cs;
-  c.nt = tile_nt((int64_t)W << lg);
+  c.nt = tile_nt((int64_t)plan.L << lg, plan);
   return c;
 }
 
 // four-step column pass: 2^lg adjacent columns of length B per workgroup
-static LineCfg col_cfg(int A, int B, size_t cs, int min_grid = 1024) {
+static LineCfg col_cfg(int A, const FftPlan& plan, size_t cs, int min_grid = 1024,
+                       bool mixed = false) {
   LineCfg c{};
+  const int B = plan.L;
   int lg = 0;
-  while (tile_grows(lg, B, cs) && (size_t)(2 << lg) * B * cs <= kLdsSmall && (2 << lg) <= A)
+  while (tile_grows(lg, plan, B, cs, mixed) && (size_t)(2 << lg) * B * cs <= kLdsSmall && (2 << lg) <= A)
     ++lg;
   const int lg_min = std::min(lg, min_tile_lg(cs));
   auto grid_of = [&](int l) { return (A + (1 << l) - 1) >> l; };
@@ -912,32 +939,34 @@ static LineCfg col_cfg(int A, int B, size_t cs, int min_grid = 1024) {
   c.ntile1 = (A + (1 << lg) - 1) >> lg;
   c.grid = c.ntile1;
   c.lds = (size_t)(1 << lg) * B * cs;
-  c.nt = tile_nt((int64_t)B << lg);
+  c.nt = tile_nt((int64_t)B << lg, plan);
   return c;
 }
 
 // four-step row pass: 2^lg rows of length A per workgroup (LDS stride padded)
-static Dim1Cfg row_cfg(int A, int B, size_t cs, int min_grid = 1024) {
+static Dim1Cfg row_cfg(const FftPlan& plan, int B, size_t cs, int min_grid = 1024,
+                       bool mixed = false) {
   Dim1Cfg c{};
+  const int A = plan.L;
   int lg = 0;
   auto lds_of = [&](int l) { return (size_t)A * ((1 << l) + 1) * cs; };
-  while ((2 << lg) * A <= kTileGrow && lds_of(lg + 1) <= kLdsSmall && (2 << lg) <= B) ++lg;
+  while (tile_grows(lg, plan, A, cs, mixed) && lds_of(lg + 1) <= kLdsSmall && (2 << lg) <= B) ++lg;
   while (lg > 0 && ((B + (1 << lg) - 1) >> lg) < min_grid) --lg;
   c.lg = lg;
   c.ps = (1 << lg) + 1;
   c.grid = (B + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
-  c.nt = tile_nt((int64_t)A << lg);
+  c.nt = tile_nt((int64_t)A << lg, plan);
   return c;
 }
 
-static Dim1Cfg dim1_cfg(int W, int R, int nlines, size_t cs, int min_grid = 1024,
-                        int lg_cap = 30) {
+static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int min_grid = 1024,
+                        int lg_cap = 30, bool mixed = false) {
   Dim1Cfg c{};
   c.npairs = (nlines + 1) / 2;
   int lg = 0;
   auto lds_of = [&](int l) { return (size_t)R * ((1 << l) + (l > 0 ? 1 : 0)) * cs; };
-  while ((2 << lg) * W <= kTileGrow && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
+  while (tile_grows(lg, plan, R, cs, mixed) && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
          lg < lg_cap)
     ++lg;
   while (lg > 0 && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
@@ -945,7 +974,7 @@ static Dim1Cfg dim1_cfg(int W, int R, int nlines, size_t cs, int min_grid = 1024
   c.ps = (1 << lg) + (lg > 0 ? 1 : 0);
   c.grid = (c.npairs + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
-  c.nt = tile_nt((int64_t)W << lg);
+  c.nt = tile_nt((int64_t)plan.L << lg, plan);
   return c;
 }
 
@@ -1118,6 +1147,7 @@ int launch_pass(csipm_op* h, const PassArgs<T>& a, int grid, int nt, size_t lds)
 #define CSIPM_IS(LD, MID, ST) a.ld == LD && a.mid == MID && a.st == ST
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST);      \
     if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
     if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
   }
@@ -1921,8 +1951,8 @@ static int upload_big1d(csipm_op* h) {
 static int set_shapes(csipm_op* h, PrecState& ps, size_t cs) {
   const int dim = h->dim;
   if (h->big) {
-    ps.col = col_cfg(h->bA, h->bB, cs);
-    ps.row = row_cfg(h->bA, h->bB, cs);
+    ps.col = col_cfg(h->bA, h->planB, cs);
+    ps.row = row_cfg(h->planA, h->bB, cs);
     if (ps.col.lds > kLdsMax || ps.row.lds > kLdsMax)
       return fail(CSIPM_ERR_UNSUPPORTED, "four-step plan of length %d exceeds the LDS", h->n[0]);
     return CSIPM_OK;
@@ -1930,12 +1960,12 @@ static int set_shapes(csipm_op* h, PrecState& ps, size_t cs) {
   // FFT length W (line length, Bluestein's M, Rader's L - 1) and LDS rows of a
   // dim-1 line (L, M, Rader's 2L + 1)
   const int F0 = h->plan[0].L;
-  ps.d1 = dim1_cfg(F0, h->rows[0], (int)(h->N / h->n[0]), cs);
+  ps.d1 = dim1_cfg(h->plan[0], h->rows[0], (int)(h->N / h->n[0]), cs);
   if (F0 > kTileLong || ps.d1.lds > kLdsMax)
     return fail(CSIPM_ERR_UNSUPPORTED, "dimension-1 length %d (FFT length %d) exceeds one "
                 "workgroup", h->n[0], F0);
-  if (dim >= 2) ps.lines[1] = line_cfg(h->H1, h->plan[1].L, h->rows[1], h->n[2], cs);
-  if (dim == 3) ps.lines[2] = line_cfg(h->H1, h->plan[2].L, h->rows[2], h->n[1], cs);
+  if (dim >= 2) ps.lines[1] = line_cfg(h->H1, h->plan[1], h->rows[1], h->n[2], cs);
+  if (dim == 3) ps.lines[2] = line_cfg(h->H1, h->plan[2], h->rows[2], h->n[1], cs);
   for (int ax = 1; ax < dim; ++ax)
     if (h->plan[ax].L > kTile || ps.lines[ax].lds > kLdsMax)
       return fail(CSIPM_ERR_UNSUPPORTED, "dimension-%d length %d (%d LDS rows) exceeds one "

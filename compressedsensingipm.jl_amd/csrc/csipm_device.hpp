@@ -412,15 +412,20 @@ __device__ __forceinline__ void dft_odd_store(cpx<T>* v, cpx<T>* __restrict__ ds
     dst[k * stride] = {re + sre, im - sim};
     dst[(R - k) * stride] = {re - sre, im + sim};
   };
-  if constexpr (R < 17) {
+  if constexpr (R < 29) {
+    // one output after another: scheduled across outputs the (H x H) products
+    // took hundreds of registers in FP64
 #pragma unroll
-    for (int k = 1; k <= H; ++k)
+    for (int k = 1; k <= H; ++k) {
       output(k, [&](int j) { return (T)OddRadix<R>::c[(j * k) % R]; },
              [&](int j) { return (T)OddRadix<R>::s[(j * k) % R]; });
+      if constexpr (R >= 11) __builtin_amdgcn_sched_barrier(0);
+    }
   } else {
-    // a loop over the outputs, their coefficients by scalar loads: unrolled,
-    // the (H x H) products were scheduled across outputs and spilled hundreds
-    // of registers in FP64 (and radix 31 alone was 900 instructions)
+    // a loop over the outputs, their coefficients by scalar loads: unrolled
+    // (900 instructions for radix 31) these two took 20 registers more than
+    // the rest.  Slower per output: radices 17 to 23 in this form took the
+    // FP32 185^3 product (Bluestein 23 x 17) from 402 to 525 us
 #pragma unroll 1
     for (int k = 1; k <= H; ++k) {
       const T* row = OddRows<T, R>::cs[k - 1];
@@ -446,8 +451,8 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
 // reads elements j + r*L/R, multiplies input r by exp(-2 pi i r k/(Ns*R)),
 // k = j mod Ns, and writes elements (j - k)*R + k + r*Ns.  Butterflies are
 // numbered b = j * 2^lg + l, so the lines of a tile run on adjacent lanes and
-// share twiddles.  The caller guarantees 2^lg * L <= NT * E: a thread holds
-// max(E, R) complex values in a stage.
+// share twiddles.  A thread takes ceil(E / R) butterflies; the caller
+// guarantees that NT threads then cover the (L / R) 2^lg of every stage.
 // What bounds a stage: the number of waves a SIMD holds.  With E = 16 (two
 // radix-9..15 butterflies and their twiddles per thread) the FP64 passes
 // took 248-260 registers, one or two waves per SIMD, and the 1024-thread ones

@@ -194,6 +194,7 @@ int launch_sub(const ChainSub& a, hipStream_t st) {
   } while (0)
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
+    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST);      \
     if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
     if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
   }
@@ -470,7 +471,8 @@ int vblocks(int64_t n) {
 }
 
 // launch shapes of instance h inside a chain over `members` instances: the
-// workgroup-count target of a single launch is shared among them
+// workgroup-count target of a single launch is shared among them (mixed: they
+// are of several kinds)
 struct BatchCfg {
   LineCfg lines[3];
   Dim1Cfg d1;
@@ -479,22 +481,23 @@ struct BatchCfg {
 };
 
 template <typename T>
-BatchCfg batch_cfg(csipm_op* h, int members) {
+BatchCfg batch_cfg(csipm_op* h, int members, bool mixed) {
   const int target = std::max(1, 1024 / std::max(1, members));
   const size_t cs = sizeof(cpx<T>);
   BatchCfg b{};
   if (h->big) {
-    b.col = col_cfg(h->bA, h->bB, cs, target);
-    b.row = row_cfg(h->bA, h->bB, cs, target);
+    b.col = col_cfg(h->bA, h->planB, cs, target, mixed);
+    b.row = row_cfg(h->planA, h->bB, cs, target, mixed);
     return b;
   }
   const TuneVal t0 = tune_lookup(1, cs, h->plan[0].L, h->rows[0]);
-  b.d1 = dim1_cfg(h->plan[0].L, h->rows[0], (int)(h->N / h->n[0]), cs, target, t0.lg_cap);
+  b.d1 = dim1_cfg(h->plan[0], h->rows[0], (int)(h->N / h->n[0]), cs, target, t0.lg_cap,
+                  mixed);
   TuneVal ta[3];
   for (int a = 1; a < h->dim; ++a) {
     ta[a] = tune_lookup(0, cs, h->plan[a].L, h->rows[a]);
-    b.lines[a] = line_cfg(h->H1, h->plan[a].L, h->rows[a], h->n[a == 1 ? 2 : 1], cs, target,
-                          ta[a].lg_cap);
+    b.lines[a] = line_cfg(h->H1, h->plan[a], h->rows[a], h->n[a == 1 ? 2 : 1], cs, target,
+                          ta[a].lg_cap, mixed);
   }
   return b;
 }
@@ -569,6 +572,13 @@ inline int pass_nt(const PassSpec& s, const BatchCfg& bc) {
   return s.kind == PK_COL ? bc.col.nt : bc.row.nt;
 }
 
+// several kinds of chains, whose launches are shared
+bool mixed_kinds(Engine* E, const std::vector<int>& ids) {
+  for (int id : ids)
+    if (chain_key(E->inst[(size_t)id].h) != chain_key(E->inst[(size_t)ids[0]].h)) return true;
+  return false;
+}
+
 // Block map of a launch over members with `grids` tiles each.  Block b runs on
 // XCD b % 8, each XCD with its own L2: a member's tiles go to the XCDs in
 // eight consecutive ranges (adjacent tiles share cache lines), the few tiles
@@ -611,6 +621,7 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
   };
   // whole 1D lines first: their workgroups run longest
   std::vector<Member> mem;
+  const bool mixed = mixed_kinds(E, ids);   // no launches of their own for 128 threads
   for (bool line : {true, false})
     for (int id : ids) {
       csipm_op* h = E->inst[(size_t)id].h;
@@ -618,11 +629,11 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
       Member m;
       m.id = id;
       m.np = chain_specs(h, call == CALL_MTZ ? CH_MTZ : CH_MTM, m.specs);
-      m.bc = batch_cfg<T>(h, (int)ids.size());
+      m.bc = batch_cfg<T>(h, (int)ids.size(), mixed);
       mem.push_back(m);
     }
   for (int p = 0; p < 8; ++p)
-    for (int nt : {kNTLong, 1024, 512, 256}) {
+    for (int nt : {kNTLong, 1024, 512, 256, 128}) {
       ChainSub sub;
       sub.pass = p;
       sub.nt = nt;
@@ -630,7 +641,9 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
       std::vector<PassArgs<T>> tab;
       std::vector<int> grids;
       for (const Member& m : mem) {
-        if (p >= m.np || pass_nt(m.specs[p], m.bc) != nt) continue;
+        if (p >= m.np) continue;
+        const int want = pass_nt(m.specs[p], m.bc);
+        if ((mixed ? std::max(want, 256) : want) != nt) continue;
         const PassSpec& s = m.specs[p];
         PassArgs<T> a{};
         CHK(chain_call_args<T>(E, m.id, call, nb, s, m.bc, a));
@@ -664,8 +677,8 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
 // final-pass partial count of the CG apply of instance h (precision T) in a
 // chain over `members` instances
 template <typename T>
-int cg_final_grid(csipm_op* h, int members) {
-  const BatchCfg bc = batch_cfg<T>(h, members);
+int cg_final_grid(csipm_op* h, int members, bool mixed) {
+  const BatchCfg bc = batch_cfg<T>(h, members, mixed);
   if (h->big) return bc.col.grid;
   if (h->dim == 1) return bc.d1.grid;
   return bc.lines[h->dim - 1].grid;
@@ -699,9 +712,10 @@ int engine_upload_records(Engine* E) {
 template <typename TC>
 int update_gcg(Engine* E) {
   const int m = (int)E->active.size();
+  const bool mixed = mixed_kinds(E, E->active);
   for (int id : E->active) {
     Engine::Inst& in = E->inst[(size_t)id];
-    const int g = cg_final_grid<TC>(in.h, m);
+    const int g = cg_final_grid<TC>(in.h, m, mixed);
     if (g + (int64_t)vblocks(in.h->U) > in.len / kSlotAlign * kPartPerAlign)
       return fail(CSIPM_ERR_UNSUPPORTED, "partial sums of instance exceed its share");
     E->info_h[(size_t)id].gcg = g;
@@ -805,7 +819,7 @@ int engine_admit(Engine* E, csipm_op* h, const double* z0, double lam, double* b
   const int64_t len = slots_of(h);
   // partial-sum capacity: 8 quantities per vector block, the CG apply's final pass
   const int64_t pcap = len / kSlotAlign * kPartPerAlign;
-  const int gcg = E->tc_size == 8 ? cg_final_grid<double>(h, 1) : cg_final_grid<float>(h, 1);
+  const int gcg = E->tc_size == 8 ? cg_final_grid<double>(h, 1, false) : cg_final_grid<float>(h, 1, false);
   // (the apply's p'q partials and the CG update's r'z partials side by side)
   if (8 * (int64_t)vblocks(h->U) > pcap || gcg + (int64_t)vblocks(h->U) > pcap)
     return fail(CSIPM_ERR_UNSUPPORTED, "partial sums of instance exceed its share");

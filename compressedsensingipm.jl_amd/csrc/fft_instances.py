@@ -47,7 +47,7 @@ ENTRY_DIM1 = [
 ]
 # workgroup sizes with the elements per thread: of tiles up to 4096 elements,
 # and of longer lines (dimension 1 only)
-NT_SHORT = ["256 8", "512 8"]
+NT_SHORT = ["128 8", "256 8", "512 8"]
 NT_LONG = ["1024 8", "1024 16"]
 MIXED = "-1 -1 -1"
 

@@ -6,8 +6,8 @@ rounded once to double (printed with 17 significant digits)."""
 import os
 import numpy as np
 
-ODD = [3, 5, 7, 9, 11, 13, 15]
-ROWS = [17, 19, 23, 29, 31]
+ODD = [3, 5, 7, 9, 11, 13, 15, 17, 19, 23]
+ROWS = [29, 31]
 
 
 def main(path):
