@@ -301,6 +301,7 @@ constexpr int kTileLong = 16384;
 constexpr int kNTLong = 2048;
 constexpr size_t kLdsSmall = 64 * 1024;
 constexpr size_t kLdsMax = 160 * 1024;
+constexpr int kDenseVariant = 2;   // FftPlan::variant of a dense axis (no stages)
 // elements a thread takes through the stages of a plan
 inline int plan_cap(const FftPlan& p) {
   int cap = 2 * kE;
@@ -320,6 +321,7 @@ inline int tile_threads(int64_t elems, const FftPlan& p) {
 // (256^3 FP64: 617 us on 256 threads, 652 on 128).  391 = 23 x 17 points in 4
 // lines keep 92 threads busy.
 inline int tile_nt(int64_t elems, const FftPlan& p) {
+  if (p.variant == kDenseVariant) return 256;
   const int t = tile_threads(elems, p);
   if (t <= 128 && elems > 1024 && elems <= 14 * 128) return 128;
   return t <= 256 ? 256 : t <= 512 ? 512 : t <= 1024 ? 1024 : kNTLong;
@@ -333,6 +335,11 @@ inline int tile_nt(int64_t elems, const FftPlan& p) {
 // 56.6 against 59.6 ms).
 inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed) {
   const int64_t e = (int64_t)(2 << lg) * p.L;
+  // dense: the matrix tiles want 16 real columns, and more share their
+  // coefficients; four waves hold 16 k-tiles of 16 columns, 8 of 32 or 4 of 64
+  if (p.variant == kDenseVariant)
+    return lg < 3 || (lg < (p.L <= 127 ? 5 : p.L <= 255 ? 4 : 3) &&
+                      ((size_t)2 << lg) * rows * cs <= (mixed ? 16 : 32) * 1024);
   const int t = tile_threads(e, p);
   if (e > kTile) return false;
   if (mixed && e > kTile / 2 && ((size_t)1 << lg) * cs >= 64) return false;
@@ -379,7 +386,8 @@ struct csipm_op {
   int H1 = 0;
   int64_t N = 0, Nc = 0, U = 0;  // U = 2*Nc: length of the spectrum-ordered copy of beta
   FftPlan plan[3]{};             // line FFT of each axis (Bluestein: length M; Rader: L - 1)
-  int bs[3] = {0, 0, 0};         // line transform of each axis: 0 direct, 1 Bluestein, 2 Rader
+  int bs[3] = {0, 0, 0};         // line transform of each axis: 0 direct, 1 Bluestein, 2 Rader,
+                                 // 3 dense
   int rows[3] = {1, 1, 1};       // LDS rows per line (L, M, or 2L + 1 for Rader)
   int* rperm[3] = {nullptr, nullptr, nullptr};   // Rader permutation tables (2L ints)
   // 1D lines longer than one workgroup holds: four-step over B rows x A
@@ -469,26 +477,45 @@ static bool is_prime(int n) {
 static std::mutex g_blue_mu;
 static std::map<int, int> g_blue_m;
 
+// Dense form (on the matrix cores): an axis of a 2D / 3D problem whose length
+// does not factor, L <= kDenseMax, unless a tuned Bluestein length asks for the
+// older forms.  A tile of eight lines takes L^2 / 16 cycles in FP32 (twice
+// that in FP64) on its CU whatever the launch's size, so above kDenseAny it
+// serves launches that fill the chip (eight-line tiles for every CU).
+constexpr int kDenseMax = 511;
+constexpr int kDenseAny = 256;
+static bool dense_axis(int L, int64_t lines) {
+  return L > 32 && L <= kDenseMax && (L <= kDenseAny || lines >= 8 * 256);
+}
+
 // axis plan: the direct mixed-radix plan when L factors into the supported
-// radices; for a prime L whose L - 1 does, Rader's form (plan of length
-// L - 1); else Bluestein with the tuned convolution length of L, or the
-// smallest M >= 2L - 1 that factors.  rows: LDS rows a line needs.
-static bool plan_axis(int L, FftPlan& p, int& bs, int& rows) {
+// radices; else the dense form (dense_axis); for a prime L whose L - 1
+// factors, Rader's form (plan of length L - 1); else Bluestein with the tuned
+// convolution length of L, or the smallest M >= 2L - 1 that factors.  rows:
+// LDS rows a line needs; lines: lines along the axis, 0 for a 1D problem.
+static bool plan_axis(int L, int64_t lines, FftPlan& p, int& bs, int& rows) {
   bs = 0;
   rows = L;
   if (factorize(L, p)) return true;
-  if (L > 2 && is_prime(L) && factorize(L - 1, p)) {
-    bs = 2;
-    rows = 2 * L + 1;
-    return true;
-  }
-  bs = 1;
   int tuned = 0;
   {
     std::lock_guard<std::mutex> lk(g_blue_mu);
     const auto it = g_blue_m.find(L);
     if (it != g_blue_m.end()) tuned = it->second;
   }
+  if (!tuned && lines > 0 && dense_axis(L, lines)) {
+    bs = 3;
+    p = FftPlan{};
+    p.L = L;
+    p.variant = kDenseVariant;
+    return true;
+  }
+  if (L > 2 && is_prime(L) && factorize(L - 1, p)) {
+    bs = 2;
+    rows = 2 * L + 1;
+    return true;
+  }
+  bs = 1;
   if (tuned && factorize(tuned, p)) {
     rows = tuned;
     return true;
@@ -754,7 +781,8 @@ static int upload_rader(int p, void** bfw) {
 
 // Twiddles in the op precision: exp(-2 pi i t / L), t < L, in their order
 // (plan null; the four-step passes' table) or laid out for the stages of a
-// plan (FftStage::tw; L - radix_0 entries).  Tables are shared by the
+// plan (FftStage::tw; L - radix_0 entries), or the coefficients of a dense
+// axis.  Tables are shared by the
 // handles on a device and counted: a table no handle holds stays cached
 // (a serving process meets the same lengths again) until the unheld tables
 // exceed kTwiddleKeepBytes, when the least recently used go back to the
@@ -775,6 +803,28 @@ static std::unordered_map<void*, int64_t> g_tw_key;         // table -> key
 static std::set<std::pair<uint64_t, int64_t>> g_tw_unheld;  // (last use, key), refs == 0
 static size_t g_tw_unheld_bytes = 0;
 static uint64_t g_tw_clock = 0;
+
+// dense form: the packed cosine and sine tiles of a line length (dense_dft)
+template <typename T>
+static void dense_table(int L, const std::vector<std::complex<double>>& r, std::vector<T>& h) {
+  const int Mt = dense_mt(L), Kc = dense_kc(L), Ks = dense_ks(L), Hc = L / 2, Hs = (L - 1) / 2;
+  h.assign((size_t)Mt * (Kc + Ks) * 64, (T)0);
+  for (int mt = 0; mt < Mt; ++mt)
+    for (int lane = 0; lane < 64; ++lane) {
+      const int k = 16 * mt + (lane & 15), q = lane >> 4;
+      if (k > Hc) continue;
+      for (int kt = 0; kt < Kc; ++kt) {
+        const int j = 4 * kt + q;
+        if (j <= Hc) h[((size_t)mt * Kc + kt) * 64 + lane] = (T)r[(size_t)((int64_t)j * k % L)].real();
+      }
+      for (int kt = 0; kt < Ks; ++kt) {
+        const int j = 1 + 4 * kt + q;
+        if (j <= Hs)
+          h[((size_t)Mt * Kc + (size_t)mt * Ks + kt) * 64 + lane] =
+              (T)(-r[(size_t)((int64_t)j * k % L)].imag());   // roots are exp(-2 pi i t / L)
+      }
+    }
+}
 
 template <typename T>
 static int upload_twiddles(int L, const FftPlan* plan, void** out) {
@@ -817,11 +867,15 @@ static int upload_twiddles(int L, const FftPlan* plan, void** out) {
         for (int k = 0; k < ns; ++k) put(q * k * step);
     }
   h.resize((size_t)L);
+  std::vector<T> dense;
+  if (plan && plan->variant == kDenseVariant) dense_table<T>(L, r, dense);
+  const void* src = dense.empty() ? (const void*)h.data() : (const void*)dense.data();
+  const size_t bytes = dense.empty() ? sizeof(cpx<T>) * (size_t)L : sizeof(T) * dense.size();
   void* p = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_capture_mu);
-    HIPCHK(dmalloc(&p, sizeof(cpx<T>) * (size_t)L));
-    const hipError_t e = hipMemcpy(p, h.data(), sizeof(cpx<T>) * (size_t)L, hipMemcpyHostToDevice);
+    HIPCHK(dmalloc(&p, bytes));
+    const hipError_t e = hipMemcpy(p, src, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
       dfree(p);
       return fail(CSIPM_ERR_HIP, "twiddle upload: %s", hipGetErrorString(e));
@@ -836,7 +890,7 @@ static int upload_twiddles(int L, const FftPlan* plan, void** out) {
       dup = p;            // another thread made the same table meanwhile
     } else {
       e.ptr = p;
-      e.bytes = sizeof(cpx<T>) * (size_t)L;
+      e.bytes = bytes;
       g_tw_key[p] = key;
     }
     hold(e, fresh);
@@ -913,8 +967,10 @@ static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size
   // below 64-byte rows only while the launch would not even give a
   // quarter of the workgroup target (small single instances: latency first)
   const int lg_min = std::min(lg, min_tile_lg(cs));
+  // (a dense tile takes as long for one line as for eight)
+  const int lg_end = plan.variant == kDenseVariant ? std::min(lg, 3) : 0;
   auto grid_of = [&](int l) { return (int64_t)((H1 + (1 << l) - 1) >> l) * others; };
-  while (lg > 0 && grid_of(lg) < min_grid && !(lg <= lg_min && 4 * grid_of(lg) >= min_grid))
+  while (lg > lg_end && grid_of(lg) < min_grid && !(lg <= lg_min && 4 * grid_of(lg) >= min_grid))
     --lg;
   c.lg = lg;
   c.ntile1 = (H1 + (1 << lg) - 1) >> lg;
@@ -969,7 +1025,8 @@ static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int m
   while (tile_grows(lg, plan, R, cs, mixed) && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
          lg < lg_cap)
     ++lg;
-  while (lg > 0 && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
+  const int lg_end = plan.variant == kDenseVariant ? std::min(lg, 3) : 0;
+  while (lg > lg_end && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
   c.lg = lg;
   c.ps = (1 << lg) + (lg > 0 ? 1 : 0);
   c.grid = (c.npairs + (1 << lg) - 1) >> lg;
@@ -1021,6 +1078,7 @@ PassArgs<T> base_args(csipm_op* h, int axis) {
   a.len = h->n[axis];
   a.bs = h->bs[axis];
   a.rperm = h->rperm[axis];
+  a.dense = (const T*)h->ps<T>().tw[axis];
   a.chirp = (const cpx<T>*)h->ps<T>().chirp[axis];
   a.bfw = (const cpx<T>*)h->ps<T>().bfw[axis];
   return a;
@@ -1136,26 +1194,34 @@ void set_steps(PassArgs<T>& a, const PassSpec& s, bool obs) {
 // one pass of one instance: grid tiles on workgroups sized nt (tile_nt)
 template <typename T>
 int launch_pass(csipm_op* h, const PassArgs<T>& a, int grid, int nt, size_t lds) {
-#define CSIPM_PASS(NT, E, LD, MID, ST)                                           \
+#define CSIPM_PASS(NT, E, LD, MID, ST, FORM) \
   do {                                                                           \
-    auto kern = k_pass<T, NT, E, LD, MID, ST>;                                   \
+    auto kern = k_pass<T, NT, E, LD, MID, ST, FORM>; \
     CHK(allow_lds(kern, lds));                                                   \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, h->stream, a);           \
     HIPCHK(hipGetLastError());                                                   \
     return CSIPM_OK;                                                             \
   } while (0)
 #define CSIPM_IS(LD, MID, ST) a.ld == LD && a.mid == MID && a.st == ST
+#define CSIPM_DENSE(LD, MID, ST) \
+  if (CSIPM_IS(LD, MID, ST)) CSIPM_PASS(256, kE, LD, MID, ST, FORM_DENSE);
+  if (a.bs == 3) {
+    CSIPM_DENSE_CHAIN(CSIPM_DENSE)
+    CSIPM_DENSE_ENTRY(CSIPM_DENSE)
+    return fail(CSIPM_ERR_UNSUPPORTED, "no dense kernel for pass (%d, %d, %d)", a.ld, a.mid, a.st);
+  }
+#undef CSIPM_DENSE
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
-    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST);      \
-    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
-    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
+    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST, FORM_FFT);      \
+    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST, FORM_FFT);      \
+    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST, FORM_FFT);      \
   }
 #define CSIPM_DIM1(LD, MID, ST)                           \
   CSIPM_SHORT(LD, MID, ST)                                \
   if (CSIPM_IS(LD, MID, ST)) {                            \
-    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST);    \
-    CSIPM_PASS(1024, 16, LD, MID, ST);                    \
+    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST, FORM_FFT);    \
+    CSIPM_PASS(1024, 16, LD, MID, ST, FORM_FFT);                    \
   }
   CSIPM_CHAIN_DIM1(CSIPM_DIM1)
   CSIPM_ENTRY_DIM1(CSIPM_DIM1)
@@ -2004,7 +2070,7 @@ static int plan_impl(csipm_op* h, int dim, const int64_t sizes[3], int rdft, int
   h->U = 2 * h->Nc;
   if (dim == 1 && h->n[0] > kBig1D) CHK(plan_big1d(h));
   for (int i = 0; i < dim && !h->big; ++i)
-    if (!plan_axis(h->n[i], h->plan[i], h->bs[i], h->rows[i]))
+    if (!plan_axis(h->n[i], dim == 1 ? 0 : h->N / h->n[i], h->plan[i], h->bs[i], h->rows[i]))
       return fail(CSIPM_ERR_UNSUPPORTED, "no FFT plan for size %d", h->n[i]);
   if (h->has64()) CHK(set_shapes(h, h->p64, sizeof(cpx<double>)));
   if (h->has32()) CHK(set_shapes(h, h->p32, sizeof(cpx<float>)));
@@ -2160,7 +2226,7 @@ int csipm_op_fft_shape(csipm_op_t h, int axis, int* fft_len, int* rows, int* mod
   }
   *fft_len = h->plan[axis].L;
   *rows = h->rows[axis];
-  *mode = h->bs[axis];
+  *mode = h->bs[axis] == 3 ? 4 : h->bs[axis];
   return CSIPM_OK;
 }
 

@@ -691,13 +691,17 @@ __host__ __device__ __forceinline__ cpx<T> u_map(cpx<T> w, int mode) {
   return {x, mode == 2 ? -y : y};
 }
 
-// u_map on the way into a pass, with one multiplication instead of the
-// division (as exact: the constant and the product are rounded once each)
+// u_map on the way into a pass, without its division: w / sqrt2 as w h + w l
+// with h + l the reciprocal of the rounded sqrt2 (the product alone would add
+// h's rounding to that of the sqrt2 on the way out, where the quotient's
+// cancels it: 5.7e-16 instead of 4.5e-16 off in M^T M of 1024 samples)
 template <typename T>
 __device__ __forceinline__ cpx<T> u_scale(cpx<T> w, int mode) {
   const T h = (T)0.70710678118654752440;
+  const T l = sizeof(T) == 8 ? (T)-9.667293313452912e-17 : (T)2.4203234416068298e-08;
   if (mode == 1) return {w.x, (T)0};
-  return {w.x * h, mode == 2 ? -(w.y * h) : w.y * h};
+  const T x = fma(w.x, l, w.x * h), y = fma(w.y, l, w.y * h);
+  return {x, mode == 2 ? -y : y};
 }
 
 // sqrt2 * v, v_to_u of a representative element (kept apart from any

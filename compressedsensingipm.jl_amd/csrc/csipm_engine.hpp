@@ -146,7 +146,8 @@ struct ChainSub {
   int pass = 0;          // position in the chains
   std::vector<int> ids;  // member instance ids
   bool side = false;     // only whole 1D lines of long transforms: independent of the rest
-  int ld = -1, mid = -1, st = -1;   // the members' steps, -1 when they differ
+  int ld = -1, mid = -1, st = -1;   // the members' steps, if they share them
+  int form = FORM_ANY;              // and their transform (FORM_ANY: they differ)
   int nt = kNT, grid = 0;
   size_t lds = 0;
   void* tab = nullptr;        // device PassArgs<T>[members] (in a table arena)
@@ -183,28 +184,40 @@ struct VsegOff {
 template <typename T>
 int launch_sub(const ChainSub& a, hipStream_t st) {
   const int nt = a.nt;
-#define CSIPM_PASS(NT, E, LD, MID, ST)                                                \
+#define CSIPM_PASS(NT, E, LD, MID, ST, FORM) \
   do {                                                                                \
-    auto kern = kb_pass<T, NT, E, LD, MID, ST>;                                       \
+    auto kern = kb_pass<T, NT, E, LD, MID, ST, FORM>; \
     CHK(allow_lds(kern, a.lds));                                                      \
     hipLaunchKernelGGL(kern, dim3(a.grid), dim3(NT), a.lds, st, (const PassArgs<T>*)a.tab, \
                        a.map);                                                        \
     HIPCHK(hipGetLastError());                                                        \
     return CSIPM_OK;                                                                  \
   } while (0)
+  if (a.form == FORM_ANY) {
+    if (nt == 256) CSIPM_PASS(256, kE, -1, -1, -1, FORM_ANY);
+    if (nt == 512) CSIPM_PASS(512, kE, -1, -1, -1, FORM_ANY);
+    if (nt == 1024) CSIPM_PASS(1024, kE, -1, -1, -1, FORM_ANY);
+    if (nt == kNTLong) CSIPM_PASS(1024, 16, -1, -1, -1, FORM_ANY);
+  }
+#define CSIPM_DENSE(LD, MID, ST) \
+  if (CSIPM_IS(LD, MID, ST)) CSIPM_PASS(256, kE, LD, MID, ST, FORM_DENSE);
+  if (a.form == FORM_DENSE) {
+    CSIPM_DENSE_CHAIN(CSIPM_DENSE)
+    return fail(CSIPM_ERR_UNSUPPORTED, "no dense kernel for pass (%d, %d, %d)", a.ld, a.mid, a.st);
+  }
+#undef CSIPM_DENSE
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
-    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST);      \
-    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST);      \
-    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST);      \
+    if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST, FORM_FFT);      \
+    if (nt == 256) CSIPM_PASS(256, kE, LD, MID, ST, FORM_FFT);      \
+    if (nt == 512) CSIPM_PASS(512, kE, LD, MID, ST, FORM_FFT);      \
   }
 #define CSIPM_DIM1(LD, MID, ST)                           \
   CSIPM_SHORT(LD, MID, ST)                                \
   if (CSIPM_IS(LD, MID, ST)) {                            \
-    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST);    \
-    CSIPM_PASS(1024, 16, LD, MID, ST);                    \
+    if (nt == 1024) CSIPM_PASS(1024, kE, LD, MID, ST, FORM_FFT);    \
+    CSIPM_PASS(1024, 16, LD, MID, ST, FORM_FFT);                    \
   }
-  CSIPM_DIM1(-1, -1, -1)
   CSIPM_CHAIN_DIM1(CSIPM_DIM1)
   CSIPM_CHAIN_SHORT(CSIPM_SHORT)
 #undef CSIPM_PASS
@@ -647,10 +660,15 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
         const PassSpec& s = m.specs[p];
         PassArgs<T> a{};
         CHK(chain_call_args<T>(E, m.id, call, nb, s, m.bc, a));
-        const bool same = tab.empty() || (sub.ld == a.ld && sub.mid == a.mid && sub.st == a.st);
-        sub.ld = same ? a.ld : -1;
-        sub.mid = same ? a.mid : -1;
-        sub.st = same ? a.st : -1;
+        const int form = a.bs == 3 ? FORM_DENSE : FORM_FFT;
+        if (tab.empty()) {
+          sub.ld = a.ld;
+          sub.mid = a.mid;
+          sub.st = a.st;
+          sub.form = form;
+        } else if (sub.ld != a.ld || sub.mid != a.mid || sub.st != a.st || sub.form != form) {
+          sub.form = FORM_ANY;
+        }
         tab.push_back(a);
         sub.ids.push_back(m.id);
         if (m.np > 1) sub.side = false;

@@ -440,12 +440,14 @@ struct PassArgs {
   const int* done;
   // line transform: length len; bs = 1 selects Bluestein's chirp-z form, in
   // which case plan is the convolution FFT of length M >= 2 len - 1; bs = 2
-  // selects Rader's form for a prime len, plan being the FFT of length len - 1
+  // selects Rader's form for a prime len, plan being the FFT of length len -
+  // 1; bs = 3 the dense form, dense its coefficients (see dense_dft)
   int len;
   int bs;
   const cpx<T>* chirp;  // w_n = exp(-i pi n^2 / len), n < len
   const cpx<T>* bfw;    // FFT_M(b) / M of the forward kernel b = conj(w) (wrapped);
                         // Rader: FFT_{L-1}(b) / (L-1) of b_j = exp(-2 pi i g^-j / L)
+  const T* dense;       // dense form: cosine, then sine tiles
   const int* rperm;     // Rader: [e] row of element e in the convolution order
                         // (e = 0: row L), [L + m] element g^-m mod L of output m
   // long 1D lines (four-step): the length-F transform (F = len, or the
@@ -455,6 +457,201 @@ struct PassArgs {
   uint32_t am;          // ceil(2^32 / A)
   const cpx<T>* twF;    // exp(-2 pi i j / F), j < F
 };
+
+// Dense form of the forward DFT for line lengths L <= 511 that no plan of the
+// radices covers, on the matrix cores: with H = L / 2 and, for j = 1 ..
+// (L - 1) / 2, a_j = x_j + x_{L-j} and b_j = x_j - x_{L-j} (a_0 = x_0, and
+// a_H = x_H when L is even),
+//   X_k = sum_j a_j cos(2 pi j k / L) - i sum_j b_j sin(2 pi j k / L),
+// X_{L-k} the same with + i: two real matrix products of about H x H with the
+// tile's 2 nl real columns.  a and b replace x in LDS rows j and L - j; a wave
+// takes output tiles of 16 k by 16 columns, eight accumulators each (C and S)
+// at most four at a time, and the outputs replace a and b when all waves have
+// read them.  The coefficients come packed in lane order, 64 to a 16 x 4 tile
+// (the wave reads them from the L2, one load feeding N products).
+// What bounds it: the matrix rate, L^2 / 128 cycles a line and CU in FP32 (L^2
+// / 64 in FP64) at 256 (128) operations a cycle.  Rader's and Bluestein's forms of
+// such lengths spent over a thousand cycles a line on two transforms and the
+// moves between, in twice the LDS rows: the operator product of 127^3 took 187
+// us in FP32 and 75 with this (185^3: 400 to 243, FP64 784 to 392).
+template <typename T>
+using Vec4 = T __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ Vec4<float> mfma16x16x4(float a, float b, Vec4<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ Vec4<double> mfma16x16x4(double a, double b, Vec4<double> c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// row of accumulator i in a 16 x 16 tile (column: lane & 15)
+template <typename T>
+__device__ __forceinline__ int mfma_row(int lane, int i) {
+  return sizeof(T) == 4 ? 4 * (lane >> 4) + i : (lane >> 4) + 4 * i;
+}
+// the value of lane ^ 1
+__device__ __forceinline__ float lane_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double lane_swap(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// tiles of the coefficient matrices: ceil((H + 1) / 16) by ceil((H + 1) / 4)
+// (cosine) and by ceil(((L - 1) / 2) / 4) (sine), the latter two made even
+// (zero tiles; their rows stay inside the line for L > 16)
+__host__ __device__ __forceinline__ int dense_mt(int L) { return (L / 2 + 16) / 16; }
+__host__ __device__ __forceinline__ int dense_kc(int L) { return (L / 2 + 8) / 8 * 2; }
+__host__ __device__ __forceinline__ int dense_ks(int L) { return ((L - 1) / 2 + 7) / 8 * 2; }
+
+// acc += coefficients (tile 0 at p[u], 64 entries a tile) x rows of x: tile kt
+// takes rows r0 + step * (4 kt + lane / 16); two tiles a turn, the next two
+// loaded before the products of these.  Chains that can be longer than 64 (U > 1) are
+// summed in parts of 32: one chain over the whole line rounds as often as it
+// has terms.  M^T M off by, FP32 / FP64: 127 x 127 (no parts) 3.1e-7 / 5.7e-16
+// (Rader's form 3.2e-7 / 7.2e-16); 509 x 2100 4.5e-7 / 8.3e-16 in one chain,
+// 2.5e-7 / 4.7e-16 in parts (Rader's 3.0e-7 / 7.1e-16)
+template <typename T, int U, int N>
+__device__ __forceinline__ void dense_product(Vec4<T> (&acc)[U][N], const T* const (&p)[U],
+                                              int tiles, const T* x, int r0, int step, int rs,
+                                              const int (&col)[N]) {
+  const int kk = ((int)threadIdx.x & 63) >> 4;
+  constexpr bool kParts = U > 1;
+  T q[2][U], qn[2][U];
+  Vec4<T> part[U][N];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int v = 0; v < N; ++v) part[u][v] = Vec4<T>{0, 0, 0, 0};
+    q[0][u] = p[u][0];
+    q[1][u] = p[u][64];
+  }
+#pragma unroll 1
+  for (int kt = 0; kt < tiles; kt += 2) {
+    const int nx = min(kt + 2, tiles - 2) * 64;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      qn[0][u] = p[u][nx];
+      qn[1][u] = p[u][nx + 64];
+    }
+    T b[2][N];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int v = 0; v < N; ++v) b[h][v] = x[(r0 + step * (4 * (kt + h) + kk)) * rs + col[v]];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+          Vec4<T>& r = kParts ? part[u][v] : acc[u][v];
+          r = mfma16x16x4(q[h][u], b[h][v], r);
+        }
+    if (kParts && ((kt & 6) == 6 || kt + 2 >= tiles)) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+          acc[u][v] += part[u][v];
+          part[u][v] = Vec4<T>{0, 0, 0, 0};
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      q[0][u] = qn[0][u];
+      q[1][u] = qn[1][u];
+    }
+  }
+}
+
+// U k-tiles of a wave (k-tile wave + u NT / 64) by N column tiles
+template <typename T, int NT, int U, int N>
+__device__ __forceinline__ void dense_tiles(cpx<T>* lds, const T* __restrict__ coef, int L,
+                                            int cols, int rs) {
+  constexpr int W = NT / 64;
+  const int wave = uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  const int n = lane & 15;
+  const int Mt = dense_mt(L), Kc = dense_kc(L), Ks = dense_ks(L);
+  T* x = reinterpret_cast<T*>(lds);
+  Vec4<T> c[U][N], s[U][N];
+  const T* ac[U];
+  const T* as[U];
+  int col[N];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int mt = min(wave + u * W, Mt - 1);   // tiles past the last: repeated, not stored
+    ac[u] = coef + (int64_t)mt * Kc * 64 + lane;
+    as[u] = coef + ((int64_t)Mt * Kc + (int64_t)mt * Ks) * 64 + lane;
+#pragma unroll
+    for (int v = 0; v < N; ++v) c[u][v] = s[u][v] = Vec4<T>{0, 0, 0, 0};
+  }
+#pragma unroll
+  for (int v = 0; v < N; ++v) col[v] = min(n + 16 * v, cols - 1);
+  // columns of the cosine matrix: a_j in row j; rows past H hold other finite
+  // values of the same column and meet zero coefficients.  Of the sine
+  // matrix: b_j in row L - j
+  dense_product<T, U, N>(c, ac, Kc, x, 0, 1, rs, col);
+  dense_product<T, U, N>(s, as, Ks, x, L - 1, -1, rs, col);
+  __syncthreads();
+  const bool im = n & 1;   // column pairs hold real and imaginary parts
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int mt = wave + u * W;
+#pragma unroll
+    for (int v = 0; v < N; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const T other = lane_swap(s[u][v][i]);
+        const T plus = c[u][v][i] + other, minus = c[u][v][i] - other;
+        const int k = 16 * mt + mfma_row<T>(lane, i);
+        if (mt < Mt && k <= L / 2 && n + 16 * v < cols) {
+          x[k * rs + col[v]] = im ? minus : plus;
+          if (k > 0 && 2 * k != L) x[(L - k) * rs + col[v]] = im ? plus : minus;
+        }
+      }
+  }
+  __syncthreads();
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void dense_dft(cpx<T>* lds, const T* __restrict__ coef, int L,
+                                          int lg, int ps) {
+  const int nl = 1 << lg;
+  for (int idx = threadIdx.x; idx < ((L - 1) / 2) << lg; idx += NT) {
+    const int line = idx & (nl - 1), j = 1 + (idx >> lg);
+    cpx<T>*p = lds + j * ps + line, *q = lds + (L - j) * ps + line;
+    const cpx<T> x = *p, y = *q;
+    *p = cadd(x, y);
+    *q = csub(x, y);
+  }
+  __syncthreads();
+  const int cols = 2 << lg, rs = 2 * ps;
+  const int u = (dense_mt(L) + NT / 64 - 1) / (NT / 64);
+  if (u == 1) {
+    if (lg <= 3) dense_tiles<T, NT, 1, 1>(lds, coef, L, cols, rs);
+    else if (lg == 4) dense_tiles<T, NT, 1, 2>(lds, coef, L, cols, rs);
+    else dense_tiles<T, NT, 1, 4>(lds, coef, L, cols, rs);
+  } else if (u == 2) {
+    if (lg <= 3) dense_tiles<T, NT, 2, 1>(lds, coef, L, cols, rs);
+    else dense_tiles<T, NT, 2, 2>(lds, coef, L, cols, rs);
+  } else if (u == 3) {
+    dense_tiles<T, NT, 3, 1>(lds, coef, L, cols, rs);
+  } else {
+    dense_tiles<T, NT, 4, 1>(lds, coef, L, cols, rs);
+  }
+}
+
+// the same as a call, for the kernels of mixed launches: its registers are
+// not added to those of their other steps (a mixed launch of 48 requests, FP32,
+// 256 threads: inlined 31.5 us and 31 of 128 registers spilled, called 28.0)
+template <typename T>
+using LdsTile = __attribute__((address_space(3))) cpx<T>*;
+template <typename T, int NT>
+__device__ __noinline__ void dense_dft_call(LdsTile<T> lds, const T* coef, int L, int lg, int ps) {
+  dense_dft<T, NT>((cpx<T>*)lds, coef, L, lg, ps);
+}
 
 // Forward DFT of length a.len of the 2^lg lines in LDS ([element][line],
 // stride ps), in place.  Direct: the Stockham plan.  Bluestein (lengths with a
@@ -1266,8 +1463,12 @@ __device__ __forceinline__ void row_store(const PassArgs<T>& a, cpx<T>* lds, int
   }
 }
 
-// one workgroup's tile of a pass; LD, MID, ST < 0: the steps PassArgs names
-template <typename T, int NT, int E, int LD, int MID, int ST>
+// one workgroup's tile of a pass; LD, MID, ST < 0: the steps PassArgs names.
+// FORM: the line transforms it is compiled for, FORM_FFT (direct, Rader,
+// Bluestein), FORM_DENSE or any (together they take more registers: the FP32
+// 256^3 product 357 against 374 us)
+enum { FORM_FFT = 0, FORM_DENSE = 1, FORM_ANY = 2 };
+template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
 __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
   const int ld = LD < 0 ? a.ld : LD, mid = MID < 0 ? a.mid : MID, st = ST < 0 ? a.st : ST;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -1307,10 +1508,20 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
   __syncthreads();
 #pragma unroll 1
   for (int turn = 0;; ++turn) {
-    if constexpr (LD >= LD_COL_FIRST_U)   // four-step passes transform directly
+    if constexpr (LD >= LD_COL_FIRST_U) {   // four-step passes transform directly
       lds_fft<T, E, NT>(lds, pl, a.lg, a.ps, a.tw);
-    else
-      line_dft<T, E, NT>(lds, a, pl, a.lg, a.ps);
+    } else if constexpr (FORM == FORM_DENSE) {
+      dense_dft<T, NT>(lds, a.dense, a.len, a.lg, a.ps);
+    } else {
+      bool fft = true;
+      if constexpr (FORM == FORM_ANY && NT == 256) {   // (dense tiles run on 256 threads)
+        if (a.bs == 3) {
+          dense_dft_call<T, NT>((LdsTile<T>)lds, a.dense, a.len, a.lg, a.ps);
+          fft = false;
+        }
+      }
+      if (fft) line_dft<T, E, NT>(lds, a, pl, a.lg, a.ps);
+    }
     if (turn == 1 || mid == MID_NONE) break;
     switch (mid) {
       case MID_DIM1_MASK: dim1_mask<T, NT, false>(a, lds, mw, tile); break;
@@ -1358,9 +1569,9 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
 }
 
 // a pass of one instance
-template <typename T, int NT, int E, int LD, int MID, int ST>
+template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
 __global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_pass(PassArgs<T> a) {
-  pass_body<T, NT, E, LD, MID, ST>(a, xcd_block());
+  pass_body<T, NT, E, LD, MID, ST, FORM>(a, xcd_block());
 }
 
 // member and tile of a block of a launch over several instances; member < 0:
@@ -1370,14 +1581,16 @@ struct BlockMap {
 };
 
 // passes of several instances (LD < 0: each its own kind): the host's block map keeps
-// adjacent tiles of an instance on one XCD (block b runs on XCD b % 8)
-template <typename T, int NT, int E, int LD, int MID, int ST>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void kb_pass(
+// adjacent tiles of an instance on one XCD (block b runs on XCD b % 8).  The
+// mixed FP32 ones keep four waves a SIMD instead of five: 70 registers of their
+// many steps spilled at 96, none at 128 (512 threads: 39.2 to 36.0 us)
+template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
+__global__ __launch_bounds__(NT, (LD < 0 && sizeof(T) == 4 ? 4 : pass_waves<T, NT>())) void kb_pass(
     const PassArgs<T>* __restrict__ tab, const BlockMap* __restrict__ map) {
   const int i = uniform(map[blockIdx.x].member), tile = uniform(map[blockIdx.x].tile);
   if (i < 0) return;
   const PassArgs<T> a = tab[i];  // loaded before any store: stays in scalar registers
-  pass_body<T, NT, E, LD, MID, ST>(a, tile);
+  pass_body<T, NT, E, LD, MID, ST, FORM>(a, tile);
 }
 
 // beta <-> u (exact: a signed permutation), one thread per half-spectrum element.

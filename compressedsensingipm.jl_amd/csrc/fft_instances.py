@@ -50,15 +50,22 @@ ENTRY_DIM1 = [
 NT_SHORT = ["128 8", "256 8", "512 8"]
 NT_LONG = ["1024 8", "1024 16"]
 MIXED = "-1 -1 -1"
+# of these, the passes of 2D / 3D axes in the dense form (256 threads)
+DENSE_CHAIN = [s for s in CHAIN_SHORT if "LINES" in s] + CHAIN_DIM1[1:2] + CHAIN_DIM1[3:]
+DENSE_ENTRY = [s for s in ENTRY_SHORT if "LINES" in s] + ENTRY_DIM1[2:3]
 
 
 def instances():
-    def rows(nts, steps):
-        return [f"{n} {s}" for n in nts for s in steps]
+    def rows(nts, steps, form="FORM_FFT"):
+        return [f"{n} {s} {form}" for n in nts for s in steps]
+    dense = NT_SHORT[1:2]
     table = {
         "k_pass": rows(NT_SHORT + NT_LONG, CHAIN_DIM1 + ENTRY_DIM1) +
-        rows(NT_SHORT, CHAIN_SHORT + ENTRY_SHORT),
-        "kb_pass": rows(NT_SHORT + NT_LONG, CHAIN_DIM1 + [MIXED]) + rows(NT_SHORT, CHAIN_SHORT),
+        rows(NT_SHORT, CHAIN_SHORT + ENTRY_SHORT) +
+        rows(dense, DENSE_CHAIN + DENSE_ENTRY, "FORM_DENSE"),
+        "kb_pass": rows(NT_SHORT + NT_LONG, CHAIN_DIM1) + rows(NT_SHORT, CHAIN_SHORT) +
+        rows(dense, DENSE_CHAIN, "FORM_DENSE") +
+        rows(NT_SHORT[1:] + NT_LONG, [MIXED], "FORM_ANY"),
     }
     out = []
     for t in ("float", "double"):
@@ -74,7 +81,8 @@ def write(outdir, nunits):
     ext = ["// generated by fft_instances.py"]
     # the steps as X-macros, for the host's dispatch
     for name, steps in (("CHAIN_SHORT", CHAIN_SHORT), ("CHAIN_DIM1", CHAIN_DIM1),
-                        ("ENTRY_SHORT", ENTRY_SHORT), ("ENTRY_DIM1", ENTRY_DIM1)):
+                        ("ENTRY_SHORT", ENTRY_SHORT), ("ENTRY_DIM1", ENTRY_DIM1),
+                        ("DENSE_CHAIN", DENSE_CHAIN), ("DENSE_ENTRY", DENSE_ENTRY)):
         ext += [f"#define CSIPM_{name}(X) " +
                 " ".join("X(" + ", ".join(s.split()) + ")" for s in steps)]
     ext += ["namespace csipm {"]

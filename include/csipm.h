@@ -120,7 +120,8 @@ int csipm_op_info(csipm_op_t h, int64_t* n, int64_t* nc, int* precision);
 /* The line transform of axis `axis` (0-based) of h: FFT length (the line
  * length; Bluestein's convolution length; L - 1 for Rader's form; the
  * four-step length of long 1D lines), LDS rows per line, and the form
- * (0 direct, 1 Bluestein, 2 Rader, 3 four-step).  No counterpart in the
+ * (0 direct, 1 Bluestein, 2 Rader, 3 four-step, 4 dense: a 2D/3D axis of up
+ * to 511 that does not factor, unless csipm_tune_bluestein names it).  No counterpart in the
  * reference (rocFFT/FFTW plans are opaque there); the autotuner keys its
  * table on (FFT length, rows).                                            */
 int csipm_op_fft_shape(csipm_op_t h, int axis, int* fft_len, int* rows, int* mode);

@@ -240,3 +240,27 @@ def test_workgroup_sizes(cuda, dims, dtype):
     assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
     assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
     assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
+
+
+# axes of lengths the radices do not cover, as dense products on the matrix
+# cores: one to four blocks of output rows a wave (up to 126, 127..254 and on),
+# odd and even, primes and not, both sides of 256 (above it only where the
+# other axes give 2048 lines), few lines and many, the longest
+@pytest.mark.parametrize("dims", [(37, 3), (2, 41), (62, 74), (5, 126, 2), (127, 33), (128, 127),
+                                  (3, 129, 2), (254, 74), (253, 2, 3), (2, 3, 251), (43, 47, 53),
+                                  (257, 33), (4, 262, 1100), (383, 2300), (2100, 386),
+                                  (509, 4000), (6, 800, 511)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_dense_lengths(cuda, dims, dtype):
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("dense", dims, dtype, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 7)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    tol = TOL64 if dtype == torch.float64 else TOL32
+    o = _make(dims, miss, dtype)
+    xt = torch.from_numpy(x).to(cuda, dtype)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
