@@ -591,14 +591,6 @@ __device__ __forceinline__ void stockham_stage(cpx<T>* __restrict__ lds, int L, 
   __syncthreads();
 }
 
-// waves per SIMD asked of the compiler for the pass kernels (of 512 registers
-// a SIMD lane: 96 per thread in FP32, 168 in FP64; a 1024-thread workgroup
-// needs four waves, 128 registers)
-template <typename T, int NT>
-constexpr int pass_waves() {
-  return NT >= 1024 ? 4 : sizeof(T) == 4 ? 5 : 3;
-}
-
 // forward DFT of the tile; pl: the wave's plan register (plan_load)
 template <typename T, int E, int NT>
 __device__ __forceinline__ void lds_fft(cpx<T>* lds, int pl, int lg, int ps,

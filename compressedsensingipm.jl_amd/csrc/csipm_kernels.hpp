@@ -1568,9 +1568,20 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
   if (a.epi.dot_part) store_partial(a.epi.dot_part, acc, tile);
 }
 
+// waves per SIMD asked of the compiler for the pass kernels (of 512 registers
+// a SIMD lane: 96 per thread in FP32, 168 in FP64; a 1024-thread workgroup
+// needs four waves, 128 registers).  The dense and the mixed FP32 ones keep
+// four as well, nothing spilled at 128 registers: a mixed launch of 512 threads
+// 39.2 to 36.0 us (70 spilled at 96), the dense product of 127^3 80 to 77
+template <typename T, int NT, int LD, int FORM>
+constexpr int pass_waves() {
+  if (NT >= 1024 || (sizeof(T) == 4 && (LD < 0 || FORM == FORM_DENSE))) return 4;
+  return sizeof(T) == 4 ? 5 : 3;
+}
+
 // a pass of one instance
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT>())) void k_pass(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT, LD, FORM>())) void k_pass(PassArgs<T> a) {
   pass_body<T, NT, E, LD, MID, ST, FORM>(a, xcd_block());
 }
 
@@ -1581,11 +1592,9 @@ struct BlockMap {
 };
 
 // passes of several instances (LD < 0: each its own kind): the host's block map keeps
-// adjacent tiles of an instance on one XCD (block b runs on XCD b % 8).  The
-// mixed FP32 ones keep four waves a SIMD instead of five: 70 registers of their
-// many steps spilled at 96, none at 128 (512 threads: 39.2 to 36.0 us)
+// adjacent tiles of an instance on one XCD (block b runs on XCD b % 8).
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
-__global__ __launch_bounds__(NT, (LD < 0 && sizeof(T) == 4 ? 4 : pass_waves<T, NT>())) void kb_pass(
+__global__ __launch_bounds__(NT, (pass_waves<T, NT, LD, FORM>())) void kb_pass(
     const PassArgs<T>* __restrict__ tab, const BlockMap* __restrict__ map) {
   const int i = uniform(map[blockIdx.x].member), tile = uniform(map[blockIdx.x].tile);
   if (i < 0) return;
