@@ -72,7 +72,9 @@ __device__ __forceinline__ void bstore_partials(double* part, const double (&acc
 // nb = 1: reduced system, diagonal preconditioner P11.
 // ===========================================================================
 struct CgState {
-  double gamma;
+  double gamma;   // r'z before the residual update, for the kernel that takes p on
+  double gnew;    // r'z now; moved to gamma by the update that first reads it (a
+                  // launch never writes the one that its workgroups read)
   double pq;
   double alpha;
   double beta;
@@ -166,6 +168,7 @@ __global__ void bk_cg_start(BSeg vseg, const int* ids, const BInst* __restrict__
   if (threadIdx.x == 0) {
     CgState& st = cg[inst];
     st.gamma = g;
+    st.gnew = g;
     st.rnorm = sqrt(g > 0 ? g : 0.0);
     st.eps = atol + rtol * sqrt(gb > 0 ? gb : 0.0);
     st.iters = 0;
@@ -182,24 +185,56 @@ __global__ void bk_cg_start(BSeg vseg, const int* ids, const BInst* __restrict__
   }
 }
 
+// slots of a thread whose operands the two vector kernels below load before
+// they wait for the sums: all of them up to 2M slots (vblocks() gives a
+// workgroup of 256 threads 1024)
+constexpr int kCgSlots = 4;
+
 // after q = K p (its last pass left gcg partials of p'q): alpha = gamma / p'q
 // (every workgroup sums the apply's p'q partials itself,
 // in the same order, so all agree; the first one records it and a zero
 // curvature), then x += alpha p; r -= alpha q; z = P r; partial r'z at
-// pbase + gcg, beside the p'q partials other workgroups are still reading
-template <typename T>
+// pbase + gcg, beside the p'q partials other workgroups are still reading.
+// The loads of a thread's slots go out together and ahead of the sum: one
+// after another they bound the kernel in small problems (255 x 255 FP64 6.8 us before,
+// 5.6 now; 48 mixed requests FP32 17.0 and 14.8)
+template <typename T, int NB>
 __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __restrict__ info,
-                                                    CgState* cg, T* x, T* r, T* z,
+                                                    CgState* cg, T* __restrict__ x,
+                                                    T* __restrict__ r, T* __restrict__ z,
                                                     const T* __restrict__ p,
                                                     const T* __restrict__ q,
                                                     const T* __restrict__ P11,
                                                     const T* __restrict__ P12,
-                                                    const T* __restrict__ P22, int nb,
-                                                    double* part) {
+                                                    const T* __restrict__ P22, double* part) {
   const BFlags* flags = nullptr;
   BSEG_BEGIN
   CgState& st = cg[inst];
   if (st.done) return;
+  const int64_t step = (int64_t)nbk * blockDim.x, end = I.off + I.n;
+  int64_t i0 = I.off + (int64_t)lb * blockDim.x + threadIdx.x;
+  T xv[kCgSlots][NB], rv[kCgSlots][NB], pv[kCgSlots][NB], qv[kCgSlots][NB], d[kCgSlots][2 * NB - 1];
+  auto load = [&]() {
+#pragma unroll
+    for (int k = 0; k < kCgSlots; ++k) {
+      const int64_t i = i0 + k * step;
+      if (i >= end) continue;
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        const int64_t j = i + I.off + c * I.n;
+        xv[k][c] = x[j];
+        rv[k][c] = r[j];
+        pv[k][c] = p[j];
+        qv[k][c] = q[j];
+      }
+      d[k][0] = P11[i];
+      if constexpr (NB == 2) {
+        d[k][1] = P12[i];
+        d[k][2] = P22[i];
+      }
+    }
+  };
+  load();
   __shared__ double s_pq;
   const double pq0 = sum_partials(part + I.pbase, I.gcg);
   if (threadIdx.x == 0) s_pq = pq0;
@@ -213,41 +248,48 @@ __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __res
     }
     return;
   }
-  const double ad = st.gamma / pq;
+  const double ad = st.gnew / pq;
   if (lb == 0 && threadIdx.x == 0) {
     st.pq = pq;
     st.alpha = ad;
+    st.gamma = st.gnew;
   }
   const T alpha = (T)ad;
   double acc = 0.0;
-  BFOR(i) {
-    const int64_t j = i + I.off;
-    if (nb == 1) {
-      x[j] += alpha * p[j];
-      const T rb = r[j] - alpha * q[j];
-      const T zb = P11[i] * rb;
-      r[j] = rb;
-      z[j] = zb;
-      acc += (double)rb * zb;
-      continue;
+  while (true) {
+#pragma unroll
+    for (int k = 0; k < kCgSlots; ++k) {
+      const int64_t i = i0 + k * step;
+      if (i >= end) continue;
+      const int64_t j = i + I.off;
+      T rb[NB], zb[NB];
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        x[j + c * I.n] = xv[k][c] + alpha * pv[k][c];
+        rb[c] = rv[k][c] - alpha * qv[k][c];
+        r[j + c * I.n] = rb[c];
+      }
+      if constexpr (NB == 1) {
+        zb[0] = d[k][0] * rb[0];
+        z[j] = zb[0];
+        acc += (double)rb[0] * zb[0];
+      } else {
+        zb[0] = d[k][0] * rb[0] + d[k][1] * rb[1];
+        zb[1] = d[k][1] * rb[0] + d[k][2] * rb[1];
+        z[j] = zb[0];
+        z[j + I.n] = zb[1];
+        acc += (double)rb[0] * zb[0] + (double)rb[1] * zb[1];
+      }
     }
-    const int64_t k = j + I.n;
-    x[j] += alpha * p[j];
-    x[k] += alpha * p[k];
-    const T rb = r[j] - alpha * q[j];
-    const T rz = r[k] - alpha * q[k];
-    r[j] = rb;
-    r[k] = rz;
-    const T zb = P11[i] * rb + P12[i] * rz;
-    const T zz = P12[i] * rb + P22[i] * rz;
-    z[j] = zb;
-    z[k] = zz;
-    acc += (double)rb * zb + (double)rz * zz;
+    i0 += kCgSlots * step;
+    if (i0 >= end) break;
+    load();
   }
   store_partial(part + I.pbase + I.gcg, acc, lb);
 }
 
-// gamma <- r'z, beta = gamma_new / gamma_old, stopping tests
+// r'z after an update that a true residual follows (the other iterations take
+// it in bk_cg_pupdate): beta = gamma_new / gamma_old, stopping tests
 __global__ void bk_cg_gamma(BSeg vseg, const int* ids, const BInst* __restrict__ info,
                             CgState* cg, const double* part) {
   const int inst = ids[blockIdx.x];
@@ -260,7 +302,7 @@ __global__ void bk_cg_gamma(BSeg vseg, const int* ids, const BInst* __restrict__
     st.iters += 1;
     st.rnorm = sqrt(g > 0 ? g : 0.0);
     st.beta = g / st.gamma;
-    st.gamma = g;
+    st.gnew = g;
     if (st.rnorm <= st.eps) {
       st.done = 1;
       st.status = 0;
@@ -318,7 +360,7 @@ __global__ void bk_cg_regamma(BSeg vseg, const int* ids, const BInst* __restrict
   const double g = sum_partials(part + I.pbase, vseg.first[inst + 1] - vseg.first[inst]);
   if (threadIdx.x == 0) {
     st.rnorm = sqrt(g > 0 ? g : 0.0);
-    st.gamma = g;
+    st.gnew = g;
     st.beta = 0.0;
     if (st.rnorm <= st.eps) {
       st.done = 1;
@@ -327,19 +369,73 @@ __global__ void bk_cg_regamma(BSeg vseg, const int* ids, const BInst* __restrict
   }
 }
 
-// p = z + beta p
-template <typename T>
+// p = z + beta p.  SUM: beta = gamma_new / gamma_old from the update's partial
+// sums of r'z, which every workgroup adds itself in the same order; the first
+// one records it and the stopping tests (a workgroup that starts later may see
+// done: it leaves a p that nothing reads).  Otherwise beta as bk_cg_regamma
+// left it.
+// (A kernel of its own for the sum took 4.0 us of the 44 of an iteration of
+// 255 x 255 in FP64, a launch and a round trip; p's kernel 4.0 and, with the
+// sum, 4.9.)
+template <typename T, bool SUM>
 __global__ __launch_bounds__(256) void bk_cg_pupdate(BSeg seg, const BInst* __restrict__ info,
-                                                     const CgState* cg, T* p,
-                                                     const T* __restrict__ z, int nb) {
+                                                     CgState* cg, T* __restrict__ p,
+                                                     const T* __restrict__ z, int nb,
+                                                     const double* __restrict__ part) {
   const BFlags* flags = nullptr;
   BSEG_BEGIN
-  if (cg[inst].done) return;
-  const T beta = (T)cg[inst].beta;
-  BFOR(i) {
-    const int64_t j = i + I.off;
-    p[j] = z[j] + beta * p[j];
-    if (nb == 2) p[j + I.n] = z[j + I.n] + beta * p[j + I.n];
+  CgState& st = cg[inst];
+  if (st.done) return;
+  const int64_t n = nb * I.n, step = (int64_t)nbk * blockDim.x;
+  const T* zi = z + 2 * I.off;
+  T* pi = p + 2 * I.off;
+  int64_t i0 = (int64_t)lb * blockDim.x + threadIdx.x;
+  constexpr int K = 2 * kCgSlots;
+  T zv[K], pv[K];
+  auto load = [&]() {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t i = i0 + k * step;
+      if (i < n) {
+        zv[k] = zi[i];
+        pv[k] = pi[i];
+      }
+    }
+  };
+  load();
+  T beta;
+  if constexpr (SUM) {
+    __shared__ double s_g;
+    const double g0 = sum_partials(part + I.pbase + I.gcg, nbk);
+    if (threadIdx.x == 0) s_g = g0;
+    __syncthreads();
+    const double g = s_g, bd = g / st.gamma;
+    beta = (T)bd;
+    if (lb == 0 && threadIdx.x == 0) {
+      st.iters += 1;
+      st.rnorm = sqrt(g > 0 ? g : 0.0);
+      st.beta = bd;
+      st.gnew = g;
+      if (st.rnorm <= st.eps) {
+        st.done = 1;
+        st.status = 0;
+      } else if (st.iters >= st.itmax) {
+        st.done = 1;
+        st.status = 1;
+      }
+    }
+  } else {
+    beta = (T)st.beta;
+  }
+  while (true) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t i = i0 + k * step;
+      if (i < n) pi[i] = zv[k] + beta * pv[k];
+    }
+    i0 += K * step;
+    if (i0 >= n) break;
+    load();
   }
 }
 

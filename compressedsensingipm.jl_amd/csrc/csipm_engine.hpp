@@ -955,19 +955,21 @@ int cg_iteration(Engine* E, int nb, bool reliable) {
   TC *P11 = E->C<TC>(C_P11), *P12 = E->C<TC>(C_P12), *P22 = E->C<TC>(C_P22);
   hipStream_t st = E->stream;
   CHK(run_chain<TC>(E->chains[CALL_CGA], st, E->side, E->fork_ev, E->join_ev));
-  hipLaunchKernelGGL((bk_cg_update<TC>), dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info,
-                     E->cg, x, r, z, p, q, P11, P12, P22, nb, E->part);
-  hipLaunchKernelGGL(bk_cg_gamma, dim3(na), dim3(kNT), 0, st, E->vseg, E->ids, E->info, E->cg,
-                     E->part);
+  auto update = nb == 1 ? bk_cg_update<TC, 1> : bk_cg_update<TC, 2>;
+  hipLaunchKernelGGL(update, dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info, E->cg, x, r, z, p,
+                     q, P11, P12, P22, E->part);
   if (reliable) {
+    hipLaunchKernelGGL(bk_cg_gamma, dim3(na), dim3(kNT), 0, st, E->vseg, E->ids, E->info, E->cg,
+                       E->part);
     CHK(run_chain<TC>(E->chains[CALL_CGR], st, E->side, E->fork_ev, E->join_ev));
     hipLaunchKernelGGL((bk_cg_residual<TC>), dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info,
                        E->cg, b, q, r, z, P11, P12, P22, nb, E->part);
     hipLaunchKernelGGL(bk_cg_regamma, dim3(na), dim3(kNT), 0, st, E->vseg, E->ids, E->info,
                        E->cg, E->part);
   }
-  hipLaunchKernelGGL((bk_cg_pupdate<TC>), dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info,
-                     E->cg, p, z, nb);
+  auto pupdate = reliable ? bk_cg_pupdate<TC, false> : bk_cg_pupdate<TC, true>;
+  hipLaunchKernelGGL(pupdate, dim3(E->vgrid), dim3(kNT), 0, st, E->vseg, E->info, E->cg, p, z, nb,
+                     E->part);
   HIPCHK(hipGetLastError());
   return CSIPM_OK;
 }
