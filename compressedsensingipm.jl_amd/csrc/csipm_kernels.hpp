@@ -1572,10 +1572,12 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
 // a SIMD lane: 96 per thread in FP32, 168 in FP64; a 1024-thread workgroup
 // needs four waves, 128 registers).  The dense and the mixed FP32 ones keep
 // four as well, nothing spilled at 128 registers: a mixed launch of 512 threads
-// 39.2 to 36.0 us (70 spilled at 96), the dense product of 127^3 80 to 77
+// 39.2 to 36.0 us (70 spilled at 96), the dense product of 127^3 80 to 77.
+// The mixed FP64 ones two (256 threads 82 to 73 us; 106 spilled at 168)
 template <typename T, int NT, int LD, int FORM>
 constexpr int pass_waves() {
   if (NT >= 1024 || (sizeof(T) == 4 && (LD < 0 || FORM == FORM_DENSE))) return 4;
+  if (LD < 0) return 2;
   return sizeof(T) == 4 ? 5 : 3;
 }
 
