@@ -420,12 +420,12 @@ struct PassArgs {
   MapGeom g;
   const FftPlan* plan;  // device-resident
   const cpx<T>* tw;     // the plan's twiddles, stage by stage
-  int axis;      // k_lines: 1 or 2
+  int axis;      // line passes: 1 or 2
   int H1;
   int lg;        // log2 of lines (pairs) per workgroup
   int ps;        // LDS line stride
-  int ntile1;    // k_lines: tiles along k1
-  int nlines;    // k_dim1: real lines N2*N3
+  int ntile1;    // line passes: tiles along k1
+  int nlines;    // dimension 1: real lines N2*N3
   int npairs;
   uint32_t h1m;  // ceil(2^32 / H1)
   uint32_t n1m;  // ceil(2^32 / N1)
@@ -507,17 +507,18 @@ __host__ __device__ __forceinline__ int dense_ks(int L) { return ((L - 1) / 2 + 
 
 // acc += coefficients (tile 0 at p[u], 64 entries a tile) x rows of x: tile kt
 // takes rows r0 + step * (4 kt + lane / 16); two tiles a turn, the next two
-// loaded before the products of these.  Chains that can be longer than 64 (U > 1) are
-// summed in parts of 32: one chain over the whole line rounds as often as it
-// has terms.  M^T M off by, FP32 / FP64: 127 x 127 (no parts) 3.1e-7 / 5.7e-16
-// (Rader's form 3.2e-7 / 7.2e-16); 509 x 2100 4.5e-7 / 8.3e-16 in one chain,
-// 2.5e-7 / 4.7e-16 in parts (Rader's 3.0e-7 / 7.1e-16)
+// loaded before the products of these.  The products are summed in parts of 8
+// (lines up to 127, U = 1) or 32: one chain over the whole line rounds as often
+// as it has terms.  M^T M off by, FP32 / FP64: 127 x 127 in one chain 3.1e-7 /
+// 5.7e-16, in parts of 8 2.0e-7 / 3.6e-16 (Rader's form 3.2e-7 / 7.2e-16, the
+// radix plan of 116 x 124 2.1e-7 / 3.9e-16); 509 x 2100 4.5e-7 / 8.3e-16 in one
+// chain, 2.5e-7 / 4.7e-16 in parts of 32 (Rader's 3.0e-7 / 7.1e-16; parts of 8
+// took 185^3 in FP64 from 406 to 432 us)
 template <typename T, int U, int N>
 __device__ __forceinline__ void dense_product(Vec4<T> (&acc)[U][N], const T* const (&p)[U],
                                               int tiles, const T* x, int r0, int step, int rs,
                                               const int (&col)[N]) {
   const int kk = ((int)threadIdx.x & 63) >> 4;
-  constexpr bool kParts = U > 1;
   T q[2][U], qn[2][U];
   Vec4<T> part[U][N];
 #pragma unroll
@@ -545,11 +546,8 @@ __device__ __forceinline__ void dense_product(Vec4<T> (&acc)[U][N], const T* con
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int v = 0; v < N; ++v) {
-          Vec4<T>& r = kParts ? part[u][v] : acc[u][v];
-          r = mfma16x16x4(q[h][u], b[h][v], r);
-        }
-    if (kParts && ((kt & 6) == 6 || kt + 2 >= tiles)) {
+        for (int v = 0; v < N; ++v) part[u][v] = mfma16x16x4(q[h][u], b[h][v], part[u][v]);
+    if (U == 1 || (kt & 6) == 6 || kt + 2 >= tiles) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll

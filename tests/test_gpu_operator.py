@@ -245,11 +245,12 @@ def test_workgroup_sizes(cuda, dims, dtype):
 # axes of lengths the radices do not cover, as dense products on the matrix
 # cores: one to four blocks of output rows a wave (up to 126, 127..254 and on),
 # odd and even, primes and not, both sides of 256 (above it only where the
-# other axes give 2048 lines), few lines and many, the longest
+# other axes give 2048 lines), few lines and many, the longest, and the short
+# ones with a factor 29 or 31
 @pytest.mark.parametrize("dims", [(37, 3), (2, 41), (62, 74), (5, 126, 2), (127, 33), (128, 127),
                                   (3, 129, 2), (254, 74), (253, 2, 3), (2, 3, 251), (43, 47, 53),
                                   (257, 33), (4, 262, 1100), (383, 2300), (2100, 386),
-                                  (509, 4000), (6, 800, 511)])
+                                  (509, 4000), (6, 800, 511), (58, 93), (124, 3, 87), (2, 116)])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_dense_lengths(cuda, dims, dtype):
     from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
