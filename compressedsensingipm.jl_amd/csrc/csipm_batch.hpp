@@ -288,8 +288,7 @@ __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __res
   store_partial(part + I.pbase + I.gcg, acc, lb);
 }
 
-// r'z after an update that a true residual follows (the other iterations take
-// it in bk_cg_pupdate): beta = gamma_new / gamma_old, stopping tests
+// r'z after the update, where bk_cg_pupdate does not sum it: beta = gamma_new / gamma_old, stopping tests
 __global__ void bk_cg_gamma(BSeg vseg, const int* ids, const BInst* __restrict__ info,
                             CgState* cg, const double* part) {
   const int inst = ids[blockIdx.x];
@@ -372,8 +371,8 @@ __global__ void bk_cg_regamma(BSeg vseg, const int* ids, const BInst* __restrict
 // p = z + beta p.  SUM: beta = gamma_new / gamma_old from the update's partial
 // sums of r'z, which every workgroup adds itself in the same order; the first
 // one records it and the stopping tests (a workgroup that starts later may see
-// done: it leaves a p that nothing reads).  Otherwise beta as bk_cg_regamma
-// left it.
+// done: it leaves a p that nothing reads).  Otherwise beta as bk_cg_gamma or
+// bk_cg_regamma left it.
 // (A kernel of its own for the sum took 4.0 us of the 44 of an iteration of
 // 255 x 255 in FP64, a launch and a round trip; p's kernel 4.0 and, with the
 // sum, 4.9.)
