@@ -71,11 +71,14 @@ __device__ __forceinline__ void bstore_partials(double* part, const double (&acc
 // nb = 2: condensed system, block preconditioner [[P11, P12], [P12, P22]];
 // nb = 1: reduced system, diagonal preconditioner P11.
 // ===========================================================================
+// A kernel that several workgroups run for one instance reads no field that the
+// same launch writes: its waves would not agree on the value, and a wave that
+// left early would be missing from the workgroup's sums.
 struct CgState {
   double gamma;   // r'z before the residual update, for the kernel that takes p on
-  double gnew;    // r'z now; moved to gamma by the update that first reads it (a
-                  // launch never writes the one that its workgroups read)
-  double pq;
+  double gnew;    // r'z now; moved to gamma by the update that first reads it
+  double pq;      // p'q of bk_cg_update; not above 0: zero curvature, or the instance
+                  // was done before (the kernels after it test this, not done)
   double alpha;
   double beta;
   double rnorm;
@@ -192,8 +195,7 @@ constexpr int kCgSlots = 4;
 
 // after q = K p (its last pass left gcg partials of p'q): alpha = gamma / p'q
 // (every workgroup sums the apply's p'q partials itself,
-// in the same order, so all agree; the first one records it and a zero
-// curvature), then x += alpha p; r -= alpha q; z = P r; partial r'z at
+// in the same order, so all agree; the first one records it), then x += alpha p; r -= alpha q; z = P r; partial r'z at
 // pbase + gcg, beside the p'q partials other workgroups are still reading.
 // The loads of a thread's slots go out together and ahead of the sum: one
 // after another they bound the kernel in small problems (255 x 255 FP64 6.8 us before,
@@ -210,7 +212,10 @@ __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __res
   const BFlags* flags = nullptr;
   BSEG_BEGIN
   CgState& st = cg[inst];
-  if (st.done) return;
+  if (st.done) {
+    if (lb == 0 && threadIdx.x == 0) st.pq = 0.0;
+    return;
+  }
   const int64_t step = (int64_t)nbk * blockDim.x, end = I.off + I.n;
   int64_t i0 = I.off + (int64_t)lb * blockDim.x + threadIdx.x;
   T xv[kCgSlots][NB], rv[kCgSlots][NB], pv[kCgSlots][NB], qv[kCgSlots][NB], d[kCgSlots][2 * NB - 1];
@@ -240,17 +245,10 @@ __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __res
   if (threadIdx.x == 0) s_pq = pq0;
   __syncthreads();
   const double pq = s_pq;
-  if (!(pq > 0.0)) {
-    if (lb == 0 && threadIdx.x == 0) {
-      st.pq = pq;
-      st.done = 1;
-      st.status = 2;
-    }
-    return;
-  }
+  if (lb == 0 && threadIdx.x == 0) st.pq = pq;
+  if (!(pq > 0.0)) return;
   const double ad = st.gnew / pq;
   if (lb == 0 && threadIdx.x == 0) {
-    st.pq = pq;
     st.alpha = ad;
     st.gamma = st.gnew;
   }
@@ -288,12 +286,23 @@ __global__ __launch_bounds__(256) void bk_cg_update(BSeg seg, const BInst* __res
   store_partial(part + I.pbase + I.gcg, acc, lb);
 }
 
+// no step was taken: zero curvature ends the solve (unless it had ended before);
+// one thread of the instance
+__device__ __forceinline__ void cg_no_step(CgState& st) {
+  if (st.done) return;
+  st.done = 1;
+  st.status = 2;
+}
+
 // r'z after the update, where bk_cg_pupdate does not sum it: beta = gamma_new / gamma_old, stopping tests
 __global__ void bk_cg_gamma(BSeg vseg, const int* ids, const BInst* __restrict__ info,
                             CgState* cg, const double* part) {
   const int inst = ids[blockIdx.x];
   CgState& st = cg[inst];
-  if (st.done) return;
+  if (!(st.pq > 0.0)) {
+    if (threadIdx.x == 0) cg_no_step(st);
+    return;
+  }
   const BInst& I = info[inst];
   const double g =
       sum_partials(part + I.pbase + I.gcg, vseg.first[inst + 1] - vseg.first[inst]);
@@ -370,8 +379,7 @@ __global__ void bk_cg_regamma(BSeg vseg, const int* ids, const BInst* __restrict
 
 // p = z + beta p.  SUM: beta = gamma_new / gamma_old from the update's partial
 // sums of r'z, which every workgroup adds itself in the same order; the first
-// one records it and the stopping tests (a workgroup that starts later may see
-// done: it leaves a p that nothing reads).  Otherwise beta as bk_cg_gamma or
+// one records it and the stopping tests.  Otherwise beta as bk_cg_gamma or
 // bk_cg_regamma left it.
 // (A kernel of its own for the sum took 4.0 us of the 44 of an iteration of
 // 255 x 255 in FP64, a launch and a round trip; p's kernel 4.0 and, with the
@@ -384,7 +392,14 @@ __global__ __launch_bounds__(256) void bk_cg_pupdate(BSeg seg, const BInst* __re
   const BFlags* flags = nullptr;
   BSEG_BEGIN
   CgState& st = cg[inst];
-  if (st.done) return;
+  if constexpr (SUM) {
+    if (!(st.pq > 0.0)) {
+      if (lb == 0 && threadIdx.x == 0) cg_no_step(st);
+      return;
+    }
+  } else {
+    if (st.done) return;
+  }
   const int64_t n = nb * I.n, step = (int64_t)nbk * blockDim.x;
   const T* zi = z + 2 * I.off;
   T* pi = p + 2 * I.off;

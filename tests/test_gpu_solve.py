@@ -201,3 +201,43 @@ def test_admm_vs_oracle(cuda, case):
     assert abs(st.iterations - ref.iterations) <= 1
     z = st.solution.cpu().numpy()
     assert np.linalg.norm(z - ref.beta) <= 1e-8 * np.linalg.norm(ref.beta) + 1e-10
+
+
+# CG that meets a direction of non-positive curvature: at the first step, and
+# after 12 and 18 steps (the margin is 1e-2 of |p|^2); few vector blocks (r'z
+# summed by the kernel that updates p) and 551 of them (by a kernel of its own)
+@pytest.mark.parametrize("dims", [(40, 36), (96, 80, 72)])
+@pytest.mark.parametrize("first", [True, False])
+def test_zero_curvature(cuda, dims, first):
+    import ctypes
+
+    from csipm import _lib
+    from csipm.fft_operator import FFTOperator
+    print("zero curvature", dims, first, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(5)
+    miss = np.sort(rng.choice(n, n // 8, replace=False))
+    L1 = np.exp(rng.standard_normal(n))
+    L1[::7] *= -0.02
+    if first:
+        L1 = -2.0 - L1 * L1
+    b = rng.standard_normal(2 * n)
+    A = lambda v: np.concatenate([op.mtm(v[:n], dims, miss) + L1 * v[:n], L1 * v[n:]])  # noqa: E731
+    want, its, _, how = kkt.pcg(A, b, None, atol=1e-12)
+    assert how == "zero-curvature" and (its == 0) == first
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    one, zero = T(np.ones(n)), T(np.zeros(n))
+    bt, L1t = T(b), T(L1)
+    x = torch.full((2 * n,), 7.0, dtype=torch.float64, device=cuda)
+    it, res, st = ctypes.c_int64(), ctypes.c_double(), ctypes.c_int()
+    o = FFTOperator(n, len(dims), dims, miss)
+    for _ in range(2):   # eager and replayed iterations
+        _lib.call("csipm_cg_solve", o.handle, *[ctypes.c_void_p(t.data_ptr()) for t in
+                                                (bt, x, L1t, zero, one, zero, one)],
+                  1e-12, 0.0, 0, ctypes.byref(it), ctypes.byref(res), ctypes.byref(st))
+        assert (st.value, it.value) == (2, its)
+        got = x.cpu().numpy()
+        if first:
+            assert np.array_equal(got, want)
+        else:
+            assert _rel(got, want) <= 1e-10
