@@ -66,6 +66,19 @@ int64_t geomchk_rows(int dim, const int64_t* sizes) {
   const MapGeom g = geom(dim, sizes);
   return dim == 2 ? rows_off<2>(g) : rows_off<3>(g);
 }
+// u_scale and u_map of n complex values
+void geomchk_u_scale(int64_t n, const double* w, double* scaled, double* mapped, int mode) {
+  for (int64_t i = 0; i < n; ++i) {
+    reinterpret_cast<cpx<double>*>(scaled)[i] = u_scale(reinterpret_cast<const cpx<double>*>(w)[i], mode);
+    reinterpret_cast<cpx<double>*>(mapped)[i] = u_map(reinterpret_cast<const cpx<double>*>(w)[i], mode);
+  }
+}
+void geomchk_u_scalef(int64_t n, const float* w, float* scaled, float* mapped, int mode) {
+  for (int64_t i = 0; i < n; ++i) {
+    reinterpret_cast<cpx<float>*>(scaled)[i] = u_scale(reinterpret_cast<const cpx<float>*>(w)[i], mode);
+    reinterpret_cast<cpx<float>*>(mapped)[i] = u_map(reinterpret_cast<const cpx<float>*>(w)[i], mode);
+  }
+}
 // the geometry fields, for comparison with the oracle: n, M, P, S (3 each),
 // N, P12, P13, P23, P123, off[8]
 void geomchk_info(int dim, const int64_t* sizes, int64_t* out) {

@@ -127,3 +127,24 @@ def test_rows_equal_elements(glib, dims):
     glib.geomchk_rows.restype = ctypes.c_int64
     sz = _sizes(dims)
     assert glib.geomchk_rows(len(dims), _p(sz)) == 0
+
+
+# the passes' scaling by 1 / sqrt2 without a division is the quotient, at zeros,
+# infinities, NaN and the ends of the range as well
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_scale_is_the_quotient(glib, dtype, mode):
+    f = glib.geomchk_u_scale if dtype == np.float64 else glib.geomchk_u_scalef
+    f.argtypes = [ctypes.c_int64] + [ctypes.c_void_p] * 3 + [ctypes.c_int]
+    f.restype = None
+    rng = np.random.default_rng(3)
+    tiny, big = np.finfo(dtype).tiny, np.finfo(dtype).max
+    w = np.concatenate([rng.standard_normal(200000), [0.0, -0.0, np.inf, -np.inf, np.nan, big, -big,
+                                                      4 * tiny, -4 * tiny, 1.0]]).astype(dtype)
+    got, want = np.empty_like(w), np.empty_like(w)
+    f(w.size // 2, w.ctypes.data, got.ctypes.data, want.ctypes.data, mode)
+    # (w l of the sum w h + w l is subnormal up to here: one unit in the last place)
+    low = np.abs(w) < tiny / dtype(2) ** (-53 if dtype == np.float64 else -26)
+    assert np.array_equal(got[~low], want[~low], equal_nan=True)
+    assert np.all(np.abs(got[low] - want[low]) <= np.spacing(np.abs(want[low])))
+    assert np.array_equal(np.signbit(got[~np.isnan(got)]), np.signbit(want[~np.isnan(want)]))

@@ -265,3 +265,15 @@ def test_dense_lengths(cuda, dims, dtype):
     assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
     assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
     assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
+
+
+def test_infinite_entry(cuda):
+    """An infinite spectrum entry gives infinite samples, not NaN, where the
+    transform only adds it: beta of frequency 1 of four samples, cos(pi n / 2)."""
+    from csipm.fft_operator import M_perp_beta
+    print("infinite entry", flush=True)
+    for dtype in (torch.float64, torch.float32):
+        o = _make((4,), np.zeros(0, np.int64), dtype)
+        beta = torch.tensor([0.0, 0.0, np.inf, 0.0], dtype=dtype, device=cuda)
+        x = M_perp_beta(o, beta).cpu().numpy()
+        assert x[0] == np.inf and x[2] == -np.inf
