@@ -489,9 +489,9 @@ static bool dense_axis(int L, int64_t lines) {
 }
 
 // and, up to 127 (one block of output rows a wave), instead of the direct plan
-// with radix 29 or 31, whose butterflies run in a loop on a quarter of the
-// threads: operator product 87^3 FP32 97 to 47 us, 124^3 142 to 78, its solve
-// 20.6 to 14 ms.  Above, the plan is the better one (155^3 FP32 149 against 165)
+// with radix 29 or 31, whose tiles take more stages: operator product 87^3 FP32
+// 66 to 43 us, 124^3 86 to 71 (116 x 116 and 124 x 124 26 to 27).  Above, the plan is the
+// better one (155^3 FP32 124 against 165)
 static bool dense_direct(int L) {
   return L > 32 && L <= 127 && (L % 29 == 0 || L % 31 == 0);
 }

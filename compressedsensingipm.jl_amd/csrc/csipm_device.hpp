@@ -412,25 +412,13 @@ __device__ __forceinline__ void dft_odd_store(cpx<T>* v, cpx<T>* __restrict__ ds
     dst[k * stride] = {re + sre, im - sim};
     dst[(R - k) * stride] = {re - sre, im + sim};
   };
-  if constexpr (R < 29) {
-    // one output after another: scheduled across outputs the (H x H) products
-    // took hundreds of registers in FP64
+  // one output after another: scheduled across outputs the (H x H) products
+  // took hundreds of registers in FP64
 #pragma unroll
-    for (int k = 1; k <= H; ++k) {
-      output(k, [&](int j) { return (T)OddRadix<R>::c[(j * k) % R]; },
-             [&](int j) { return (T)OddRadix<R>::s[(j * k) % R]; });
-      if constexpr (R >= 11) __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
-    // a loop over the outputs, their coefficients by scalar loads: unrolled
-    // (900 instructions for radix 31) these two took 20 registers more than
-    // the rest.  Slower per output: radices 17 to 23 in this form took the
-    // FP32 185^3 product (Bluestein 23 x 17) from 402 to 525 us
-#pragma unroll 1
-    for (int k = 1; k <= H; ++k) {
-      const T* row = OddRows<T, R>::cs[k - 1];
-      output(k, [&](int j) { return row[j - 1]; }, [&](int j) { return row[H + j - 1]; });
-    }
+  for (int k = 1; k <= H; ++k) {
+    output(k, [&](int j) { return (T)OddRadix<R>::c[(j * k) % R]; },
+           [&](int j) { return (T)OddRadix<R>::s[(j * k) % R]; });
+    if constexpr (R >= 11) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -457,8 +445,7 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
 // radix-9..15 butterflies and their twiddles per thread) the FP64 passes
 // took 248-260 registers, one or two waves per SIMD, and the 1024-thread ones
 // spilled 1300 registers; E = 8 with the waves per SIMD asked for by
-// pass_waves() keeps three (FP64) or five (FP32; radices 29 and 31 spill some
-// tens of registers there).  Twiddles are laid out per stage in the order in
+// pass_waves() keeps three (FP64) or five (FP32).  Twiddles are laid out per stage in the order in
 // which adjacent lanes read them: strided reads from one table of the length
 // L cost a cache line per lane.
 // Measured (before -> after, with tile_grows' tiles): line passes of the FP64
@@ -521,6 +508,121 @@ __device__ __forceinline__ void dft15_store(cpx<T>* v, cpx<T>* __restrict__ dst,
 #pragma unroll
     for (int k1 = 0; k1 < 3; ++k1) dst[((10 * k1 + 6 * k2) % 15) * stride] = z[k1];
   }
+}
+
+// The matrix cores: 16 x 16 x 4 products, FP32 and FP64.
+template <typename T>
+using Vec4 = T __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ Vec4<float> mfma16x16x4(float a, float b, Vec4<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ Vec4<double> mfma16x16x4(double a, double b, Vec4<double> c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// row of accumulator i in a 16 x 16 tile (column: lane & 15)
+template <typename T>
+__device__ __forceinline__ int mfma_row(int lane, int i) {
+  return sizeof(T) == 4 ? 4 * (lane >> 4) + i : (lane >> 4) + 4 * i;
+}
+// the value of lane ^ 1
+__device__ __forceinline__ float lane_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double lane_swap(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// A stage of radix 29 or 31 on the matrix cores.  With H = (R - 1) / 2, a_j =
+// x_j + x_{R-j} and b_j = x_j - x_{R-j} (x twiddled, a_0 = x_0), the butterfly
+//   X_k = sum_j a_j cos(2 pi j k / R) - i sum_j b_j sin(2 pi j k / R)
+// is one 16-row tile of cosines times a and one of sines times b, eight
+// products for the 16 real columns of eight butterflies; X_{R-k} is the same
+// with + i.  a and b replace x in their LDS rows first; a wave takes every
+// (NT / 64)-th column tile and stores it when all waves have read theirs.
+// What bounds it: the LDS moves and, per column tile, eight products of 32
+// cycles.  As a butterfly a thread, its outputs in a loop, the radices kept one
+// wave in four busy and spilled 200 registers in FP64 (the pass kernels spill
+// up to 13 now): operator product 248^3 FP32 358 -> 290 us, FP64 583 -> 461;
+// 217 x 217 FP32 41.5 -> 27.2; 961 FP64 29.4 -> 17.2.  The outputs divided among
+// the waves instead: 248^3 FP32 333, FP64 799 (every wave spilled).
+template <typename T, int R, int NT>
+__device__ __forceinline__ void matrix_stage(cpx<T>* __restrict__ lds, int L, int Ns, uint32_t nsm,
+                                             int lg, int ps, const cpx<T>* __restrict__ tw) {
+  constexpr int H = (R - 1) / 2, W = NT / 64;
+  static_assert(H < 16, "one tile of output rows");
+  // column tiles of a wave: a plan gives a thread at most 16 elements
+  constexpr int NV = (2 * 16 * NT / R + 16 * W - 1) / (16 * W);
+  const int nb = L / R, nl = 1 << lg, total = nb << lg;
+  int tid = (int)threadIdx.x;   // (opaque: as in stockham_stage)
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, wave = uniform(tid >> 6), n = lane & 15, kk = lane >> 4;
+  // coefficients of output n: cosines of rows j = 4 kt + kk, sines of j + 1
+  T cc[4], ss[4];
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) {
+    const int j = 4 * kt + kk;
+    cc[kt] = j <= H ? (T)OddRadix<R>::c[(j * n) % R] : (T)0;
+    ss[kt] = j < H ? (T)OddRadix<R>::s[((j + 1) * n) % R] : (T)0;
+  }
+  const int groups = (total + 63) >> 6;
+  for (int c = wave; c < H * groups; c += W) {
+    const int p = 1 + c / groups, b = (c - (p - 1) * groups) * 64 + lane;
+    if (b < total) {
+      const int j = b >> lg;
+      cpx<T>* lo = lds + (j + p * nb) * ps + (b & (nl - 1));
+      cpx<T>* hi = lo + (R - 2 * p) * nb * ps;
+      cpx<T> x = *lo, y = *hi;
+      if (Ns > 1) {
+        const int k = j - fdiv(j, nsm) * Ns;
+        x = cmul(x, tw[(p - 1) * Ns + k]);
+        y = cmul(y, tw[(R - p - 1) * Ns + k]);
+      }
+      *lo = cadd(x, y);
+      *hi = csub(x, y);
+    }
+  }
+  __syncthreads();
+  const int tiles = (2 * total + 15) >> 4, rs = 2 * ps, step = nb * rs;
+  T* x = reinterpret_cast<T*>(lds);
+  Vec4<T> c[NV], s[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (wave + v * W >= tiles) continue;
+    const int col = min((wave + v * W) * 16 + n, 2 * total - 1), b = col >> 1, j = b >> lg;
+    const T* src = x + j * rs + 2 * (b & (nl - 1)) + (col & 1);
+    c[v] = s[v] = Vec4<T>{0, 0, 0, 0};
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      // (rows past H: any row, as zero, so that an infinity stays one)
+      const int jc = 4 * kt + kk, js = jc + 1;
+      const T a = src[jc * step], d = src[(R - js) * step];
+      c[v] = mfma16x16x4(cc[kt], jc <= H ? a : (T)0, c[v]);
+      s[v] = mfma16x16x4(ss[kt], js <= H ? d : (T)0, s[v]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (wave + v * W >= tiles) continue;
+    const int col = (wave + v * W) * 16 + n, b = col >> 1, j = b >> lg;
+    const int k = Ns > 1 ? j - fdiv(j, nsm) * Ns : 0;
+    T* dst = x + ((j - k) * R + k) * rs + 2 * (b & (nl - 1)) + (col & 1);
+    const bool im = n & 1;   // column pairs hold real and imaginary parts
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const T other = lane_swap(s[v][i]);
+      const T plus = c[v][i] + other, minus = c[v][i] - other;
+      const int r = mfma_row<T>(lane, i);
+      if (col < 2 * total && r <= H) {
+        dst[r * Ns * rs] = im ? minus : plus;
+        if (r > 0) dst[(R - r) * Ns * rs] = im ? plus : minus;
+      }
+    }
+  }
+  __syncthreads();
 }
 
 template <typename T, int R, int E, int NT>
@@ -617,8 +719,8 @@ __device__ __forceinline__ void lds_fft(cpx<T>* lds, int pl, int lg, int ps,
       case 17: stockham_stage<T, 17, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
       case 19: stockham_stage<T, 19, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
       case 23: stockham_stage<T, 23, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
-      case 29: stockham_stage<T, 29, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
-      case 31: stockham_stage<T, 31, E, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 29: matrix_stage<T, 29, NT>(lds, L, ns, nsm, lg, ps, tws); break;
+      case 31: matrix_stage<T, 31, NT>(lds, L, ns, nsm, lg, ps, tws); break;
       default: break;  // the host planner only emits the radices above
     }
   }

@@ -474,30 +474,6 @@ struct PassArgs {
 // such lengths spent over a thousand cycles a line on two transforms and the
 // moves between, in twice the LDS rows: the operator product of 127^3 took 187
 // us in FP32 and 75 with this (185^3: 400 to 243, FP64 784 to 392).
-template <typename T>
-using Vec4 = T __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ Vec4<float> mfma16x16x4(float a, float b, Vec4<float> c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ Vec4<double> mfma16x16x4(double a, double b, Vec4<double> c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-// row of accumulator i in a 16 x 16 tile (column: lane & 15)
-template <typename T>
-__device__ __forceinline__ int mfma_row(int lane, int i) {
-  return sizeof(T) == 4 ? 4 * (lane >> 4) + i : (lane >> 4) + 4 * i;
-}
-// the value of lane ^ 1
-__device__ __forceinline__ float lane_swap(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
-}
-__device__ __forceinline__ double lane_swap(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
 // tiles of the coefficient matrices: ceil((H + 1) / 16) by ceil((H + 1) / 4)
 // (cosine) and by ceil(((L - 1) / 2) / 4) (sine), the latter two made even
 // (zero tiles; their rows stay inside the line for L > 16)

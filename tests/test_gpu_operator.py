@@ -277,3 +277,30 @@ def test_infinite_entry(cuda):
         beta = torch.tensor([0.0, 0.0, np.inf, 0.0], dtype=dtype, device=cuda)
         x = M_perp_beta(o, beta).cpu().numpy()
         assert x[0] == np.inf and x[2] == -np.inf
+
+
+# stages of radix 29 and 31 (matrix products): alone, twice (twiddles between),
+# with every kind of stage after them; column tiles full and not, one line and
+# 16, 128 to 1024 threads, four-step (7192), Rader's inner transforms (59: 58;
+# 311 on few lines: 310)
+@pytest.mark.parametrize("dims", [(29,), (31,), (58,), (59,), (841,), (899,), (961,), (3596,), (7192,),
+                                  (29791,), (155, 3), (3, 217), (145, 155, 7), (4, 6, 248), (3596, 2),
+                                  (2, 3596), (8990, 2), (16, 217, 1030), (311, 5), (5, 311)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_matrix_stages(cuda, dims, dtype):
+    from csipm import tune
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("matrix stages", dims, dtype, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 11)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    tol = TOL64 if dtype == torch.float64 else TOL32
+    o = _make(dims, miss, dtype)
+    for axis, length in enumerate(dims):
+        if length % 29 == 0 or length % 31 == 0:
+            assert tune.fft_shape(o, axis)[2] in (0, 3)   # a plan, four-step or not
+    xt = torch.from_numpy(x).to(cuda, dtype)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
