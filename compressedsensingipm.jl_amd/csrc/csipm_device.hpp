@@ -540,14 +540,15 @@ __device__ __forceinline__ double lane_swap(double v) {
 //   X_k = sum_j a_j cos(2 pi j k / R) - i sum_j b_j sin(2 pi j k / R)
 // is one 16-row tile of cosines times a and one of sines times b, eight
 // products for the 16 real columns of eight butterflies; X_{R-k} is the same
-// with + i.  a and b replace x in their LDS rows first; a wave takes every
-// (NT / 64)-th column tile and stores it when all waves have read theirs.
-// What bounds it: the LDS moves and, per column tile, eight products of 32
-// cycles.  As a butterfly a thread, its outputs in a loop, the radices kept one
+// with + i.  A wave takes every (NT / 64)-th column tile and stores it when all
+// waves have read theirs.
+// What bounds it: per column tile eight products of 32 cycles and as many LDS
+// reads.  As a butterfly a thread, its outputs in a loop, the radices kept one
 // wave in four busy and spilled 200 registers in FP64 (the pass kernels spill
-// up to 13 now): operator product 248^3 FP32 358 -> 290 us, FP64 583 -> 461;
-// 217 x 217 FP32 41.5 -> 27.2; 961 FP64 29.4 -> 17.2.  The outputs divided among
-// the waves instead: 248^3 FP32 333, FP64 799 (every wave spilled).
+// up to 13 now): operator product 248^3 FP32 358 -> 272 us, FP64 583 -> 433;
+// 217 x 217 FP32 41.5 -> 24.1; 961 FP64 29.4 -> 13.3.  The outputs divided among
+// the waves instead: 248^3 FP32 333, FP64 799 (every wave spilled); a and b
+// formed in LDS first: 290, 461.
 template <typename T, int R, int NT>
 __device__ __forceinline__ void matrix_stage(cpx<T>* __restrict__ lds, int L, int Ns, uint32_t nsm,
                                              int lg, int ps, const cpx<T>* __restrict__ tw) {
@@ -559,48 +560,46 @@ __device__ __forceinline__ void matrix_stage(cpx<T>* __restrict__ lds, int L, in
   int tid = (int)threadIdx.x;   // (opaque: as in stockham_stage)
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, wave = uniform(tid >> 6), n = lane & 15, kk = lane >> 4;
-  // coefficients of output n: cosines of rows j = 4 kt + kk, sines of j + 1
+  const bool im = n & 1;   // column pairs hold real and imaginary parts
+  const int tiles = (2 * total + 15) >> 4, rs = 2 * ps;
+  // input rows j = 4 kt + kk and R - j, and their coefficients in output n
   T cc[4], ss[4];
+  int lo[4], hi[4];
 #pragma unroll
   for (int kt = 0; kt < 4; ++kt) {
     const int j = 4 * kt + kk;
     cc[kt] = j <= H ? (T)OddRadix<R>::c[(j * n) % R] : (T)0;
-    ss[kt] = j < H ? (T)OddRadix<R>::s[((j + 1) * n) % R] : (T)0;
+    ss[kt] = j <= H ? (T)OddRadix<R>::s[(j * n) % R] : (T)0;
+    lo[kt] = j * nb * rs;
+    hi[kt] = (j ? R - j : 0) * nb * rs;
   }
-  const int groups = (total + 63) >> 6;
-  for (int c = wave; c < H * groups; c += W) {
-    const int p = 1 + c / groups, b = (c - (p - 1) * groups) * 64 + lane;
-    if (b < total) {
-      const int j = b >> lg;
-      cpx<T>* lo = lds + (j + p * nb) * ps + (b & (nl - 1));
-      cpx<T>* hi = lo + (R - 2 * p) * nb * ps;
-      cpx<T> x = *lo, y = *hi;
-      if (Ns > 1) {
-        const int k = j - fdiv(j, nsm) * Ns;
-        x = cmul(x, tw[(p - 1) * Ns + k]);
-        y = cmul(y, tw[(R - p - 1) * Ns + k]);
-      }
-      *lo = cadd(x, y);
-      *hi = csub(x, y);
-    }
-  }
-  __syncthreads();
-  const int tiles = (2 * total + 15) >> 4, rs = 2 * ps, step = nb * rs;
   T* x = reinterpret_cast<T*>(lds);
   Vec4<T> c[NV], s[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     if (wave + v * W >= tiles) continue;
-    const int col = min((wave + v * W) * 16 + n, 2 * total - 1), b = col >> 1, j = b >> lg;
-    const T* src = x + j * rs + 2 * (b & (nl - 1)) + (col & 1);
+    const int col = min((wave + v * W) * 16 + n, 2 * total - 1), b = col >> 1, jb = b >> lg;
+    const T* src = x + jb * rs + 2 * (b & (nl - 1)) + (col & 1);
+    const int k = Ns > 1 ? jb - fdiv(jb, nsm) * Ns : 0;
     c[v] = s[v] = Vec4<T>{0, 0, 0, 0};
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      // (rows past H: any row, as zero, so that an infinity stays one)
-      const int jc = 4 * kt + kk, js = jc + 1;
-      const T a = src[jc * step], d = src[(R - js) * step];
-      c[v] = mfma16x16x4(cc[kt], jc <= H ? a : (T)0, c[v]);
-      s[v] = mfma16x16x4(ss[kt], js <= H ? d : (T)0, s[v]);
+      const int j = 4 * kt + kk;
+      T y = src[lo[kt]], z = src[hi[kt]];
+      if (Ns > 1) {
+        cpx<T> w = {(T)1, (T)0}, u = w;
+        if (j > 0) {
+          w = tw[(j - 1) * Ns + k];
+          u = tw[(R - j - 1) * Ns + k];
+        }
+        const T yo = lane_swap(y), zo = lane_swap(z);
+        y = y * w.x + (im ? yo : -yo) * w.y;
+        z = z * u.x + (im ? zo : -zo) * u.y;
+      }
+      // (zeros where the coefficients are zero, so that an infinity stays one)
+      const T a = j > H ? (T)0 : j ? y + z : y, d = j > H || j == 0 ? (T)0 : y - z;
+      c[v] = mfma16x16x4(cc[kt], a, c[v]);
+      s[v] = mfma16x16x4(ss[kt], d, s[v]);
     }
   }
   __syncthreads();
@@ -610,7 +609,6 @@ __device__ __forceinline__ void matrix_stage(cpx<T>* __restrict__ lds, int L, in
     const int col = (wave + v * W) * 16 + n, b = col >> 1, j = b >> lg;
     const int k = Ns > 1 ? j - fdiv(j, nsm) * Ns : 0;
     T* dst = x + ((j - k) * R + k) * rs + 2 * (b & (nl - 1)) + (col & 1);
-    const bool im = n & 1;   // column pairs hold real and imaginary parts
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const T other = lane_swap(s[v][i]);
