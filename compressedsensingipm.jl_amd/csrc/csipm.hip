@@ -332,8 +332,15 @@ inline int tile_nt(int64_t elems, const FftPlan& p) {
 // transform.  185^3 in FP32 (391 rows): 414 us with four lines on 256 threads,
 // 453 with eight on 512.  mixed: a launch of several kinds of passes, whose
 // workgroups all hold the LDS of the largest tile: 2048 elements (48 requests,
-// 56.6 against 59.6 ms).
-inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed) {
+// 56.6 against 59.6 ms).  kkt: the last pass of a KKT product in the packed
+// layout, which reads four operands and writes two results in runs of half a
+// row: up to 512 threads while the rows span less than 128 bytes, once
+// operands and results pass kKktWide bytes and no longer stay in the 256 MB
+// Infinity Cache (FP32 255^3 393 -> 347 us, 210^3 245 -> 232; below, 192^3 170
+// -> 174; in the other line passes the same tiles are the slower ones, 12 to 20%
+// of an operator product).
+constexpr int64_t kKktWide = 200 << 20;
+inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed, bool kkt = false) {
   const int64_t e = (int64_t)(2 << lg) * p.L;
   // dense: the matrix tiles want 16 real columns, and more share their
   // coefficients; four waves hold 16 k-tiles of 16 columns, 8 of 32 or 4 of 64
@@ -343,8 +350,9 @@ inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed
   const int t = tile_threads(e, p);
   if (e > kTile) return false;
   if (mixed && e > kTile / 2 && ((size_t)1 << lg) * cs >= 64) return false;
-  return (t <= 256 && ((size_t)2 << lg) * rows * cs <= 32 * 1024) ||
-         (t <= 512 && ((size_t)1 << lg) * cs < 32);
+  const bool fits = ((size_t)2 << lg) * rows * cs <= 32 * 1024;
+  return (t <= 256 && fits) || (t <= 512 && ((size_t)1 << lg) * cs < 32) ||
+         (kkt && t <= 512 && fits && ((size_t)1 << lg) * cs < 128);
 }
 
 struct LineCfg {
@@ -365,6 +373,7 @@ struct PrecState {
   void* chirp[3] = {nullptr, nullptr, nullptr};   // Bluestein tables (axes with bs)
   void* bfw[3] = {nullptr, nullptr, nullptr};
   LineCfg lines[3];
+  LineCfg kkt;   // the last line pass of a KKT product in the packed layout
   Dim1Cfg d1;
   // long 1D lines (four-step): twiddles of the column (B) and row (A)
   // transforms (tw[0] holds those of the full length F, chirp[0].. the outer
@@ -967,10 +976,11 @@ static int min_tile_lg(size_t cs) {
 // workgroups (1024 for one instance; a batch shares the target among its
 // instances)
 static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size_t cs,
-                        int min_grid = 1024, int lg_cap = 30, bool mixed = false) {
+                        int min_grid = 1024, int lg_cap = 30, bool mixed = false,
+                        bool kkt = false) {
   LineCfg c{};
   int lg = 0;
-  while (tile_grows(lg, plan, R, cs, mixed) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
+  while (tile_grows(lg, plan, R, cs, mixed, kkt) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
          lg < lg_cap)
     ++lg;
   // below 64-byte rows only while the launch would not even give a
@@ -1245,8 +1255,9 @@ int launch_pass(csipm_op* h, const PassArgs<T>& a, int grid, int nt, size_t lds)
 
 template <typename T, int D, int SRC, int DST, bool FWD>
 int launch_lines(csipm_op* h, int axis, const void* src, const Epi<T>& epi, const int* done) {
-  const LineCfg& c = h->ps<T>().lines[axis];
-  PassArgs<T> a = lines_args<T>(h, axis, src, epi, done);
+  const PrecState& ps = h->ps<T>();
+  const LineCfg& c = DST == DST_BETA && epi.kind != 0 ? ps.kkt : ps.lines[axis];
+  PassArgs<T> a = lines_args<T>(h, axis, src, epi, done, &c);
   set_steps(a, {PK_LINES, D, SRC, DST, FWD ? 1 : 0, axis}, false);
   return launch_pass(h, a, c.grid, c.nt, c.lds);
 }
@@ -2041,6 +2052,9 @@ static int set_shapes(csipm_op* h, PrecState& ps, size_t cs) {
                 "workgroup", h->n[0], F0);
   if (dim >= 2) ps.lines[1] = line_cfg(h->H1, h->plan[1], h->rows[1], h->n[2], cs);
   if (dim == 3) ps.lines[2] = line_cfg(h->H1, h->plan[2], h->rows[2], h->n[1], cs);
+  if (dim >= 2)
+    ps.kkt = line_cfg(h->H1, h->plan[dim - 1], h->rows[dim - 1], dim == 3 ? h->n[1] : 1, cs, 1024,
+                      30, false, 6 * (int64_t)h->N * (int64_t)(cs / 2) > kKktWide);
   for (int ax = 1; ax < dim; ++ax)
     if (h->plan[ax].L > kTile || ps.lines[ax].lds > kLdsMax)
       return fail(CSIPM_ERR_UNSUPPORTED, "dimension-%d length %d (%d LDS rows) exceeds one "
