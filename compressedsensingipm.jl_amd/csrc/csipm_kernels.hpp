@@ -1442,8 +1442,22 @@ __device__ __forceinline__ void row_store(const PassArgs<T>& a, cpx<T>* lds, int
 // Bluestein), FORM_DENSE or any (together they take more registers: the FP32
 // 256^3 product 357 against 374 us)
 enum { FORM_FFT = 0, FORM_DENSE = 1, FORM_ANY = 2 };
+// args: the kernel's arguments in memory, where it loads them again.  The 3D
+// line store to beta uses most of them; held from the load on, they went
+// through the transform as spilled scalars, read back one by one in the store's
+// loops, a fifth of the kernel's vector instructions.  (Adjoint of 256^3 FP32
+// 148 -> 138 us, FP64 240 -> 221; the dense kernels, 127^3, took 1% longer with
+// it, and the store to a 2D beta 3%.)
+template <typename T>
+using ArgsPtr = const __attribute__((address_space(4))) PassArgs<T>*;
+template <typename T>
+__device__ __forceinline__ PassArgs<T> load_args(ArgsPtr<T> p) {
+  asm volatile("" : "+s"(p));   // (not the values loaded before)
+  return *(const PassArgs<T>*)p;
+}
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
-__device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
+__device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile,
+                                          ArgsPtr<T> args = nullptr) {
   const int ld = LD < 0 ? a.ld : LD, mid = MID < 0 ? a.mid : MID, st = ST < 0 ? a.st : ST;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
@@ -1526,7 +1540,12 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile) {
           case ST_LINES_U2: acc = lines_store<T, NT, 2, DST_U, true>(a, lds, tile); break;
           case ST_LINES_U3: acc = lines_store<T, NT, 3, DST_U, true>(a, lds, tile); break;
           case ST_LINES_BETA2: acc = lines_store<T, NT, 2, DST_BETA, true>(a, lds, tile); break;
-          case ST_LINES_BETA3: acc = lines_store<T, NT, 3, DST_BETA, true>(a, lds, tile); break;
+          case ST_LINES_BETA3:
+            if constexpr (ST == ST_LINES_BETA3 && FORM == FORM_FFT)
+              acc = lines_store<T, NT, 3, DST_BETA, true>(load_args<T>(args), lds, tile);
+            else
+              acc = lines_store<T, NT, 3, DST_BETA, true>(a, lds, tile);
+            break;
           case ST_COL_BUF_FWD: col_store<T, NT, DST_BUF, true>(a, lds, tile); return;
           case ST_COL_BUF_INV: col_store<T, NT, DST_BUF, false>(a, lds, tile); return;
           case ST_COL_U: acc = col_store<T, NT, DST_U, true>(a, lds, tile); break;
@@ -1558,7 +1577,12 @@ constexpr int pass_waves() {
 // a pass of one instance
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
 __global__ __launch_bounds__(NT, (pass_waves<T, NT, LD, FORM>())) void k_pass(PassArgs<T> a) {
-  pass_body<T, NT, E, LD, MID, ST, FORM>(a, xcd_block());
+  if constexpr (ST == ST_LINES_BETA3 && FORM == FORM_FFT) {
+    const ArgsPtr<T> args = (ArgsPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
+    pass_body<T, NT, E, LD, MID, ST, FORM>(load_args<T>(args), xcd_block(), args);
+  } else {
+    pass_body<T, NT, E, LD, MID, ST, FORM>(a, xcd_block());
+  }
 }
 
 // member and tile of a block of a launch over several instances; member < 0:
