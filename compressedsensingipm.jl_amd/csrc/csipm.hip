@@ -1051,6 +1051,11 @@ static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int m
   c.grid = (c.npairs + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
   c.nt = tile_nt((int64_t)plan.L << lg, plan);
+  // one line alone: a launch of one workgroup, which waits for its loads more
+  // than for its stages (operator product, 256 and 512 threads: 2048 FP32 17.8
+  // and 15.9 us, 4096 26.8 and 22.2, 4096 FP64 26.1 and 22.9; of many lines
+  // the smaller workgroups run beside each other)
+  if (nlines == 1 && min_grid >= 1024 && plan.L > 1024) c.nt = std::max(c.nt, 512);
   return c;
 }
 
