@@ -9,19 +9,21 @@ For every line-transform shape the serving and batch workloads meet (the odd
 configurations), it builds a batch of instances of that shape, and for each
 pass kind (line pass, dimension-1 pass) times the batch's FP32 CG operator
 apply (csipm_batch_apply_timed, HIP events) under the candidate launch
-shapes: the tile capped at the built-in size and one or two halvings of it,
-on 128 or 256 threads where the tile allows.  The fastest candidate that
-beats the built-in choice by more than 3% is written to the table
+shapes: the tile capped at 8, 4 or 2 lines (the workgroup size follows from
+the tile).  The fastest candidate that beats the built-in choice by more than
+3%, in each of two timings, is written to the table
 (tune_table.json beside this module), keyed on (pass kind, element bytes,
 FFT length, LDS rows), which `load()` hands to the library
 (csipm_tune_set) whenever libcsipm is loaded.
 
---bluestein chooses the convolution length M of every Bluestein line length
-of those shapes: the smallest factorable M >= 2L - 1 and the cheapest few
-in [2L - 1, 2.25 L] by a stage-cost model are each timed (the shape's FP32
-apply at its best launch shapes), and an M that beats the smallest by more
-than 3% is added to the table's "bluestein" list (csipm_tune_bluestein),
-with the launch-shape entries of its passes; the rest of the table is kept.
+--bluestein looks for a convolution length M for every line length of those
+shapes that neither factors nor has Rader's form: the smallest factorable
+M >= 2L - 1 and the cheapest few in [2L - 1, 2.25 L] by a stage-cost model are
+each timed against the plan the library chooses by itself (the dense form, up
+to 511; the shape's FP32 apply at its best launch shapes).  An M that beats
+that plan by more than 3% is added to the table's "bluestein" list
+(csipm_tune_bluestein: the axis then takes Bluestein's form), with the
+launch-shape entries of its passes; the rest of the table is kept.
 """
 from __future__ import annotations
 
@@ -50,7 +52,7 @@ def load(lib=None, path=TABLE):
     n = 0
     for e in tab.get("entries", []):
         rc = lib.csipm_tune_set(int(e["kind"]), int(e["elem_bytes"]), int(e["fft_len"]),
-                                int(e["rows"]), int(e["lg_cap"]), int(e["nt"]))
+                                int(e["rows"]), int(e["lg_cap"]), int(e.get("nt", 0)))
         if rc == 0:
             n += 1
     for e in tab.get("bluestein", []):
@@ -103,43 +105,41 @@ def tune_shape(dims, count, reps, lib, log):
             tag = lambda n: ("dim1" in n and n.startswith(f"{d}d:"))          # noqa: E731
         else:
             tag = lambda n: ("lines" in n and n.startswith(f"{d}d:"))         # noqa: E731
+        def timed(cap):
+            lib.csipm_tune_set(kind, 8, w, r, -1 if cap is None else cap, 0)
+            return _time(probs, ops, tag, reps)
+        first = {cap: timed(cap) for cap in (None, 3, 2, 1)}
+        cap = min(first, key=first.get)
+        # the better of several timings of equal launches is better by chance:
+        # the winner has to win again
+        again = {c: timed(c) for c in (None, cap)} if cap is not None else first
         lib.csipm_tune_set(kind, 8, w, r, -1, 0)
-        base = _time(probs, ops, tag, reps)
-        best = (base, None)
-        for cap in (3, 2, 1):
-            for nt in (128, 256):
-                lib.csipm_tune_set(kind, 8, w, r, cap, nt)
-                t = _time(probs, ops, tag, reps)
-                if t < best[0]:
-                    best = (t, (cap, nt))
-        lib.csipm_tune_set(kind, 8, w, r, -1, 0)
-        gain = base / best[0] if best[1] else 1.0
+        base, best = max((first[None], first[cap]), (again[None], again[cap]),
+                         key=lambda t: t[1] / t[0])
         log(f"{'x'.join(map(str, dims))} {KIND_NAMES[kind]} W={w} R={r} mode={mode}: built-in "
-            f"{base:.4f} ms, best {best[0]:.4f} ms {best[1]} ({gain:.3f}x)")
-        if best[1] and gain > 1.03:
-            out.append({"kind": kind, "elem_bytes": 8, "fft_len": w, "rows": r,
-                        "lg_cap": best[1][0], "nt": best[1][1],
+            f"{base:.4f} ms, cap {cap} {best:.4f} ms ({base / best:.3f}x)")
+        if cap is not None and base / best > 1.03:
+            out.append({"kind": kind, "elem_bytes": 8, "fft_len": w, "rows": r, "lg_cap": cap,
                         "shape": list(dims), "ms_builtin": round(base, 5),
-                        "ms_tuned": round(best[0], 5)})
+                        "ms_tuned": round(best, 5)})
     del ops
     return out
 
 
 def radix_stages(m):
-    """Radices of the library's plan of length m (its factorisation order:
-    31, 29, 23, 19, then 16, 8, 4, 2, then 17, 13, 11, 7, 15, 9, 5, 3), or
-    None when m does not factor."""
+    """Radices of the library's plan of length m (in its order: the odd ones
+    31 to 7, 15, 9, 5, 3, then 16, 8, 4, 2), or None when m does not factor."""
     out = []
-    for r in (31, 29, 23, 19, 16, 8, 4, 2, 17, 13, 11, 7, 15, 9, 5, 3):
+    for r in (31, 29, 23, 19, 17, 13, 11, 7, 15, 9, 5, 3, 16, 8, 4, 2):
         while m % r == 0:
             out.append(r)
             m //= r
     return out if m == 1 else None
 
 
-# relative cost of one radix-r stage per element (least-squares fit to timed
-# batched applies of 3D Bluestein cubes on MI355X: a stage costs about the
-# same whatever its radix, 8 and 16 less, the large odd radices more)
+# relative cost of one radix-r stage per element, which only orders the
+# candidates to time (least-squares fit to batched applies of 3D Bluestein cubes
+# on MI355X, before the radices 29 and 31 went to the matrix cores)
 STAGE_COST = {2: 4.6, 3: 4.6, 4: 4.4, 5: 4.2, 7: 4.3, 8: 3.1, 9: 4.1, 11: 4.3, 13: 5.4,
               15: 6.4, 16: 3.6, 17: 4.3, 19: 5.1, 23: 5.8, 29: 7.8, 31: 6.1}
 
@@ -156,17 +156,16 @@ def bluestein_candidates(L, keep=5):
 
 def _shape_best(dims, count, reps, lib):
     """Best FP32 apply time (ms) of each pass kind of the shape under the
-    launch-shape candidates: ({kind: (ms, (cap, nt) or None, built-in ms)},
-    shapes)."""
+    launch-shape candidates: ({kind: (ms, cap or None, built-in ms)}, shapes)."""
     probs, ops = _batch(dims, count)
     d = len(dims)
     kinds = [(1, 0)] + ([(0, 1)] if d >= 2 else [])
     shp = {kind: fft_shape(ops[0], axis) for kind, axis in kinds}
     best = {}
-    for cand in [None, (3, 128), (3, 256), (2, 128), (2, 256), (1, 128), (1, 256)]:
+    for cap in (None, 3, 2, 1):
         for kind, _ in kinds:
             w, r, _m = shp[kind]
-            lib.csipm_tune_set(kind, 8, w, r, *(cand or (-1, 0)))
+            lib.csipm_tune_set(kind, 8, w, r, -1 if cap is None else cap, 0)
         from csipm.batch import BatchSolver, slots_of
         bs = BatchSolver(sum(slots_of(o) for o in ops), max_instances=len(ops), mixed=True)
         for p, o in zip(probs, ops):
@@ -178,11 +177,11 @@ def _shape_best(dims, count, reps, lib):
         for kind, _ in kinds:
             tag = "dim1" if kind == 1 else "lines"
             t = sum(ms for name, ms, _ in launches if tag in name and name.startswith(f"{d}d:"))
-            if cand is None:
+            if cap is None:
                 base = t
-                best[kind] = (t, cand, base)
+                best[kind] = (t, cap, base)
             elif t < best[kind][0]:
-                best[kind] = (t, cand, best[kind][2])
+                best[kind] = (t, cap, best[kind][2])
     for kind, _ in kinds:
         w, r, _m = shp[kind]
         lib.csipm_tune_set(kind, 8, w, r, -1, 0)
@@ -192,36 +191,36 @@ def _shape_best(dims, count, reps, lib):
 
 
 def tune_bluestein(dims, count, reps, lib, log):
-    """(bluestein entry or None, launch-shape entries) of a shape whose
-    sides all equal L and take Bluestein's form."""
+    """(bluestein entry or None, launch-shape entries) of a shape whose sides
+    all equal L, a length without a plan of the radices or Rader's form."""
     L = dims[0]
     m0, cands = bluestein_candidates(L)
     if m0 is None:
         return None, []
     res = {}
-    for m in dict.fromkeys([m0] + cands):
+    for m in dict.fromkeys([0, m0] + cands):      # 0: the library's own choice
         lib.csipm_tune_bluestein(L, m)
         best, shp = _shape_best(dims, count, reps, lib)
         res[m] = (sum(v[0] for v in best.values()), best, shp)
     lib.csipm_tune_bluestein(L, 0)
     mb = min(res, key=lambda m: res[m][0])
-    gain = res[m0][0] / res[mb][0]
-    log(f"{'x'.join(map(str, dims))} Bluestein L={L}: " +
-        ", ".join(f"M={m} {radix_stages(m)} {res[m][0]:.4f} ms" for m in res) +
+    gain = res[0][0] / res[mb][0]
+    log(f"{'x'.join(map(str, dims))} L={L}: built-in {res[0][0]:.4f} ms, " +
+        ", ".join(f"M={m} {radix_stages(m)} {res[m][0]:.4f} ms" for m in res if m) +
         f" -> M={mb} ({gain:.3f}x)")
-    if mb == m0 or gain <= 1.03:
+    if mb == 0 or gain <= 1.03:
         return None, []
     total, best, shp = res[mb]
     out = []
-    for kind, (t, cand, base) in best.items():
-        if cand is None or base / t <= 1.03:
+    for kind, (t, cap, base) in best.items():
+        if cap is None or base / t <= 1.03:
             continue
         w, r, _m = shp[kind]
-        out.append({"kind": kind, "elem_bytes": 8, "fft_len": w, "rows": r,
-                    "lg_cap": cand[0], "nt": cand[1], "shape": list(dims),
-                    "ms_builtin": round(base, 5), "ms_tuned": round(t, 5)})
+        out.append({"kind": kind, "elem_bytes": 8, "fft_len": w, "rows": r, "lg_cap": cap,
+                    "shape": list(dims), "ms_builtin": round(base, 5),
+                    "ms_tuned": round(t, 5)})
     return ({"line_len": L, "conv_len": mb, "shape": list(dims),
-             "ms_smallest": round(res[m0][0], 5), "ms_tuned": round(total, 5)}, out)
+             "ms_builtin": round(res[0][0], 5), "ms_tuned": round(total, 5)}, out)
 
 
 def main_bluestein(args, lib, log):
