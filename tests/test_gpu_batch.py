@@ -336,3 +336,24 @@ def test_failure_statuses(cuda):
         bad = FFTNLPModel(FFTParameters(2, p.dims, z, p.lam, p.missing), mixed=mixed)
         st = ipm_solve(bad, tol=1e-8, max_iter=50)
         assert st.status == "failure" and st.iterations <= 1, (mixed, st.status, st.iterations)
+
+
+# launches that hold dense and other members: of one dimensionality (the same
+# steps, two forms of the transform) and of all three; (64, 127, 127) has dense
+# tiles of 16 lines, 17 of 32 of them past the last line
+@pytest.mark.parametrize("shapes", [
+    [(37, 41, 43), (40, 36, 42), (31, 37, 64), (64, 127, 127)],
+    [(61, 53), (64, 60), (127, 100), (35, 58)],
+    [(61, 53), (64, 60), (37, 41, 43), (40, 36, 42), (64, 127, 127), (1500,), (12289,)],
+])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_dense_and_other_members(cuda, shapes, mixed):
+    import csipm.workloads as wl
+    from csipm.batch import solve_batch
+    print("dense members", shapes, "mixed" if mixed else "f64", flush=True)
+    tol = 1e-8
+    probs = [wl.batch_instance(s, seed=40 + k) for k, s in enumerate(shapes)]
+    ops = [_op(p, mixed) for p in probs]
+    res = solve_batch(ops, [p.z0 for p in probs], [p.lam for p in probs], mixed=mixed, tol=tol)
+    for p, r in zip(probs, res):
+        _same(r, _alone(p, mixed, tol), p.name)

@@ -304,3 +304,58 @@ def test_matrix_stages(cuda, dims, dtype):
     assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
     assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
     assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
+
+
+# The form each axis is planned in (0 direct, 1 Bluestein, 2 Rader, 4 dense), on
+# line passes as well as along dimension 1.  Axes up to 256 that do not factor
+# are dense, those to 511 where 2048 lines share the launch (so the 2D / 3D sizes
+# of RADER, BLUESTEIN and LARGE_RADIX above are); beyond, a prime whose
+# predecessor factors is Rader's and the rest Bluestein's (433 - 1 and 1021 - 1
+# factor, 509 - 1 and 262 do not).
+FORMS = [((24, 257), (0, 2)), ((257, 24), (2, 0)), ((6, 5, 433), (0, 0, 2)), ((6, 433, 5), (0, 2, 0)),
+         ((433, 6, 5), (2, 0, 0)), ((3, 1021), (0, 2)), ((1021, 3), (2, 0)),
+         ((24, 262), (0, 1)), ((262, 24), (1, 0)), ((6, 5, 509), (0, 0, 1)), ((6, 509, 5), (0, 1, 0)),
+         ((509, 6, 5), (1, 0, 0)), ((3, 514), (0, 1)), ((514, 3), (1, 0)), ((433, 262), (2, 1)),
+         ((155, 217), (0, 0)), ((145, 186, 4), (0, 0, 0)),
+         ((191, 127), (4, 4)), ((37, 41, 47), (4, 4, 4)), ((111, 20), (4, 0)), ((9, 8, 83), (0, 0, 4)),
+         ((31, 62), (0, 4)), ((57, 87), (0, 4)), ((383, 2300), (4, 0)), ((2300, 383), (0, 4))]
+
+
+@pytest.mark.parametrize("dims,forms", FORMS)
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_forms(cuda, dims, forms, dtype):
+    from csipm import tune
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("forms", dims, dtype, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 13)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    tol = TOL64 if dtype == torch.float64 else TOL32
+    o = _make(dims, miss, dtype)
+    assert tuple(tune.fft_shape(o, axis)[2] for axis in range(len(dims))) == forms
+    xt = torch.from_numpy(x).to(cuda, dtype)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
+
+
+# dense tiles of 16 and 32 lines (32 or 64 real columns), which a launch takes
+# when it has 1024 of them: 32 lines of 37 (18 of 32 valid), 16 of 185 (FP32; 8 in
+# FP64) and of 126, along dimension 1 32 pairs of 37 and 16 of 131 (FP32)
+@pytest.mark.parametrize("dims", [(34, 37, 1030), (18, 185, 1030), (17, 1030, 126), (37, 260, 256),
+                                  (131, 182, 182)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_wide_dense_tiles(cuda, dims, dtype):
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("wide dense tiles", dims, dtype, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 17)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    tol = TOL64 if dtype == torch.float64 else TOL32
+    o = _make(dims, miss, dtype)
+    xt = torch.from_numpy(x).to(cuda, dtype)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
