@@ -299,20 +299,19 @@ constexpr int kE = 8;
 constexpr int kTile = 4096;
 constexpr int kTileLong = 16384;
 constexpr int kNTLong = 2048;
+// FP32 line and dimension-1 passes of 2D / 3D problems also go to kTile with
+// kNTWide (a name for 256 threads of 16 elements)
+constexpr int kNTWide = 272;
 constexpr size_t kLdsSmall = 64 * 1024;
 constexpr size_t kLdsMax = 160 * 1024;
 constexpr int kDenseVariant = 2;   // FftPlan::variant of a dense axis (no stages)
-// elements a thread takes through the stages of a plan
-inline int plan_cap(const FftPlan& p) {
+// threads that take a tile through the stages of a plan
+inline int tile_threads(int64_t elems, const FftPlan& p) {
   int cap = 2 * kE;
   for (int s = 0; s < p.nstages; ++s) {
     const int R = p.st[s].radix;
     cap = std::min(cap, R * ((kE + R - 1) / R));
   }
-  return cap;
-}
-inline int tile_threads(int64_t elems, const FftPlan& p) {
-  const int cap = plan_cap(p);
   return (int)((elems + cap - 1) / cap);
 }
 // workgroup size of a tile: as many threads as the stages keep busy, but 256
@@ -353,6 +352,21 @@ inline bool tile_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed
   const bool fits = ((size_t)2 << lg) * rows * cs <= 32 * 1024;
   return (t <= 256 && fits) || (t <= 512 && ((size_t)1 << lg) * cs < 32) ||
          (kkt && t <= 512 && fits && ((size_t)1 << lg) * cs < 128);
+}
+
+// Whether an FP32 tile of 2^lg lines goes on to 2^(lg + 1) on 256 threads of 16
+// elements: up to rows of 64 bytes (lengths above 256, whose tiles of 8 elements
+// a thread end at 32), and in the batched chains to 128 where the lines fill the
+// threads (255 = 17 x 15 in 16 lines keeps all of them busy, in 8 half).  One CG
+// apply, 8 and 16 elements: 384^3 1008 and 885 us, 320^3 626 and 552, 255^3 265
+// and 236, 256 problems of 255 x 255 177 and 163; 189^3 in 16 lines, three
+// quarters full, 143 and 167.  The passes that read or write beta keep 8 (255^3
+// in 16 lines 1.05 to 1.18 times the time).  FP64 has no registers for 16.
+inline bool wide_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed, bool chain) {
+  const int64_t e = ((int64_t)2 << lg) * p.L;
+  const size_t row = ((size_t)2 << lg) * cs;
+  return cs == 8 && !mixed && p.variant != kDenseVariant && e <= kTile && row * rows <= kLdsSmall &&
+         (row <= 64 || (chain && row <= 128 && 16 * e >= 15 * kTile));
 }
 
 struct LineCfg {
@@ -974,10 +988,10 @@ static int min_tile_lg(size_t cs) {
 // line FFTs along dim 2/3: 2^lg lines per workgroup, as many as tile_grows
 // allows, fewer when that would leave the launch with under min_grid
 // workgroups (1024 for one instance; a batch shares the target among its
-// instances)
+// instances).  wide: 1 with wide_grows, 2 as in a batched chain
 static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size_t cs,
                         int min_grid = 1024, int lg_cap = 30, bool mixed = false,
-                        bool kkt = false) {
+                        bool kkt = false, int wide = 0) {
   LineCfg c{};
   int lg = 0;
   while (tile_grows(lg, plan, R, cs, mixed, kkt) && (size_t)(2 << lg) * R * cs <= kLdsSmall && (1 << lg) < H1 &&
@@ -991,11 +1005,17 @@ static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size
   auto grid_of = [&](int l) { return (int64_t)((H1 + (1 << l) - 1) >> l) * others; };
   while (lg > lg_end && grid_of(lg) < min_grid && !(lg <= lg_min && 4 * grid_of(lg) >= min_grid))
     --lg;
+  c.nt = tile_nt((int64_t)plan.L << lg, plan);
+  // (not where the wider tiles reach over a tenth more lines past the last one)
+  while (wide && wide_grows(lg, plan, R, cs, mixed, wide == 2) && (1 << lg) < H1 && lg < lg_cap &&
+         grid_of(lg + 1) >= min_grid && 10 * (grid_of(lg + 1) << (lg + 1)) <= 11 * (grid_of(lg) << lg)) {
+    ++lg;
+    c.nt = kNTWide;
+  }
   c.lg = lg;
   c.ntile1 = (H1 + (1 << lg) - 1) >> lg;
   c.grid = (int)(c.ntile1 * others);
   c.lds = (size_t)(1 << lg) * R * cs;
-  c.nt = tile_nt((int64_t)plan.L << lg, plan);
   return c;
 }
 
@@ -1036,7 +1056,7 @@ static Dim1Cfg row_cfg(const FftPlan& plan, int B, size_t cs, int min_grid = 102
 }
 
 static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int min_grid = 1024,
-                        int lg_cap = 30, bool mixed = false) {
+                        int lg_cap = 30, bool mixed = false, bool chain = false) {
   Dim1Cfg c{};
   c.npairs = (nlines + 1) / 2;
   int lg = 0;
@@ -1046,11 +1066,16 @@ static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int m
     ++lg;
   const int lg_end = plan.variant == kDenseVariant ? std::min(lg, 3) : 0;
   while (lg > lg_end && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
+  c.nt = tile_nt((int64_t)plan.L << lg, plan);
+  while (wide_grows(lg, plan, R, cs, mixed, chain) && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
+         lg < lg_cap && ((c.npairs + (2 << lg) - 1) >> (lg + 1)) >= min_grid) {
+    ++lg;
+    c.nt = kNTWide;
+  }
   c.lg = lg;
   c.ps = (1 << lg) + (lg > 0 ? 1 : 0);
   c.grid = (c.npairs + (1 << lg) - 1) >> lg;
   c.lds = lds_of(lg);
-  c.nt = tile_nt((int64_t)plan.L << lg, plan);
   // one line alone: a launch of one workgroup, which waits for its loads more
   // than for its stages (operator product, 256 and 512 threads: 2048 FP32 17.8
   // and 15.9 us, 4096 26.8 and 22.2, 4096 FP64 26.1 and 22.9; of many lines
@@ -1235,6 +1260,15 @@ int launch_pass(csipm_op* h, const PassArgs<T>& a, int grid, int nt, size_t lds)
     return fail(CSIPM_ERR_UNSUPPORTED, "no dense kernel for pass (%d, %d, %d)", a.ld, a.mid, a.st);
   }
 #undef CSIPM_DENSE
+#define CSIPM_WIDE(LD, MID, ST) \
+  if (CSIPM_IS(LD, MID, ST)) CSIPM_PASS(256, 16, LD, MID, ST, FORM_FFT);
+  if constexpr (sizeof(T) == 4) {
+    if (nt == kNTWide) {
+      CSIPM_DENSE_CHAIN(CSIPM_WIDE)
+      CSIPM_DENSE_ENTRY(CSIPM_WIDE)
+    }
+  }
+#undef CSIPM_WIDE
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
     if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST, FORM_FFT);      \
@@ -2055,7 +2089,9 @@ static int set_shapes(csipm_op* h, PrecState& ps, size_t cs) {
   if (F0 > kTileLong || ps.d1.lds > kLdsMax)
     return fail(CSIPM_ERR_UNSUPPORTED, "dimension-1 length %d (FFT length %d) exceeds one "
                 "workgroup", h->n[0], F0);
-  if (dim >= 2) ps.lines[1] = line_cfg(h->H1, h->plan[1], h->rows[1], h->n[2], cs);
+  if (dim >= 2)
+    ps.lines[1] = line_cfg(h->H1, h->plan[1], h->rows[1], h->n[2], cs, 1024, 30, false, false,
+                           dim == 3 ? 1 : 0);
   if (dim == 3) ps.lines[2] = line_cfg(h->H1, h->plan[2], h->rows[2], h->n[1], cs);
   if (dim >= 2)
     ps.kkt = line_cfg(h->H1, h->plan[dim - 1], h->rows[dim - 1], dim == 3 ? h->n[1] : 1, cs, 1024,

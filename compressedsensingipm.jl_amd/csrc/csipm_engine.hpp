@@ -206,6 +206,14 @@ int launch_sub(const ChainSub& a, hipStream_t st) {
     return fail(CSIPM_ERR_UNSUPPORTED, "no dense kernel for pass (%d, %d, %d)", a.ld, a.mid, a.st);
   }
 #undef CSIPM_DENSE
+#define CSIPM_WIDE(LD, MID, ST) \
+  if (CSIPM_IS(LD, MID, ST)) CSIPM_PASS(256, 16, LD, MID, ST, FORM_FFT);
+  if constexpr (sizeof(T) == 4) {
+    if (nt == kNTWide) {
+      CSIPM_DENSE_CHAIN(CSIPM_WIDE)
+    }
+  }
+#undef CSIPM_WIDE
 #define CSIPM_SHORT(LD, MID, ST)                          \
   if (CSIPM_IS(LD, MID, ST)) {                            \
     if (nt == 128) CSIPM_PASS(128, kE, LD, MID, ST, FORM_FFT);      \
@@ -505,12 +513,12 @@ BatchCfg batch_cfg(csipm_op* h, int members, bool mixed) {
   }
   const TuneVal t0 = tune_lookup(1, cs, h->plan[0].L, h->rows[0]);
   b.d1 = dim1_cfg(h->plan[0], h->rows[0], (int)(h->N / h->n[0]), cs, target, t0.lg_cap,
-                  mixed);
+                  mixed, true);
   TuneVal ta[3];
   for (int a = 1; a < h->dim; ++a) {
     ta[a] = tune_lookup(0, cs, h->plan[a].L, h->rows[a]);
     b.lines[a] = line_cfg(h->H1, h->plan[a], h->rows[a], h->n[a == 1 ? 2 : 1], cs, target,
-                          ta[a].lg_cap, mixed);
+                          ta[a].lg_cap, mixed, false, 2);
   }
   return b;
 }
@@ -646,7 +654,7 @@ int build_chain(Engine* E, TableArena& A, const std::vector<int>& ids, int call,
       mem.push_back(m);
     }
   for (int p = 0; p < 8; ++p)
-    for (int nt : {kNTLong, 1024, 512, 256, 128}) {
+    for (int nt : {kNTLong, 1024, 512, kNTWide, 256, 128}) {
       ChainSub sub;
       sub.pass = p;
       sub.nt = nt;

@@ -1567,16 +1567,16 @@ __device__ __forceinline__ void pass_body(const PassArgs<T>& a, int tile,
 // four as well, nothing spilled at 128 registers: a mixed launch of 512 threads
 // 39.2 to 36.0 us (70 spilled at 96), the dense product of 127^3 80 to 77.
 // The mixed FP64 ones two (256 threads 82 to 73 us; 106 spilled at 168)
-template <typename T, int NT, int LD, int FORM>
+template <typename T, int NT, int E, int LD, int FORM>
 constexpr int pass_waves() {
-  if (NT >= 1024 || (sizeof(T) == 4 && (LD < 0 || FORM == FORM_DENSE))) return 4;
+  if (E == 16 || NT >= 1024 || (sizeof(T) == 4 && (LD < 0 || FORM == FORM_DENSE))) return 4;
   if (LD < 0) return 2;
   return sizeof(T) == 4 ? 5 : 3;
 }
 
 // a pass of one instance
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT, LD, FORM>())) void k_pass(PassArgs<T> a) {
+__global__ __launch_bounds__(NT, (pass_waves<T, NT, E, LD, FORM>())) void k_pass(PassArgs<T> a) {
   if constexpr (ST == ST_LINES_BETA3 && FORM == FORM_FFT) {
     const ArgsPtr<T> args = (ArgsPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
     pass_body<T, NT, E, LD, MID, ST, FORM>(load_args<T>(args), xcd_block(), args);
@@ -1594,7 +1594,7 @@ struct BlockMap {
 // passes of several instances (LD < 0: each its own kind): the host's block map keeps
 // adjacent tiles of an instance on one XCD (block b runs on XCD b % 8).
 template <typename T, int NT, int E, int LD, int MID, int ST, int FORM>
-__global__ __launch_bounds__(NT, (pass_waves<T, NT, LD, FORM>())) void kb_pass(
+__global__ __launch_bounds__(NT, (pass_waves<T, NT, E, LD, FORM>())) void kb_pass(
     const PassArgs<T>* __restrict__ tab, const BlockMap* __restrict__ map) {
   const int i = uniform(map[blockIdx.x].member), tile = uniform(map[blockIdx.x].tile);
   if (i < 0) return;

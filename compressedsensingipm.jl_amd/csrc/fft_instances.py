@@ -49,8 +49,10 @@ ENTRY_DIM1 = [
 # and of longer lines (dimension 1 only)
 NT_SHORT = ["128 8", "256 8", "512 8"]
 NT_LONG = ["1024 8", "1024 16"]
+# FP32 tiles of the 2D / 3D passes in which a thread holds 16 elements
+NT_WIDE = ["256 16"]
 MIXED = "-1 -1 -1"
-# of these, the passes of 2D / 3D axes in the dense form (256 threads)
+# of these, the passes of 2D / 3D axes: in the dense form (256 threads)
 DENSE_CHAIN = [s for s in CHAIN_SHORT if "LINES" in s] + CHAIN_DIM1[1:2] + CHAIN_DIM1[3:]
 DENSE_ENTRY = [s for s in ENTRY_SHORT if "LINES" in s] + ENTRY_DIM1[2:3]
 
@@ -69,7 +71,10 @@ def instances():
     }
     out = []
     for t in ("float", "double"):
+        wide = {"k_pass": DENSE_CHAIN + DENSE_ENTRY, "kb_pass": DENSE_CHAIN}
         for k, rs in table.items():
+            if t == "float":
+                rs = rs + rows(NT_WIDE, wide[k])
             p = f"PassArgs<{t}>" if k == "k_pass" else f"const PassArgs<{t}>*, const BlockMap*"
             out += [f"void {k}<{', '.join([t] + r.split())}>({p})" for r in rs]
     return out

@@ -357,3 +357,19 @@ def test_dense_and_other_members(cuda, shapes, mixed):
     res = solve_batch(ops, [p.z0 for p in probs], [p.lam for p in probs], mixed=mixed, tol=tol)
     for p, r in zip(probs, res):
         _same(r, _alone(p, mixed, tol), p.name)
+
+
+# 256 members share the workgroup target, so that their FP32 passes take tiles of
+# 16 elements a thread: line passes of 255 (16 lines) and 300 (8), dimension 1 of
+# 255 (16 pairs) and 320 (8)
+def test_sixteen_element_tiles(cuda):
+    import csipm.workloads as wl
+    from csipm.batch import solve_batch
+    print("sixteen elements", flush=True)
+    shapes = [(128, 255), (100, 300), (255, 160), (320, 64)]
+    probs = [wl.batch_instance(shapes[k % 4], seed=60 + k) for k in range(256)]
+    ops = [_op(p, True) for p in probs]
+    res = solve_batch(ops, [p.z0 for p in probs], [p.lam for p in probs], mixed=True, tol=1e-8)
+    assert all(r.status == "solved" for r in res)
+    for p, r in list(zip(probs, res))[:4] + list(zip(probs, res))[-4:]:
+        _same(r, _alone(p, True, 1e-8), p.name)

@@ -359,3 +359,20 @@ def test_wide_dense_tiles(cuda, dims, dtype):
     assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= tol
     assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= tol
     assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= tol
+
+
+# FP32 tiles of 16 elements a thread: along dimension 1 (270, 8 pairs) and on the
+# middle line passes (300, 8 lines; 16 of them, and 51, the last tile in part)
+@pytest.mark.parametrize("dims", [(270, 128, 130), (30, 300, 512), (100, 300, 150)])
+def test_sixteen_element_tiles(cuda, dims):
+    from csipm.fft_operator import M_perp_beta, M_perpt_M_perp_vec, M_perpt_z
+    print("sixteen elements", dims, flush=True)
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(n + 19)
+    miss = np.sort(rng.choice(n, size=n // 9, replace=False))
+    x = rng.standard_normal(n)
+    o = _make(dims, miss, torch.float32)
+    xt = torch.from_numpy(x).to(cuda, torch.float32)
+    assert _rel(M_perpt_M_perp_vec(o, xt).double().cpu().numpy(), op.mtm(x, dims, miss)) <= TOL32
+    assert _rel(M_perp_beta(o, xt).double().cpu().numpy(), op.m_perp_beta(x, dims, miss)) <= TOL32
+    assert _rel(M_perpt_z(o, xt).double().cpu().numpy(), op.m_perpt_z(x, dims)) <= TOL32
