@@ -368,6 +368,12 @@ inline bool wide_grows(int lg, const FftPlan& p, int rows, size_t cs, bool mixed
   return cs == 8 && !mixed && p.variant != kDenseVariant && e <= kTile && row * rows <= kLdsSmall &&
          (row <= 64 || (chain && row <= 128 && 16 * e >= 15 * kTile));
 }
+// and an FP32 tile of kTile elements, nearly full, takes them instead of 512
+// threads of 8 (2048 x 2048 operator product 98 -> 86 us; tiles of 3000 keep 512,
+// 3000 x 700 56 against 63)
+inline int wide_nt(int nt, int64_t elems, size_t cs, bool mixed) {
+  return nt == 512 && cs == 8 && !mixed && elems <= kTile && 16 * elems >= 15 * kTile ? kNTWide : nt;
+}
 
 struct LineCfg {
   int lg = 0, ntile1 = 0, grid = 0;
@@ -1006,6 +1012,7 @@ static LineCfg line_cfg(int H1, const FftPlan& plan, int R, int64_t others, size
   while (lg > lg_end && grid_of(lg) < min_grid && !(lg <= lg_min && 4 * grid_of(lg) >= min_grid))
     --lg;
   c.nt = tile_nt((int64_t)plan.L << lg, plan);
+  if (!kkt) c.nt = wide_nt(c.nt, (int64_t)plan.L << lg, cs, mixed);
   // (not where the wider tiles reach over a tenth more lines past the last one)
   while (wide && wide_grows(lg, plan, R, cs, mixed, wide == 2) && (1 << lg) < H1 && lg < lg_cap &&
          grid_of(lg + 1) >= min_grid && 10 * (grid_of(lg + 1) << (lg + 1)) <= 11 * (grid_of(lg) << lg)) {
@@ -1067,6 +1074,7 @@ static Dim1Cfg dim1_cfg(const FftPlan& plan, int R, int nlines, size_t cs, int m
   const int lg_end = plan.variant == kDenseVariant ? std::min(lg, 3) : 0;
   while (lg > lg_end && ((c.npairs + (1 << lg) - 1) >> lg) < min_grid) --lg;
   c.nt = tile_nt((int64_t)plan.L << lg, plan);
+  if (nlines > 1) c.nt = wide_nt(c.nt, (int64_t)plan.L << lg, cs, mixed);
   while (wide_grows(lg, plan, R, cs, mixed, chain) && lds_of(lg + 1) <= kLdsSmall && (1 << lg) < c.npairs &&
          lg < lg_cap && ((c.npairs + (2 << lg) - 1) >> (lg + 1)) >= min_grid) {
     ++lg;
