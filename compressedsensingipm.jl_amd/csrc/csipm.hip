@@ -316,9 +316,9 @@ inline int tile_threads(int64_t elems, const FftPlan& p) {
 }
 // workgroup size of a tile: as many threads as the stages keep busy, but 256
 // for tiles of up to 1024 elements (more loads in flight where the launch is
-// short) and where 128 would move 16 elements each through the global phases
-// (256^3 FP64: 617 us on 256 threads, 652 on 128).  391 = 23 x 17 points in 4
-// lines keep 92 threads busy.
+// short) and where 128 would move more than 14 elements each through the global
+// phases (256^3 FP64, 16 each: 617 us on 256 threads, 652 on 128).  391 = 23 x 17
+// points in 4 lines keep 92 of 128 threads busy and move 12.2 each.
 inline int tile_nt(int64_t elems, const FftPlan& p) {
   if (p.variant == kDenseVariant) return 256;
   const int t = tile_threads(elems, p);

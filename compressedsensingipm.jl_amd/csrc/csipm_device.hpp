@@ -400,24 +400,21 @@ __device__ __forceinline__ void dft_odd_store(cpx<T>* v, cpx<T>* __restrict__ ds
     y0 = cadd(y0, a);
   }
   dst[0] = y0;
-  auto output = [&](int k, const auto& c, const auto& s) {
-    T re = x0.x, im = x0.y, sre = 0, sim = 0;
-#pragma unroll
-    for (int j = 1; j <= H; ++j) {
-      re += v[j].x * c(j);
-      im += v[j].y * c(j);
-      sre += v[R - j].y * s(j);
-      sim += v[R - j].x * s(j);
-    }
-    dst[k * stride] = {re + sre, im - sim};
-    dst[(R - k) * stride] = {re - sre, im + sim};
-  };
   // one output after another: scheduled across outputs the (H x H) products
   // took hundreds of registers in FP64
 #pragma unroll
   for (int k = 1; k <= H; ++k) {
-    output(k, [&](int j) { return (T)OddRadix<R>::c[(j * k) % R]; },
-           [&](int j) { return (T)OddRadix<R>::s[(j * k) % R]; });
+    T re = x0.x, im = x0.y, sre = 0, sim = 0;
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      const T c = (T)OddRadix<R>::c[(j * k) % R], s = (T)OddRadix<R>::s[(j * k) % R];
+      re += v[j].x * c;
+      im += v[j].y * c;
+      sre += v[R - j].y * s;
+      sim += v[R - j].x * s;
+    }
+    dst[k * stride] = {re + sre, im - sim};
+    dst[(R - k) * stride] = {re - sre, im + sim};
     if constexpr (R >= 11) __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -450,7 +447,8 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
 // L cost a cache line per lane.
 // Measured (before -> after, with tile_grows' tiles): line passes of the FP64
 // 256^3 apply 72 -> 65 and 70 -> 57 us (270 MB each, 4.1-4.7 TB/s), its
-// dimension-1 pass 140 -> 123 us; 509 x 384 FP64 (Rader) 19 -> 13 us.
+// dimension-1 pass 140 -> 123 us (107 since radices 29 and 31 are matrix_stage's
+// and the pass kernels no longer spill); 509 x 384 FP64 (Bluestein) 19 -> 13 us.
 // ---------------------------------------------------------------------------
 constexpr int kMaxStages = 15;
 

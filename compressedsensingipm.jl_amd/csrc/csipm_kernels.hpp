@@ -469,11 +469,14 @@ struct PassArgs {
 // at most four at a time, and the outputs replace a and b when all waves have
 // read them.  The coefficients come packed in lane order, 64 to a 16 x 4 tile
 // (the wave reads them from the L2, one load feeding N products).
-// What bounds it: the matrix rate, L^2 / 128 cycles a line and CU in FP32 (L^2
-// / 64 in FP64) at 256 (128) operations a cycle.  Rader's and Bluestein's forms of
-// such lengths spent over a thousand cycles a line on two transforms and the
-// moves between, in twice the LDS rows: the operator product of 127^3 took 187
-// us in FP32 and 75 with this (185^3: 400 to 243, FP64 784 to 392).
+// What bounds it: the products take L^2 / 128 cycles a line and CU in FP32 (L^2
+// / 64 in FP64), which is 17% of the time of a 127^3 line pass (FP64 23%): its
+// waves wait 60% of theirs for memory and LDS, since in a tile of 8 lines each
+// load of a coefficient feeds one product.  At 185^3 the matrix cores are busy
+// 41%, and the waves wait half their time to issue.  Rader's and Bluestein's
+// forms of such lengths spent over a thousand cycles a line on two transforms
+// and the moves between, in twice the LDS rows: the operator product of 127^3
+// took 187 us in FP32 and 71 with this (185^3: 400 to 243, FP64 784 to 392).
 // tiles of the coefficient matrices: ceil((H + 1) / 16) by ceil((H + 1) / 4)
 // (cosine) and by ceil(((L - 1) / 2) / 4) (sine), the latter two made even
 // (zero tiles; their rows stay inside the line for L > 16)
