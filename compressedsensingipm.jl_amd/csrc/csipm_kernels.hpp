@@ -491,7 +491,7 @@ __host__ __device__ __forceinline__ int dense_ks(int L) { return ((L - 1) / 2 + 
 // as it has terms.  M^T M off by, FP32 / FP64: 127 x 127 in one chain 3.1e-7 /
 // 5.7e-16, in parts of 8 2.0e-7 / 3.6e-16 (Rader's form 3.2e-7 / 7.2e-16, the
 // radix plan of 116 x 124 2.1e-7 / 3.9e-16); 509 x 2100 4.5e-7 / 8.3e-16 in one
-// chain, 2.5e-7 / 4.7e-16 in parts of 32 (Rader's 3.0e-7 / 7.1e-16; parts of 8
+// chain, 2.5e-7 / 4.7e-16 in parts of 32 (Bluestein's 3.0e-7 / 7.1e-16; parts of 8
 // took 185^3 in FP64 from 406 to 432 us)
 template <typename T, int U, int N>
 __device__ __forceinline__ void dense_product(Vec4<T> (&acc)[U][N], const T* const (&p)[U],
